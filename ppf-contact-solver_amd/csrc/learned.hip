@@ -18,7 +18,11 @@ namespace {
 constexpr unsigned kNT = 256;
 constexpr uint32_t kH = kLpcH, kFN = kLpcFN, kFE = kLpcFE;
 constexpr uint32_t kMir = 0x80000000u;
-constexpr uint32_t kChunk = 4096; // rows per weight-gradient partial
+// Weight-gradient partials: at most kWgGrid workgroups (two rounds of the two
+// resident per CU), each of at least kWgMinRows rows.
+constexpr uint32_t kWgGrid = 512, kWgMinRows = 256;
+constexpr uint32_t kWgStep = 32; // rows a wave stages and multiplies at a time
+constexpr uint32_t kHeadWords = kH * 6 + 6 + (2 * kH + kFE) * 9 + 9; // [Wo][co][Wg][cg]
 
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -345,70 +349,173 @@ __global__ __launch_bounds__(256) void k_dense(uint32_t M, Seg s0, Seg s1, const
 constexpr uint32_t kDenseGrid = 2048;
 inline uint32_t dense_grid(uint32_t M) { return std::max(1u, std::min(kDenseGrid, (M + 63u) / 64u)); }
 
-// Weight-gradient partials: part[chunk][k][c] = sum over the chunk's rows m
-// of X[m][k] D[m][c] (X = the layer's input segments, D = [M][64] bf16), on
-// MFMA with the rows as the reduction dimension; cpart[chunk][c] = column
-// sums of D (the bias gradient).
-__global__ __launch_bounds__(256) void k_wgrad(uint32_t M, Seg s0, Seg s1, const uint16_t *D,
-                                               float *part, float *cpart) {
+// Orders a wave's LDS accesses across its lanes (LDS operations of one wave
+// complete in order; this keeps the compiler from moving them).
+__device__ inline void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Rows each wave of a weight-gradient launch covers, and its workgroups.
+inline uint32_t wgrad_grid(uint32_t M) {
+    return std::max(1u, std::min(kWgGrid, cdiv(M, kWgMinRows)));
+}
+inline uint32_t wgrad_rows(uint32_t M) {
+    return std::max(1u, cdiv(cdiv(M, 4 * wgrad_grid(M)), kWgStep)) * kWgStep;
+}
+
+// Weight-gradient partials of a dense layer: part[block] = [K][64] sums over
+// the block's rows m of X[m][k] D[m][c] (X = the layer's input segments, 16 KT
+// wide; D = [M][64] bf16), then [64] column sums of D (the bias gradient), on
+// v_mfma_f32_16x16x16_bf16 with the rows as the reduction dimension.
+// Bound by the gathered rows of X (L2): each row of X and D is read once, in
+// 16 B pieces, for all 4 KT output tiles, which a wave keeps in registers. A
+// wave stages 32 rows in its own LDS region (the next 32 are in flight
+// meanwhile) and reads the fragments down the columns; the row stride of
+// 2 (K + 64) + 8 B puts the four row groups of a fragment in different banks.
+// With gridDim.y = 2 (two 64-wide segments: the node layers) block y sums
+// segment y only, which keeps its sums in registers and doubles the blocks.
+// 459k edge rows x 80: 2,700 us with one 16x16 tile per wave and pass and
+// unstaged 2 B column loads, 76 us now; 32,768 node rows x 128: 2,000 us, 14 us
+// now.
+template <int KT>
+__global__ __launch_bounds__(256, 2) void k_wgrad(uint32_t M, uint32_t rows, Seg s0, Seg s1,
+                                                  const uint16_t *D, float *part) {
+    constexpr uint32_t K = 16 * KT, CH = (K + kH) / 8, S = K + kH + 4;
+    constexpr uint32_t kItems = kWgStep * CH / 64;
+    static_assert(kWgStep * CH % 64 == 0, "16 B pieces of a step fill whole waves");
+    static_assert(4 * kWgStep * S * 2 >= K * kH * 4, "the staging holds a wave's sums");
+    __shared__ __attribute__((aligned(16))) uint16_t stage[4][kWgStep * S];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t c0 = blockIdx.x * kChunk, c1 = min(M, c0 + kChunk);
-    const uint32_t ktot = s0.k + s1.k, nkt = ktot / 16;
     const uint32_t ar = lane & 15u, aq = lane >> 4;
-    float *pc = part + (size_t)blockIdx.x * ktot * kH;
-    for (uint32_t tile = wave; tile < nkt * 4; tile += 4) {
-        const uint32_t kt = tile / 4, nt = tile % 4;
-        const uint32_t k = kt * 16 + ar;
-        const Seg &s = k < s0.k ? s0 : s1;
-        const uint32_t kc = k < s0.k ? k : k - s0.k;
-        v4f acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-        for (uint32_t m0 = c0; m0 < c1; m0 += 16) {
-            v4s a, b;
+    const uint32_t r0 = (blockIdx.x * 4u + wave) * rows;
+    const uint32_t r1 = r0 < M ? min(M, r0 + rows) : r0;
+    if (blockIdx.y) {
+        s0 = s1;
+    }
+    uint16_t *lds = stage[wave];
+    v4f acc[KT][4];
+    float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t m = m0 + 4 * aq + r;
-                uint16_t xa = 0, db = 0;
-                if (m < c1) {
-                    const size_t rr = s.idx ? s.idx[m] : m;
-                    xa = s.x[rr * s.ld + kc];
-                    db = D[(size_t)m * kH + nt * 16 + ar];
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) acc[kt][nt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    uint4 w[kItems];
+    auto fetch = [&](uint32_t m0) {
+#pragma unroll
+        for (uint32_t it = 0; it < kItems; ++it) {
+            const uint32_t t = it * 64u + lane, m = m0 + t / CH, c = 8u * (t % CH);
+            w[it] = make_uint4(0, 0, 0, 0);
+            if (m < r1) {
+                const uint16_t *src;
+                if (c >= K) {
+                    src = D + (size_t)m * kH + (c - K);
+                } else if (c < s0.k) {
+                    src = s0.x + (size_t)(s0.idx ? s0.idx[m] : m) * s0.ld + c;
+                } else {
+                    src = s1.x + (size_t)(s1.idx ? s1.idx[m] : m) * s1.ld + (c - s0.k);
                 }
-                a[r] = (short)xa;
-                b[r] = (short)db;
+                w[it] = *reinterpret_cast<const uint4 *>(src);
             }
-            acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+        }
+    };
+    if (r0 < r1) {
+        fetch(r0);
+    }
+    for (uint32_t m0 = r0; m0 < r1; m0 += kWgStep) {
+        wave_sync(); // the last step's fragments are read
+#pragma unroll
+        for (uint32_t it = 0; it < kItems; ++it) {
+            const uint32_t t = it * 64u + lane;
+            uint2 *o = reinterpret_cast<uint2 *>(lds + (t / CH) * S + 8u * (t % CH));
+            o[0] = make_uint2(w[it].x, w[it].y);
+            o[1] = make_uint2(w[it].z, w[it].w);
+        }
+        wave_sync();
+        if (m0 + kWgStep < r1) {
+            fetch(m0 + kWgStep);
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            pc[(size_t)(kt * 16 + 4 * aq + r) * kH + nt * 16 + ar] = acc[r];
+        for (uint32_t half = 0; half < kWgStep; half += 16) {
+            const uint16_t *row = lds + (half + 4u * aq) * S + ar;
+            v4s b[4];
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint16_t h = row[r * S + K + 16 * nt];
+                    b[nt][r] = (short)h;
+                    bias[nt] += from_bf16(h);
+                }
+            }
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) {
+                v4s a;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) a[r] = (short)row[r * S + 16 * kt];
+#pragma unroll
+                for (int nt = 0; nt < 4; ++nt) {
+                    acc[kt][nt] =
+                        __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b[nt], acc[kt][nt], 0, 0, 0);
+                }
+            }
         }
     }
-    if (threadIdx.x < kH) {
-        float sum = 0.0f;
-        for (uint32_t m = c0; m < c1; ++m) {
-            sum += from_bf16(D[(size_t)m * kH + threadIdx.x]);
+    // the four waves' sums, added in wave order
+    __shared__ float bsum[4][kH];
+    float *sum = reinterpret_cast<float *>(&stage[0][0]);
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
+        bias[nt] += __shfl_xor(bias[nt], 16);
+        bias[nt] += __shfl_xor(bias[nt], 32);
+        if (aq == 0) bsum[wave][16 * nt + ar] = bias[nt];
+    }
+    for (uint32_t q = 0; q < 4; ++q) {
+        __syncthreads();
+        if (wave == q) {
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+                for (int nt = 0; nt < 4; ++nt) {
+                    v4f *o = reinterpret_cast<v4f *>(sum + (4 * kt + nt) * 256) + lane;
+                    *o = q ? *o + acc[kt][nt] : acc[kt][nt];
+                }
         }
-        cpart[(size_t)blockIdx.x * kH + threadIdx.x] = sum;
+    }
+    __syncthreads();
+    const uint32_t ktot = gridDim.y * K;
+    float *out = part + (size_t)blockIdx.x * (ktot * kH + kH) + blockIdx.y * K * kH;
+    for (uint32_t e = threadIdx.x; e < K * kH; e += 256) {
+        // element (k, c): tile (k / 16, c / 16), lane 16 ((k % 16) / 4) + c % 16
+        const uint32_t k = e / kH, c = e % kH;
+        out[e] = sum[(4 * (k / 16) + c / 16) * 256 + (16 * ((k % 16) / 4) + c % 16) * 4 + k % 4];
+    }
+    if (threadIdx.x < kH && blockIdx.y == 0) {
+        const uint32_t c = threadIdx.x;
+        out[ktot * kH + c] = ((bsum[0][c] + bsum[1][c]) + bsum[2][c]) + bsum[3][c];
     }
 }
 
-// gW[k][c] += sum over chunks of part (fixed order); gb[c] likewise.
-__global__ void k_wgrad_reduce(uint32_t nchunk, uint32_t ktot, const float *part,
-                               const float *cpart, float *gW, float *gb) {
-    const uint32_t e = blockIdx.x * kNT + threadIdx.x;
-    if (e < ktot * kH) {
-        float s = 0.0f;
-        for (uint32_t c = 0; c < nchunk; ++c) {
-            s += part[(size_t)c * ktot * kH + e];
+// out[e] += sum over the nblk partials (stride words apart) of part[e], in a
+// fixed order: 16 interleaved slices, then the slices.
+__global__ __launch_bounds__(1024) void k_wgrad_reduce(uint32_t nblk, uint32_t stride,
+                                                       uint32_t len, const float *part,
+                                                       float *out) {
+    __shared__ float lds[16][64];
+    const uint32_t c = threadIdx.x & 63u, q = threadIdx.x >> 6;
+    const uint32_t e = blockIdx.x * 64u + c;
+    float s = 0.0f;
+    if (e < len) {
+        for (uint32_t k = q; k < nblk; k += 16) {
+            s += part[(size_t)k * stride + e];
         }
-        gW[e] += s;
-    } else if (e < ktot * kH + kH) {
-        const uint32_t c = e - ktot * kH;
-        float s = 0.0f;
-        for (uint32_t k = 0; k < nchunk; ++k) {
-            s += cpart[(size_t)k * kH + c];
-        }
-        gb[c] += s;
+    }
+    lds[q][c] = s;
+    __syncthreads();
+    if (q == 0 && e < len) {
+        for (uint32_t k = 1; k < 16; ++k) s += lds[k][c];
+        out[e] += s;
     }
 }
 
@@ -631,60 +738,120 @@ __global__ void k_dhead_out(PcgPattern pt, const float *t, const float *u, float
     }
 }
 
-// Head weight gradients: gWo[c][o] = sum_j h3[j][c] dt[j][o] (fp32, per
-// chunk then reduced by k_wgrad_reduce-like sums in fixed order).
-__global__ void k_head_wgrad(PcgPattern pt, const uint16_t *h3, const uint16_t *f,
-                             const uint32_t *srow, const uint32_t *semir, const float *dt9,
-                             const float *du, float *part) {
-    // part layout per chunk: [64*6 Wo][6 co][144*9 Wg][9 cg]
-    constexpr uint32_t kP = kH * 6 + 6 + (2 * kH + kFE) * 9 + 9;
-    const uint32_t e = threadIdx.x + blockIdx.y * kNT;
-    if (e >= kP) {
-        return;
-    }
-    const uint32_t c0 = blockIdx.x * kChunk;
-    float s = 0.0f;
-    if (e < kH * 6 + 6) {
-        const uint32_t c = e / 6, o = e % 6;
-        const uint32_t c1 = min(pt.n, c0 + kChunk);
-        for (uint32_t j = c0; j < c1; ++j) {
-            const float x = c < kH ? from_bf16(h3[(size_t)j * kH + c]) : 1.0f;
-            s += x * dt9[9 * (size_t)j + o];
-        }
-    } else {
-        const uint32_t q = e - (kH * 6 + 6);
-        const uint32_t c = q / 9, o = q % 9;
-        const uint32_t c1 = min(pt.nnz, c0 + kChunk);
-        for (uint32_t sl = c0; sl < c1; ++sl) {
-            const float d = du[9 * (size_t)sl + o];
-            if (d == 0.0f) {
-                continue;
+// Weight-gradient partials of an output head: part[block] = [16 KT][NC] sums
+// over the block's rows m of X[m][k] d[m][o] (X = up to three bf16 segments
+// gathered by row, d = fp32 with 9 floats per row, the first NC used), then
+// [NC] column sums of d. With skip / skip2, a row where they agree (a stored
+// diagonal block) counts as zero. fp32 throughout (v_mfma_f32_16x16x4_f32,
+// the bf16 inputs widened exactly); staged as in k_wgrad. 290k blocks x 144:
+// 2,027 us with one thread per weight and chunk of rows, 60 us now.
+template <int KT, int NC>
+__global__ __launch_bounds__(256, 2) void k_head_wgrad(uint32_t M, uint32_t rows, Seg s0, Seg s1,
+                                                       Seg s2, const float *d,
+                                                       const uint32_t *skip,
+                                                       const uint32_t *skip2, uint32_t stride,
+                                                       float *part) {
+    constexpr uint32_t K = 16 * KT, CH = K / 8, S = K + 4, LD = 9;
+    constexpr uint32_t kItems = kWgStep * CH / 64, kD = (kWgStep * LD + 63) / 64;
+    static_assert(kWgStep * CH % 64 == 0, "16 B pieces of a step fill whole waves");
+    static_assert(4 * kWgStep * S * 2 >= K * 16 * 4, "the staging holds a wave's sums");
+    __shared__ __attribute__((aligned(16))) uint16_t stage[4][kWgStep * S];
+    __shared__ float dstage[4][kWgStep * LD];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t ar = lane & 15u, aq = lane >> 4;
+    const uint32_t r0 = (blockIdx.x * 4u + wave) * rows;
+    const uint32_t r1 = r0 < M ? min(M, r0 + rows) : r0;
+    uint16_t *lds = stage[wave];
+    float *dl = dstage[wave];
+    v4f acc[KT];
+    float bias = 0.0f;
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) acc[kt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    uint4 w[kItems];
+    float dw[kD];
+    auto fetch = [&](uint32_t m0) {
+#pragma unroll
+        for (uint32_t it = 0; it < kItems; ++it) {
+            const uint32_t t = it * 64u + lane, m = m0 + t / CH, c = 8u * (t % CH);
+            w[it] = make_uint4(0, 0, 0, 0);
+            if (m < r1 && !(skip && skip[m] == skip2[m])) {
+                const uint16_t *src;
+                if (c < s0.k) {
+                    src = s0.x + (size_t)(s0.idx ? s0.idx[m] : m) * s0.ld + c;
+                } else if (c < s0.k + s1.k) {
+                    src = s1.x + (size_t)(s1.idx ? s1.idx[m] : m) * s1.ld + (c - s0.k);
+                } else {
+                    src = s2.x + (size_t)(s2.idx ? s2.idx[m] : m) * s2.ld + (c - s0.k - s1.k);
+                }
+                w[it] = *reinterpret_cast<const uint4 *>(src);
             }
-            float x = 1.0f;
-            if (c < kH) {
-                x = from_bf16(h3[(size_t)pt.col[sl] * kH + c]);
-            } else if (c < 2 * kH) {
-                x = from_bf16(h3[(size_t)srow[sl] * kH + c - kH]);
-            } else if (c < 2 * kH + kFE) {
-                x = from_bf16(f[(size_t)semir[sl] * kFE + c - 2 * kH]);
+        }
+#pragma unroll
+        for (uint32_t it = 0; it < kD; ++it) {
+            const uint32_t t = it * 64u + lane;
+            dw[it] = t < kWgStep * LD && m0 + t / LD < r1 ? d[(size_t)m0 * LD + t] : 0.0f;
+        }
+    };
+    if (r0 < r1) {
+        fetch(r0);
+    }
+    for (uint32_t m0 = r0; m0 < r1; m0 += kWgStep) {
+        wave_sync(); // the last step's fragments are read
+#pragma unroll
+        for (uint32_t it = 0; it < kItems; ++it) {
+            const uint32_t t = it * 64u + lane;
+            uint2 *o = reinterpret_cast<uint2 *>(lds + (t / CH) * S + 8u * (t % CH));
+            o[0] = make_uint2(w[it].x, w[it].y);
+            o[1] = make_uint2(w[it].z, w[it].w);
+        }
+#pragma unroll
+        for (uint32_t it = 0; it < kD; ++it) {
+            const uint32_t t = it * 64u + lane;
+            if (t < kWgStep * LD) dl[t] = dw[it];
+        }
+        wave_sync();
+        if (m0 + kWgStep < r1) {
+            fetch(m0 + kWgStep);
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < kWgStep; q += 4) {
+            // B fragment: lane holds d[row q + aq][ar]; A: X[row q + aq][16 kt + ar]
+            const float b = ar < NC ? dl[(q + aq) * LD + (ar < NC ? ar : 0u)] : 0.0f;
+            bias += b;
+            const uint16_t *row = lds + (q + aq) * S + ar;
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) {
+                acc[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(from_bf16(row[16 * kt]), b, acc[kt],
+                                                               0, 0, 0);
             }
-            s += x * d;
         }
     }
-    part[(size_t)blockIdx.x * kP + e] = s;
-}
-
-__global__ void k_head_wgrad_reduce(uint32_t nchunk, const float *part, float *grad) {
-    constexpr uint32_t kP = kH * 6 + 6 + (2 * kH + kFE) * 9 + 9;
-    const uint32_t e = blockIdx.x * kNT + threadIdx.x;
-    if (e >= kP) {
-        return;
+    // the four waves' sums, added in wave order
+    __shared__ float bsum[4][16];
+    float *sum = reinterpret_cast<float *>(&stage[0][0]);
+    bias += __shfl_xor(bias, 16);
+    bias += __shfl_xor(bias, 32);
+    if (aq == 0) bsum[wave][ar] = bias;
+    for (uint32_t q = 0; q < 4; ++q) {
+        __syncthreads();
+        if (wave == q) {
+#pragma unroll
+            for (int kt = 0; kt < KT; ++kt) {
+                v4f *o = reinterpret_cast<v4f *>(sum + kt * 256) + lane;
+                *o = q ? *o + acc[kt] : acc[kt];
+            }
+        }
     }
-    float s = 0.0f;
-    for (uint32_t c = 0; c < nchunk; ++c) {
-        s += part[(size_t)c * kP + e];
+    __syncthreads();
+    float *out = part + (size_t)blockIdx.x * stride;
+    for (uint32_t e = threadIdx.x; e < K * NC; e += 256) {
+        const uint32_t k = e / NC, o = e % NC;
+        out[e] = sum[(k / 16) * 256 + (16 * ((k % 16) / 4) + o) * 4 + k % 4];
     }
-    grad[LpcLayout::Wo + e] += s; // Wo, co, Wg, cg are contiguous in this order
+    if (threadIdx.x < NC) {
+        const uint32_t o = threadIdx.x;
+        out[K * NC + o] = ((bsum[0][o] + bsum[1][o]) + bsum[2][o]) + bsum[3][o];
+    }
 }
 
 // dh3[j][c] = sum_o dt[j][o] Wo[c][o] + the lower-edge head's input
@@ -875,10 +1042,10 @@ int Lpc::reserve(uint32_t n, uint32_t nnz, uint32_t E) {
     ncap_ = std::max(n, ncap_), nzcap_ = std::max(nnz, nzcap_), ecap_ = std::max(E, ecap_);
     const size_t N = ncap_, Z = nzcap_, EE = std::max<uint32_t>(ecap_, 1);
     const size_t rows = std::max(N, EE);
-    const size_t nchunk = (rows + kChunk - 1) / kChunk;
+    // partials: of the weight gradients (at most kWgGrid workgroups, the
+    // widest layer or the heads), and the row sums' (3 rows: up to 768 probes)
     const size_t part_words =
-        std::max(nchunk * (2 * kH + kFE + 16) * kH + nchunk * kH,
-                 nchunk * (kH * 6 + 6 + (2 * kH + kFE) * 9 + 9));
+        std::max((size_t)kWgGrid * std::max(2 * kH * kH + kH, kHeadWords), 3 * rows);
     auto b = [](size_t count, size_t elem) { return (count * elem + 255) & ~size_t(255); };
     size_t bytes = b(N + 1, 4) + b(EE, 4) * 3 + b(N, 4) + b(Z, 4) * 3 + b(9 * N, 4) +
                    b(kFN * N, 2) + b(kFE * EE, 2) + b(EE, 4) + b(kH * N, 2) * (kLpcLayers + 1) +
@@ -1071,20 +1238,35 @@ int Lpc::gradient(PcgPlanImpl *plan, const float *val, const float *cdiag, const
     PPF_HIP(hipGetLastError());
     // head weights and dh3
     {
-        constexpr uint32_t kP = kH * 6 + 6 + (2 * kH + kFE) * 9 + 9;
-        const uint32_t nchunk = cdiv(m, kChunk);
-        dim3 grid(nchunk, cdiv(kP, kNT));
-        k_head_wgrad<<<grid, kNT, 0, s>>>(pt_, h_[kLpcLayers], f_, srow_, semir_, dgd_, dgl_,
-                                         part_);
+        Seg h3, hd, hs, fe, none;
+        h3.x = h_[kLpcLayers], h3.k = kH, h3.ld = kH;
+        hd = h3, hd.idx = pt_.col;
+        hs = h3, hs.idx = srow_;
+        fe.x = f_, fe.idx = semir_, fe.k = kFE, fe.ld = kFE;
+        const uint32_t go = wgrad_grid(n), gg = wgrad_grid(nnz_);
+        constexpr uint32_t kO = kH * 6 + 6, kG = kHeadWords - kO;
+        k_head_wgrad<kH / 16, 6><<<go, 256, 0, s>>>(n, wgrad_rows(n), h3, none, none, dgd_,
+                                                    nullptr, nullptr, kO, part_);
         PPF_HIP(hipGetLastError());
-        k_head_wgrad_reduce<<<cdiv(kP, kNT), kNT, 0, s>>>(nchunk, part_, grad_);
+        float *pg = part_ + (size_t)kWgGrid * kO;
+        k_head_wgrad<(2 * kH + kFE) / 16, 9><<<gg, 256, 0, s>>>(
+            nnz_, wgrad_rows(nnz_), hd, hs, fe, dgl_, pt_.col, srow_, kG, pg);
+        PPF_HIP(hipGetLastError());
+        k_wgrad_reduce<<<cdiv(kO, 64), 1024, 0, s>>>(go, kO, kO, part_, grad_ + LpcLayout::Wo);
+        PPF_HIP(hipGetLastError());
+        k_wgrad_reduce<<<cdiv(kG, 64), 1024, 0, s>>>(gg, kG, kG, pg, grad_ + LpcLayout::Wg);
         PPF_HIP(hipGetLastError());
         k_dh3<<<cdiv(n * kH, kNT), kNT, 0, s>>>(pt_, dgd_, dgl_, w_, dh_);
         PPF_HIP(hipGetLastError());
     }
+    // weight and bias gradients of a dense layer (contiguous in the layout)
+    auto reduce = [&](uint32_t nblk, uint32_t K, uint32_t at) {
+        const uint32_t len = K * kH + kH;
+        k_wgrad_reduce<<<cdiv(len, 64), 1024, 0, s>>>(nblk, len, len, part_, grad_ + at);
+        return hipGetLastError();
+    };
     float *dXn = reinterpret_cast<float *>(dXn_);
     float *dXe = reinterpret_cast<float *>(dXe_);
-    float *cpart = part_ + (size_t)cdiv(std::max(n, E), kChunk) * (2 * kH + kFE + 16) * kH;
     for (int l = (int)kLpcLayers - 1; l >= 0; --l) {
         // node layer: h_{l+1} = relu([h_l, M_l] Wn + cn)
         k_relu_grad<<<cdiv(n * kH, kNT), kNT, 0, s>>>(n * kH, dh_, h_[l + 1], dZ_);
@@ -1092,12 +1274,10 @@ int Lpc::gradient(PcgPlanImpl *plan, const float *val, const float *cdiag, const
         Seg hn, mn, none;
         hn.x = h_[l], hn.k = kH, hn.ld = kH;
         mn.x = M_[l], mn.k = kH, mn.ld = kH;
-        uint32_t nch = cdiv(n, kChunk);
-        k_wgrad<<<nch, 256, 0, s>>>(n, hn, mn, dZ_, part_, cpart);
+        k_wgrad<kH / 16><<<dim3(wgrad_grid(n), 2), 256, 0, s>>>(n, wgrad_rows(n), hn, mn, dZ_,
+                                                                part_);
         PPF_HIP(hipGetLastError());
-        k_wgrad_reduce<<<cdiv(2 * kH * kH + kH, kNT), kNT, 0, s>>>(
-            nch, 2 * kH, part_, cpart, grad_ + LpcLayout::Wn(l), grad_ + LpcLayout::cn(l));
-        PPF_HIP(hipGetLastError());
+        PPF_HIP(reduce(wgrad_grid(n), 2 * kH, LpcLayout::Wn(l)));
         Seg dz;
         dz.x = dZ_, dz.k = kH, dz.ld = kH;
         // dX = dZ Wn^T: Wn row-major [128][64] is the transposed operand of
@@ -1112,12 +1292,10 @@ int Lpc::gradient(PcgPlanImpl *plan, const float *val, const float *cdiag, const
             Seg hs, fe;
             hs.x = h_[l], hs.idx = esrc_, hs.k = kH, hs.ld = kH;
             fe.x = f_, fe.k = kFE, fe.ld = kFE;
-            nch = cdiv(E, kChunk);
-            k_wgrad<<<nch, 256, 0, s>>>(E, hs, fe, dY_, part_, cpart);
+            k_wgrad<(kH + kFE) / 16><<<wgrad_grid(E), 256, 0, s>>>(E, wgrad_rows(E), hs, fe, dY_,
+                                                                   part_);
             PPF_HIP(hipGetLastError());
-            k_wgrad_reduce<<<cdiv((kH + kFE) * kH + kH, kNT), kNT, 0, s>>>(
-                nch, kH + kFE, part_, cpart, grad_ + LpcLayout::We(l), grad_ + LpcLayout::ce(l));
-            PPF_HIP(hipGetLastError());
+            PPF_HIP(reduce(wgrad_grid(E), kH + kFE, LpcLayout::We(l)));
             Seg dy;
             dy.x = dY_, dy.k = kH, dy.ld = kH;
             // input gradient of h_src only: the first 64 rows of We
@@ -1137,13 +1315,9 @@ int Lpc::gradient(PcgPlanImpl *plan, const float *val, const float *cdiag, const
     {
         Seg xs, none;
         xs.x = x_, xs.k = kFN, xs.ld = kFN;
-        const uint32_t nch = cdiv(n, kChunk);
-        k_wgrad<<<nch, 256, 0, s>>>(n, xs, none, dZ_, part_, cpart);
+        k_wgrad<kFN / 16><<<wgrad_grid(n), 256, 0, s>>>(n, wgrad_rows(n), xs, none, dZ_, part_);
         PPF_HIP(hipGetLastError());
-        k_wgrad_reduce<<<cdiv(kFN * kH + kH, kNT), kNT, 0, s>>>(nch, kFN, part_, cpart,
-                                                               grad_ + LpcLayout::W0,
-                                                               grad_ + LpcLayout::c0);
-        PPF_HIP(hipGetLastError());
+        PPF_HIP(reduce(wgrad_grid(n), kFN, LpcLayout::W0));
     }
     float h[2];
     PPF_HIP(hipMemcpyAsync(h, scal_, 2 * sizeof(float), hipMemcpyDeviceToHost, s));

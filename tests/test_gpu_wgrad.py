@@ -1,0 +1,41 @@
+"""Weight gradients at row counts around the kernels' steps: fewer rows than
+one staged step (32), one more than a step, one more than a workgroup's
+minimum (256 rows), and several workgroups with ragged last waves."""
+import numpy as np
+import pytest
+import torch
+
+import learned as OL
+from ppf_amd import scenes
+from ppf_amd.learned import LearnedPreconditioner, flatten
+from ppf_amd.solver import BlockJacobiPCG
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [2, 31, 33, 257, 1030])
+def test_weight_gradient_at_ragged_row_counts(dev, n):
+    # chain systems: n rows, 2 (n - 1) edges, 2 n - 1 stored blocks
+    s = scenes.long_row_spd_system(n=n, hubs=0, fan=0, seed=n)
+    t = {k: torch.from_numpy(np.ascontiguousarray(s[k])).to(dev).reshape(-1)
+         for k in ("row_offset", "col_index", "value", "cdiag", "b")}
+    w = OL.init_weights(n, zero_head=False)
+    rng = np.random.default_rng(n)
+    w["Wo"], w["Wg"] = rng.normal(0, 0.3, w["Wo"].shape), rng.normal(0, 0.3, w["Wg"].shape)
+    plan = BlockJacobiPCG(t["row_offset"].int(), t["col_index"].int())
+    lpc = LearnedPreconditioner(flatten(w))
+    lpc.factor(plan, t["value"], t["cdiag"], t["b"])
+    z = OL.probe_vectors(n, 2, seed=n)
+    loss, grad = lpc.gradient(plan, t["value"], t["cdiag"],
+                              torch.from_numpy(z.astype(np.float32)).to(dev).contiguous())
+    g = OL.system_graph(s)
+    x, f = OL.features(g, s["b"])
+    lo, go = OL.backward(w, g, x, f, z)
+    go = flatten(go).astype(np.float64)
+    err = np.linalg.norm(grad - go) / np.linalg.norm(go)
+    print(f"n {n}: loss {loss:.6f} / {lo:.6f}, gradient rel err {err:.2e}")
+    # eight bf16-rounded layers of 2^-8 each: 3e-2. A row left out or taken
+    # twice moves the gradient by about 1 / sqrt(rows) >= 3.1e-2 beyond it.
+    assert err < 3e-2
+    lpc.close()
+    plan.close()

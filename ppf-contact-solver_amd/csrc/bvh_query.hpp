@@ -12,14 +12,17 @@
 namespace ppf {
 
 constexpr int kQueryThreads = 128; // threads per query workgroup
-// Stack entries per thread. A depth-first walk that tests children before
-// pushing them holds at most depth + 1 entries. A Karras tree over 30-bit
-// Morton codes is at most 30 levels deep over distinct codes, plus log2 of
-// the largest run of equal codes (ties split by index): 48 entries cover runs
-// of 2^17. The C3 trees (1-1.5M leaves) are 28-30 levels deep. A deeper walk
-// raises the overflow flag (a capacity error), it never writes past the stack.
-// 48 rather than 64 entries lets 12 one-wave workgroups share a CU's LDS.
-constexpr int kQueryStack = 48;
+// Stack entries per thread. A walk enters one record (two levels of the tree)
+// at a time, goes on with its rightmost overlapping child and pushes the
+// others, so a walk of a tree d levels deep holds at most 3 ceil(d / 2)
+// entries, and far fewer in use. The walks first run with kQueryStack entries
+// (16 KB of LDS per workgroup, ten per CU); a walk that needs more raises the
+// overflow flag and never writes past the stack, and the caller runs the pass
+// again with kDeepStack entries. Those cover every tree of 64 levels; a
+// Karras tree over 30-bit Morton codes is at most 30 levels deep over distinct
+// codes, plus log2 of the largest run of equal codes (ties split by index).
+constexpr int kQueryStack = 32;
+constexpr int kDeepStack = 96;
 
 // A query box and the scene of its query element (0 in a one-scene mesh).
 struct QBox {
@@ -88,32 +91,69 @@ __device__ inline uint32_t root_code(const BvhView &bvh) {
     return bvh.n == 1 ? (bvh.node[2 * (size_t)bvh.root] - 1) | kLeafCode : bvh.root;
 }
 
-// Reads internal node v's walk record and tests both children against q:
-// codes and verdicts (aabb::overlap on the stored boxes and scene tags).
-__device__ inline void enter(const BvhView &bvh, uint32_t v, const QBox &q, uint32_t code[2],
-                             bool ov[2]) {
+// Which leaves a query pairs with: all, or only primitives above (below) its
+// own. The bound prunes subtrees (tags of a tree built with the same bound)
+// and leaves.
+enum Pairing { kPairAll = 0, kPairAbove = 1, kPairBelow = -1 };
+
+// Reads internal node v's walk record and tests its children against q: codes
+// and a bit per overlapping child (aabb::overlap on the stored boxes and
+// scene tags). own: the query's primitive for kPairAbove / kPairBelow. With
+// `inner` (statistics) adds the number of node v's own internal children that
+// overlap q: their boxes are the unions of the stored pairs.
+template <int PAIR>
+__device__ inline uint32_t enter(const BvhView &bvh, uint32_t v, const QBox &q, uint32_t own,
+                                 uint32_t code[4], uint32_t *inner = nullptr) {
     const uint4 *r = reinterpret_cast<const uint4 *>(bvh.rec + (v - bvh.n));
-    const uint4 a = r[0], b = r[1], c = r[2], d = r[3];
-    const float b0[6] = {__uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z),
-                         __uint_as_float(b.w), __uint_as_float(c.x), __uint_as_float(c.y)};
-    const float b1[6] = {__uint_as_float(c.z), __uint_as_float(c.w), __uint_as_float(d.x),
-                         __uint_as_float(d.y), __uint_as_float(d.z), __uint_as_float(d.w)};
-    code[0] = a.x, code[1] = a.y;
-    const uint32_t tag[2] = {a.z, a.w};
+    const uint4 a = r[0], t = r[1];
+    float b[24];
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const float *bx = k ? b1 : b0;
-        ov[k] = (tag[k] == q.scene || tag[k] == kMixedScene) &&
-                (bx[0] <= q.mx[0] && bx[3] >= q.mn[0]) &&
-                (bx[1] <= q.mx[1] && bx[4] >= q.mn[1]) &&
-                (bx[2] <= q.mx[2] && bx[5] >= q.mn[2]);
+    for (int k = 0; k < 6; ++k) {
+        const uint4 w = r[2 + k];
+        b[4 * k] = __uint_as_float(w.x), b[4 * k + 1] = __uint_as_float(w.y);
+        b[4 * k + 2] = __uint_as_float(w.z), b[4 * k + 3] = __uint_as_float(w.w);
     }
+    code[0] = a.x, code[1] = a.y, code[2] = a.z, code[3] = a.w;
+    const uint32_t tag[4] = {t.x, t.y, t.z, t.w};
+    uint32_t hit = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float *bx = b + 6 * k;
+        bool ok = (bx[0] <= q.mx[0]) & (bx[3] >= q.mn[0]) & (bx[1] <= q.mx[1]) &
+                  (bx[4] >= q.mn[1]) & (bx[2] <= q.mx[2]) & (bx[5] >= q.mn[2]);
+        if (bvh.scenes) {
+            ok &= tag[k] == q.scene || tag[k] == kMixedScene;
+        }
+        if (PAIR != kPairAll) {
+            const uint32_t key = (code[k] & kLeafCode) ? code[k] & ~kLeafCode : tag[k];
+            const bool bounded = (code[k] & kLeafCode) != 0 || bvh.bound == PAIR;
+            ok &= !bounded || (PAIR == kPairAbove ? key > own : key < own);
+        }
+        hit |= ok ? 1u << k : 0u;
+    }
+    if (inner) {
+#pragma unroll
+        for (int k = 0; k < 4; k += 2) {
+            const float *u = b + 6 * k, *w = u + 6;
+            bool ok = code[k + 1] != kNoCode;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                ok &= fminf(u[d], w[d]) <= q.mx[d] && fmaxf(u[3 + d], w[3 + d]) >= q.mn[d];
+            }
+            if (bvh.scenes) {
+                ok &= tag[k] != tag[k + 1] || tag[k] == q.scene || tag[k] == kMixedScene;
+            }
+            *inner += ok ? 1u : 0u;
+        }
+    }
+    return hit;
 }
 
-// Work of one lane's tree walks, for the walk statistics: nodes taken off
-// the stack (the root included; an internal one costs its 64-byte walk
-// record, a leaf nothing more), leaves among them, and candidates swept
-// (queued CCD work).
+// Work of one lane's tree walks, for the walk statistics: tree nodes whose
+// box overlaps the query's (what a walk of the binary tree takes off its
+// stack, the root included: the measure of a scene, whatever the records'
+// width), leaves among them, and candidates swept (queued CCD work). The
+// statistics variants of the kernels (STATS) walk without the pairing bounds.
 struct WalkCount {
     uint32_t nodes = 0, leaves = 0, work = 0;
 };
@@ -152,47 +192,72 @@ __device__ inline void walk_flush(unsigned long long *stats, int kind, const Wal
     }
 }
 
-// Visits every leaf whose box overlaps q; `leaf(prim)` returns whether the
-// candidate was accepted. Returns the accepted count. `stk` is this thread's
-// first LDS slot (stride kQueryThreads).
-template <class F>
+// Visits every leaf whose box overlaps q (and that PAIR keeps), from the last
+// leaf to the first; `leaf(prim)` returns whether the candidate was accepted.
+// Returns the accepted count. `stk` is this thread's first LDS slot (stride
+// kQueryThreads). Bound by the dependent record loads and by divergence: two
+// tree levels per load, and lanes walk until every lane holds a leaf or is
+// done, then all run `leaf`, so the candidates' work is not paid for lane by
+// lane. Against one level per 64 B record, leaves taken off one at a time and
+// no pairing bound: vertex queries of 1M independent triangles 3,792 -> 2,378
+// us, their edge queries 2,878 -> 1,885 us; on 8 x 201 x 201 sheets 1,715 ->
+// 1,030 us and 2,401 -> 1,448 us.
+template <int STACK, int PAIR = kPairAll, bool STATS = false, class F>
 __device__ uint32_t traverse(const BvhView &bvh, const QBox &q, uint32_t *stk,
-                             uint32_t *overflow, F &&leaf, WalkCount *wc = nullptr) {
+                             uint32_t *overflow, F &&leaf, uint32_t own = 0,
+                             WalkCount *wc = nullptr) {
     if (bvh.n == 0 || !overlaps(load_box(bvh.box, bvh.root), q)) {
         return 0;
     }
     uint32_t count = 0;
     uint32_t sp = 0;
-    stk[(sp++) * kQueryThreads] = root_code(bvh);
-    while (sp) {
-        const uint32_t v = stk[(--sp) * kQueryThreads];
-        if (wc) {
-            ++wc->nodes;
-        }
-        if (v & kLeafCode) {
-            if (wc) {
-                ++wc->leaves;
+    uint32_t v = root_code(bvh);
+    bool more = true;
+    while (true) {
+        while (more && !(v & kLeafCode)) {
+            uint32_t code[4];
+            const uint32_t hit =
+                enter<STATS ? kPairAll : PAIR>(bvh, v, q, own, code, STATS ? &wc->nodes : nullptr);
+            if (STATS) {
+                ++wc->nodes;
             }
-            if (leaf(v & ~kLeafCode)) {
-                ++count;
+            if (sp + 3 > (uint32_t)STACK) {
+                atomicOr(overflow, 1u);
+                return count;
             }
-            continue;
+            bool next = false;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                if (hit & (1u << k)) {
+                    if (next) {
+                        stk[(sp++) * kQueryThreads] = v;
+                    }
+                    v = code[k];
+                    next = true;
+                }
+            }
+            if (!next) {
+                more = sp != 0;
+                if (more) {
+                    v = stk[(--sp) * kQueryThreads];
+                }
+            }
         }
-        uint32_t code[2];
-        bool ov[2];
-        enter(bvh, v, q, code, ov);
-        if (sp + 2 > (uint32_t)kQueryStack) {
-            atomicOr(overflow, 1u);
+        if (!more) {
             return count;
         }
-        if (ov[0]) {
-            stk[(sp++) * kQueryThreads] = code[0];
+        if (STATS) {
+            ++wc->nodes;
+            ++wc->leaves;
         }
-        if (ov[1]) {
-            stk[(sp++) * kQueryThreads] = code[1];
+        if (leaf(v & ~kLeafCode)) {
+            ++count;
+        }
+        more = sp != 0;
+        if (more) {
+            v = stk[(--sp) * kQueryThreads];
         }
     }
-    return count;
 }
 
 // ---- wave-cooperative traversal --------------------------------------------
@@ -212,16 +277,17 @@ template <int STACK> struct WaveScratchT {
     uint32_t stk[STACK * kWaveQueries];
     uint32_t qid[kWaveQueue], prim[kWaveQueue];
 };
-using WaveScratch = WaveScratchT<kQueryStack>;
 
 __device__ inline uint32_t lanes_below(uint64_t m) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                      __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
+// Line search of 8 x 129 x 129 falling sheets, one-level against two-level
+// records: edge sweeps 1,950 -> 1,692 us, vertex sweeps 810 -> 640 us.
 // `active`: this lane has a query (lanes past the end pass false). All lanes
 // of the workgroup must call it (the rounds are wave uniform).
-template <int STACK, class A, class W>
+template <int PAIR, bool STATS, int STACK, class A, class W>
 __device__ void traverse_wave(const BvhView &bvh, const QBox &q, bool active, uint32_t qid,
                               WaveScratchT<STACK> &ws, uint32_t *overflow, A &&accept, W &&work,
                               WalkCount *wc = nullptr) {
@@ -237,30 +303,30 @@ __device__ void traverse_wave(const BvhView &bvh, const QBox &q, bool active, ui
         uint32_t cand = 0xffffffffu;
         if (sp) {
             const uint32_t v = stk[(--sp) * kWaveQueries];
-            if (wc) {
+            if (STATS) {
                 ++wc->nodes;
             }
             if (v & kLeafCode) {
                 const uint32_t prim = v & ~kLeafCode;
-                if (wc) {
+                if (STATS) {
                     ++wc->leaves;
                 }
                 if (accept(prim)) {
                     cand = prim;
                 }
             } else {
-                uint32_t code[2];
-                bool ov[2];
-                enter(bvh, v, q, code, ov);
-                if (sp + 2 > (uint32_t)STACK) {
+                uint32_t code[4];
+                const uint32_t hit = enter<STATS ? kPairAll : PAIR>(bvh, v, q, qid, code,
+                                                                    STATS ? &wc->nodes : nullptr);
+                if (sp + 4 > (uint32_t)STACK) {
                     atomicOr(overflow, 1u);
                     sp = 0;
                 } else {
-                    if (ov[0]) {
-                        stk[(sp++) * kWaveQueries] = code[0];
-                    }
-                    if (ov[1]) {
-                        stk[(sp++) * kWaveQueries] = code[1];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        if (hit & (1u << k)) {
+                            stk[(sp++) * kWaveQueries] = code[k];
+                        }
                     }
                 }
             }
@@ -279,7 +345,7 @@ __device__ void traverse_wave(const BvhView &bvh, const QBox &q, bool active, ui
             if (lane < take) {
                 const uint32_t at = queued - 1 - lane;
                 work(ws.qid[at], ws.prim[at]);
-                if (wc) {
+                if (STATS) {
                     ++wc->work;
                 }
             }

@@ -307,12 +307,14 @@ __global__ __launch_bounds__(kNT) void k_karras(uint32_t n, const uint32_t *__re
 __global__ __launch_bounds__(kNT) void k_leaf_boxes(PrimSet p, const float *__restrict__ x0,
                                                     const float *__restrict__ x1, float t,
                                                     const uint32_t *__restrict__ node,
-                                                    Aabb *__restrict__ box) {
+                                                    Aabb *__restrict__ box,
+                                                    uint32_t *__restrict__ ext) {
     const uint32_t i = blockIdx.x * kNT + threadIdx.x;
     if (i >= p.n) {
         return;
     }
     const uint32_t prim = node[2 * (size_t)i] - 1;
+    ext[i] = prim;
     const float margin = 0.5f * p.ghat[prim] + p.offset[prim];
     float lo0[3], hi0[3], lo1[3], hi1[3];
     for (int k = 0; k < p.arity; ++k) {
@@ -430,14 +432,19 @@ __global__ __launch_bounds__(kNT) void k_depth_scatter(uint32_t m, uint32_t n,
 __global__ __launch_bounds__(kNT) void k_refit_level(const uint32_t *__restrict__ level,
                                                      uint32_t count,
                                                      const uint32_t *__restrict__ node,
-                                                     Aabb *__restrict__ box) {
+                                                     Aabb *__restrict__ box,
+                                                     uint32_t *__restrict__ ext, int bound) {
     const uint32_t k = blockIdx.x * kNT + threadIdx.x;
     if (k >= count) {
         return;
     }
     const uint32_t par = level[k];
-    const Aabb a = box[node[2 * (size_t)par] - 1];
-    const Aabb b = box[node[2 * (size_t)par + 1] - 1];
+    const uint32_t c0 = node[2 * (size_t)par] - 1, c1 = node[2 * (size_t)par + 1] - 1;
+    const Aabb a = box[c0];
+    const Aabb b = box[c1];
+    if (bound) {
+        ext[par] = bound > 0 ? max(ext[c0], ext[c1]) : min(ext[c0], ext[c1]);
+    }
     Aabb u;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -454,20 +461,38 @@ __global__ __launch_bounds__(kNT) void k_refit_level(const uint32_t *__restrict_
 __global__ __launch_bounds__(kNT) void k_walk_records(uint32_t n,
                                                       const uint32_t *__restrict__ node,
                                                       const Aabb *__restrict__ box,
-                                                      WalkRec *__restrict__ rec) {
+                                                      const uint32_t *__restrict__ ext,
+                                                      bool scenes, WalkRec *__restrict__ rec) {
     const uint32_t i = blockIdx.x * kNT + threadIdx.x;
     if (i + 1 >= n) {
         return;
     }
     const uint32_t v = n + i;
-    WalkRec w;
+    uint32_t ch[4];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
         const uint32_t c = node[2 * (size_t)v + k] - 1;
-        const bool leaf = node[2 * (size_t)c + 1] == 0;
-        w.code[k] = leaf ? (node[2 * (size_t)c] - 1) | kLeafCode : c;
+        const bool leaf = c < n;
+        ch[2 * k] = leaf ? c : node[2 * (size_t)c] - 1;
+        ch[2 * k + 1] = leaf ? kNoCode : node[2 * (size_t)c + 1] - 1;
+    }
+    WalkRec w;
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        if (ch[k] == kNoCode) {
+            w.code[k] = kNoCode;
+            w.tag[k] = kInactiveTag;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                w.box[6 * k + d] = __builtin_inff();
+                w.box[6 * k + 3 + d] = -__builtin_inff();
+            }
+            continue;
+        }
+        const uint32_t c = ch[k];
+        w.code[k] = c < n ? (node[2 * (size_t)c] - 1) | kLeafCode : c;
         const Aabb b = box[c];
-        w.tag[k] = b.active != 0.0f ? __float_as_uint(b.pad) : kInactiveTag;
+        w.tag[k] = !scenes ? ext[c] : b.active != 0.0f ? __float_as_uint(b.pad) : kInactiveTag;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             w.box[6 * k + d] = b.mn[d];
@@ -487,7 +512,7 @@ void Lbvh::release() {
     for (void *p : {(void *)node_, (void *)parent_, (void *)depth_, (void *)level_,
                     (void *)code_,
                     (void *)idx_, (void *)scratch_, (void *)cent_, (void *)part_,
-                    (void *)box_, (void *)rec_, (void *)sb_}) {
+                    (void *)box_, (void *)rec_, (void *)ext_, (void *)sb_}) {
         if (p) {
             (void)dev_free(p);
         }
@@ -496,6 +521,7 @@ void Lbvh::release() {
     cent_ = part_ = nullptr;
     box_ = nullptr;
     rec_ = nullptr;
+    ext_ = nullptr;
     sb_ = nullptr;
     sb_cap_ = 0;
     cap_ = 0;
@@ -519,6 +545,7 @@ int Lbvh::reserve(uint32_t n) {
     PPF_HIP(dev_alloc(&part_, (6 * nb + 6) * sizeof(float)));
     PPF_HIP(dev_alloc(&box_, nodes * sizeof(Aabb)));
     PPF_HIP(dev_alloc(&rec_, std::max<size_t>(n, 1) * sizeof(WalkRec)));
+    PPF_HIP(dev_alloc(&ext_, nodes * sizeof(uint32_t)));
     cap_ = n;
     return PPF_OK;
 }
@@ -534,6 +561,8 @@ int Lbvh::build(const PrimSet &p, const float *x0, const float *x1, float t,
         return PPF_ERR_ARG;
     }
     n_ = p.n;
+    bound_ = p.bound;
+    scenes_ = p.vscene && p.nscene > 1;
     root_ = n_ == 1 ? 0 : n_;
     if (n_ == 0) {
         return PPF_OK;
@@ -643,19 +672,21 @@ int Lbvh::refit(const PrimSet &p, const float *x0, const float *x1, float t,
     if (n_ == 0) {
         return PPF_OK;
     }
-    k_leaf_boxes<<<cdiv(n_, kNT), kNT, 0, s>>>(p, x0, x1, t, node_, box_);
+    k_leaf_boxes<<<cdiv(n_, kNT), kNT, 0, s>>>(p, x0, x1, t, node_, box_, ext_);
     PPF_HIP(hipGetLastError());
     // Inner boxes level by level from the deepest: a kernel boundary orders
     // each level after its children, with no fences or arrival counters.
     for (size_t d = loff_.size() - 1; d-- > 0;) {
         const uint32_t cnt = loff_[d + 1] - loff_[d];
         if (cnt) {
-            k_refit_level<<<cdiv(cnt, kNT), kNT, 0, s>>>(level_ + loff_[d], cnt, node_, box_);
+            k_refit_level<<<cdiv(cnt, kNT), kNT, 0, s>>>(level_ + loff_[d], cnt, node_, box_,
+                                                         ext_, bound_);
             PPF_HIP(hipGetLastError());
         }
     }
     if (n_ > 1) {
-        k_walk_records<<<cdiv(n_ - 1, kNT), kNT, 0, s>>>(n_, node_, box_, rec_);
+        k_walk_records<<<cdiv(n_ - 1, kNT), kNT, 0, s>>>(n_, node_, box_, ext_, scenes_,
+                                                             rec_);
         PPF_HIP(hipGetLastError());
     }
     return PPF_OK;
@@ -668,6 +699,8 @@ BvhView Lbvh::view() const {
     v.node = node_;
     v.box = box_;
     v.rec = rec_;
+    v.scenes = scenes_;
+    v.bound = scenes_ ? 0 : bound_;
     return v;
 }
 

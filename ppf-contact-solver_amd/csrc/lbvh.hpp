@@ -25,17 +25,21 @@ struct alignas(32) Aabb {
 };
 constexpr uint32_t kMixedScene = 0xffffffffu;
 
-// Walk record of internal node n + i (64 B, four 16 B loads): both children's
-// codes, scene tags and boxes, so a walk reads one record per internal node
-// it enters instead of the node and then its children's boxes. A child code
-// is the child's node id, or for a leaf its primitive | kLeafCode. An
-// inactive child's tag is kInactiveTag, which matches no query's scene.
-struct alignas(64) WalkRec {
-    uint32_t code[2];
-    uint32_t tag[2];
-    float box[12]; // child 0 min xyz, max xyz, then child 1
+// Walk record of internal node n + i (128 B, one L2 line, eight 16 B loads):
+// the node's grandchildren in leaf order, two places per child (a leaf child
+// stands for itself in the first; unused places hold kNoCode and a box that
+// overlaps nothing), so a walk takes two levels of the tree per record. A code is the child's node id, or for a leaf its
+// primitive | kLeafCode. The tag is the scene tag of the child's box in a tree
+// of many scenes (an inactive child's is kInactiveTag, which matches no
+// query's scene); in a one-scene tree it is the child's primitive bound
+// (PrimSet::bound), which lets a query skip subtrees without partners.
+struct alignas(128) WalkRec {
+    uint32_t code[4];
+    uint32_t tag[4];
+    float box[24]; // child 0 min xyz, max xyz, then children 1 to 3
 };
 constexpr uint32_t kLeafCode = 0x80000000u;
+constexpr uint32_t kNoCode = 0xffffffffu;
 constexpr uint32_t kInactiveTag = 0xfffffffeu;
 
 struct BvhView {
@@ -44,6 +48,8 @@ struct BvhView {
     const uint32_t *node = nullptr; // 2 words per node
     const Aabb *box = nullptr;
     const WalkRec *rec = nullptr;   // n - 1 records (internal nodes)
+    bool scenes = false;       // tags are scene tags
+    int bound = 0;             // tags are primitive bounds: +1 largest, -1 smallest
 };
 
 // Primitive set a tree is built over: `arity` vertex indices per primitive
@@ -61,6 +67,10 @@ struct PrimSet {
     // with its scene. Null / nscene <= 1: one scene.
     const uint32_t *vscene = nullptr;
     uint32_t nscene = 0;
+    // Primitive bound the walk records of a one-scene tree carry per child: the
+    // largest (+1) or smallest (-1) primitive below it, or none (0). Queries
+    // that pair with higher (lower) primitives only skip the other subtrees.
+    int bound = 0;
 };
 
 class Lbvh {
@@ -86,6 +96,9 @@ class Lbvh {
     float *cent_ = nullptr, *part_ = nullptr;
     Aabb *box_ = nullptr;
     WalkRec *rec_ = nullptr;
+    uint32_t *ext_ = nullptr; // primitive bound per node
+    int bound_ = 0;
+    bool scenes_ = false;
     uint32_t *sb_ = nullptr; // per-scene centroid bounds (many scenes)
     size_t sb_cap_ = 0;
     void release();

@@ -19,13 +19,13 @@ namespace ppf {
 
 namespace {
 
-constexpr int kStack = kQueryStack;
+constexpr int kStack = kDeepStack;
 // The sweeps first run with shorter stacks: 36 entries (10 KB of LDS per
-// one-wave workgroup) let 16 workgroups share a CU, 4 waves per SIMD, against
-// 12 with 48. A walk deeper than 35 levels flags an overflow, and the pass
-// runs again with 48-entry stacks.
+// one-wave workgroup) let 16 workgroups share a CU, 4 waves per SIMD. A walk
+// that needs more flags an overflow, and the pass runs again with kDeepStack
+// entries.
 constexpr int kShortStack = 36;
-constexpr int kLsWaves = 4;
+constexpr int ls_waves(int stack) { return stack <= kShortStack ? 4 : 2; } // per SIMD
 using Box6 = QBox;
 
 struct LsCtx {
@@ -87,8 +87,8 @@ __device__ inline void wave_min_out(uint32_t *out, float best, float above) {
 // (contact.cu:2266-2316) and vertex vs static face (contact.cu:1956-1994).
 // The filters run on the query's lane while it walks; the sweeps run from the
 // wave queue.
-template <int STACK>
-__global__ __launch_bounds__(kWQ, kLsWaves) void k_ls_vertex(LsCtx c) {
+template <int STACK, bool STATS>
+__global__ __launch_bounds__(kWQ, ls_waves(STACK)) void k_ls_vertex(LsCtx c) {
     __shared__ WaveScratchT<STACK> ws;
     const uint32_t leaf = xcd_logical_block() * kWQ + threadIdx.x;
     const bool active = leaf < c.vb.n;
@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kWQ, kLsWaves) void k_ls_vertex(LsCtx c) {
     const uint32_t ibody = active ? m.vbody[i] : 0u;
     float best = max_t;
     WalkCount wc;
-    traverse_wave(
+    traverse_wave<kPairAll, STATS>(
         c.fb, q, active, i, ws, c.out + 3,
         [&](uint32_t fi) {
             const uint32_t f0 = m.face[3 * (size_t)fi];
@@ -138,7 +138,7 @@ __global__ __launch_bounds__(kWQ, kLsWaves) void k_ls_vertex(LsCtx c) {
             }
             note(c, ovl, r, best, vertex_scene(m.vscene, m.nscene, v));
         }, &wc);
-    traverse_wave(
+    traverse_wave<kPairBelow, STATS>(
         c.vb, q, active, i, ws, c.out + 3,
         [&](uint32_t j) {
             const bool either = idyn || (m.vflag[j] & 1u) == 0;
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(kWQ, kLsWaves) void k_ls_vertex(LsCtx c) {
         }, &wc);
     if (c.sm.nf) {
         const bool go = active && idyn && c.lp.vmass[i] != 0.0f;
-        traverse_wave(
+        traverse_wave<kPairAll, STATS>(
             c.sfb, q, go, i, ws, c.out + 3, [&](uint32_t) { return true; },
             [&](uint32_t v, uint32_t fi) {
                 const uint32_t f0 = c.sm.face[3 * (size_t)fi], f1 = c.sm.face[3 * (size_t)fi + 1],
@@ -172,12 +172,12 @@ __global__ __launch_bounds__(kWQ, kLsWaves) void k_ls_vertex(LsCtx c) {
             }, &wc);
     }
     wave_min_out(c.out + 0, best, max_t);
-    walk_flush(c.stats, kWalkLsVertex, wc, active);
+    if (STATS) walk_flush(c.stats, kWalkLsVertex, wc, active);
 }
 
 // static vertex vs dynamic face (contact.cu:1996-2034)
 template <int STACK>
-__global__ __launch_bounds__(kWQ, kLsWaves) void k_ls_static_vertex(LsCtx c) {
+__global__ __launch_bounds__(kWQ, ls_waves(STACK)) void k_ls_static_vertex(LsCtx c) {
     __shared__ WaveScratchT<STACK> ws;
     const uint32_t i = xcd_logical_block() * kWQ + threadIdx.x;
     const bool active = i < c.sm.nv;
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(kWQ, kLsWaves) void k_ls_static_vertex(LsCtx c) {
     const Box6 q{{p.x - qm, p.y - qm, p.z - qm}, {p.x + qm, p.y + qm, p.z + qm},
                  vertex_scene(c.sm.vscene, m.nscene, ii)};
     float best = max_t;
-    traverse_wave(
+    traverse_wave<kPairAll, false>(
         c.fb, q, active, ii, ws, c.out + 3,
         [&](uint32_t fi) { return (m.fflag[fi] & 1u) == 0 && c.lp.fmass[fi] > 0.0f; },
         [&](uint32_t v, uint32_t fi) {
@@ -286,8 +286,8 @@ __global__ __launch_bounds__(256) void k_ls_analytic(LsCtx c) {
 }
 
 // edge-edge and edge vs static edge, seeded by the vertex-face minimum.
-template <int STACK>
-__global__ __launch_bounds__(kWQ, kLsWaves) void k_ls_edge(LsCtx c) {
+template <int STACK, bool STATS>
+__global__ __launch_bounds__(kWQ, ls_waves(STACK)) void k_ls_edge(LsCtx c) {
     __shared__ WaveScratchT<STACK> ws;
     const uint32_t leaf = xcd_logical_block() * kWQ + threadIdx.x;
     const bool active = leaf < c.eb.n;
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(kWQ, kLsWaves) void k_ls_edge(LsCtx c) {
     const uint32_t abody = m.vbody[a0];
     float best = seed;
     WalkCount wc;
-    traverse_wave(
+    traverse_wave<kPairAbove, STATS>(
         c.eb, q, active, ei, ws, c.out + 3,
         [&](uint32_t ej) {
             const uint32_t b0i = m.edge[2 * (size_t)ej];
@@ -365,7 +365,7 @@ __global__ __launch_bounds__(kWQ, kLsWaves) void k_ls_edge(LsCtx c) {
         }, &wc);
     if (c.sm.ne) {
         const bool go = active && edyn && c.lp.emass[ei] > 0.0f;
-        traverse_wave(
+        traverse_wave<kPairAll, STATS>(
             c.seb, q, go, ei, ws, c.out + 3, [&](uint32_t) { return true; },
             [&](uint32_t e, uint32_t sj) {
                 const uint32_t e0 = m.edge[2 * (size_t)e], e1 = m.edge[2 * (size_t)e + 1];
@@ -382,7 +382,7 @@ __global__ __launch_bounds__(kWQ, kLsWaves) void k_ls_edge(LsCtx c) {
             }, &wc);
     }
     wave_min_out(c.out + 1, best, seed);
-    walk_flush(c.stats, kWalkLsEdge, wc, active);
+    if (STATS) walk_flush(c.stats, kWalkLsEdge, wc, active);
 }
 
 template <int C, int SPLIT>
@@ -470,6 +470,7 @@ int LineSearch::run(const ppf_contact_mesh &m, const ppf_static_mesh *sm,
     v.n = m.nv, v.arity = 1, v.elem = nullptr, v.ghat = m.v_ghat, v.offset = m.v_off;
     f.vscene = e.vscene = v.vscene = m.vscene;
     f.nscene = e.nscene = v.nscene = m.nscene;
+    e.bound = 1, v.bound = -1; // edge queries pair upward, vertex queries downward
     const bool fresh = rebuild || face_.view().n != m.nf || edge_.view().n != m.ne ||
                        vert_.view().n != m.nv;
     int rc;
@@ -524,7 +525,11 @@ int LineSearch::run(const ppf_contact_mesh &m, const ppf_static_mesh *sm,
         constexpr int D = decltype(stack)::value;
         if (m.nv) {
             WalkClock clk(kWalkLsVertex, s);
-            k_ls_vertex<D><<<xcd_grid(cdiv(m.nv, kWQ)), kWQ, 0, s>>>(c);
+            if (c.stats) {
+                k_ls_vertex<kStack, true><<<xcd_grid(cdiv(m.nv, kWQ)), kWQ, 0, s>>>(c);
+            } else {
+                k_ls_vertex<D, false><<<xcd_grid(cdiv(m.nv, kWQ)), kWQ, 0, s>>>(c);
+            }
             PPF_HIP(hipGetLastError());
             clk.stop();
         }
@@ -538,7 +543,11 @@ int LineSearch::run(const ppf_contact_mesh &m, const ppf_static_mesh *sm,
         }
         if (m.ne) {
             WalkClock clk(kWalkLsEdge, s);
-            k_ls_edge<D><<<xcd_grid(cdiv(m.ne, kWQ)), kWQ, 0, s>>>(c);
+            if (c.stats) {
+                k_ls_edge<kStack, true><<<xcd_grid(cdiv(m.ne, kWQ)), kWQ, 0, s>>>(c);
+            } else {
+                k_ls_edge<D, false><<<xcd_grid(cdiv(m.ne, kWQ)), kWQ, 0, s>>>(c);
+            }
             PPF_HIP(hipGetLastError());
             clk.stop();
         }

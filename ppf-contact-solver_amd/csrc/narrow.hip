@@ -21,7 +21,6 @@ namespace ppf {
 namespace {
 
 constexpr int kQT = kQueryThreads;
-constexpr int kStack = kQueryStack;
 using Q = QBox;
 
 // Pairs the count pass keeps per query. The fill pass then copies them
@@ -87,9 +86,9 @@ __device__ inline bool query_pos(const Ctx &c, uint32_t n, uint32_t &leaf_pos) {
     return true;
 }
 
-template <bool FILL>
+template <bool FILL, int STACK, bool STATS = false>
 __global__ __launch_bounds__(kQT) void k_vertex_queries(Ctx c) {
-    __shared__ uint32_t stk_all[kStack * kQT];
+    __shared__ uint32_t stk_all[STACK * kQT];
     uint32_t leaf_pos;
     const ppf_contact_mesh &m = c.m;
     const bool has = query_pos<FILL>(c, c.vb.n, leaf_pos);
@@ -108,7 +107,7 @@ __global__ __launch_bounds__(kQT) void k_vertex_queries(Ctx c) {
     uint64_t slot = FILL ? (uint64_t)c.ofs[leaf_pos] : 0;
     uint32_t total = 0;
     // point-face (contact.cu:717-785)
-    total += traverse(c.fb, q, stk, c.overflow, [&](uint32_t fi) {
+    total += traverse<STACK, kPairAll, STATS>(c.fb, q, stk, c.overflow, [&](uint32_t fi) {
         const uint32_t f0 = m.face[3 * (size_t)fi], f1 = m.face[3 * (size_t)fi + 1],
                        f2 = m.face[3 * (size_t)fi + 2];
         const bool either_dyn = vdyn(m, i) || (m.fflag[fi] & 1u) == 0;
@@ -132,9 +131,9 @@ __global__ __launch_bounds__(kQT) void k_vertex_queries(Ctx c) {
             return true;
         }
         return false;
-    }, &wc);
+    }, 0u, &wc);
     // point-edge (contact.cu:622-715)
-    total += traverse(c.eb, q, stk, c.overflow, [&](uint32_t ei) {
+    total += traverse<STACK, kPairAll, STATS>(c.eb, q, stk, c.overflow, [&](uint32_t ei) {
         const uint32_t e0 = m.edge[2 * (size_t)ei], e1 = m.edge[2 * (size_t)ei + 1];
         const bool either_dyn = vdyn(m, i) || (m.eflag[ei] & 1u) == 0;
         const bool same_body = m.vbody[i] != 0 && m.vbody[i] == m.vbody[e0];
@@ -181,9 +180,9 @@ __global__ __launch_bounds__(kQT) void k_vertex_queries(Ctx c) {
             return true;
         }
         return false;
-    }, &wc);
+    }, 0u, &wc);
     // point-point (contact.cu:432-620)
-    total += traverse(c.vb, q, stk, c.overflow, [&](uint32_t j) {
+    total += traverse<STACK, kPairBelow, STATS>(c.vb, q, stk, c.overflow, [&](uint32_t j) {
         const bool either_dyn = vdyn(m, i) || vdyn(m, j);
         const bool same_body = m.vbody[i] != 0 && m.vbody[i] == m.vbody[j];
         const bool both_col = vcol(m, i) && vcol(m, j);
@@ -237,20 +236,20 @@ __global__ __launch_bounds__(kQT) void k_vertex_queries(Ctx c) {
             return true;
         }
         return false;
-    }, &wc);
+    }, i, &wc);
     if (!FILL) {
         c.cnt[leaf_pos] = total;
     }
     }();
-    if (!FILL) {
+    if (STATS) {
         walk_flush(c.stats, kWalkProxVertex, wc, has);
     }
 }
 
 // edge-edge (contact.cu:787-870), queries in edge-BVH leaf order.
-template <bool FILL>
+template <bool FILL, int STACK, bool STATS = false>
 __global__ __launch_bounds__(kQT) void k_edge_queries(Ctx c) {
-    __shared__ uint32_t stk_all[kStack * kQT];
+    __shared__ uint32_t stk_all[STACK * kQT];
     uint32_t leaf_pos;
     const ppf_contact_mesh &m = c.m;
     const bool has = query_pos<FILL>(c, c.eb.n, leaf_pos);
@@ -279,7 +278,7 @@ __global__ __launch_bounds__(kQT) void k_edge_queries(Ctx c) {
     q.scene = vertex_scene(m.vscene, m.nscene, a0);
     const uint32_t qpos = c.vb.n + leaf_pos;
     uint64_t slot = FILL ? (uint64_t)c.ofs[qpos] : 0;
-    const uint32_t total = traverse(c.eb, q, stk, c.overflow, [&](uint32_t ej) {
+    const uint32_t total = traverse<STACK, kPairAbove, STATS>(c.eb, q, stk, c.overflow, [&](uint32_t ej) {
         const uint32_t b0 = m.edge[2 * (size_t)ej], b1 = m.edge[2 * (size_t)ej + 1];
         const bool either_dyn = (m.eflag[ei] & 1u) == 0 || (m.eflag[ej] & 1u) == 0;
         const bool same_body = m.vbody[a0] != 0 && m.vbody[a0] == m.vbody[b0];
@@ -305,12 +304,12 @@ __global__ __launch_bounds__(kQT) void k_edge_queries(Ctx c) {
             return true;
         }
         return false;
-    }, &wc);
+    }, ei, &wc);
     if (!FILL) {
         c.cnt[qpos] = total;
     }
     }();
-    if (!FILL) {
+    if (STATS) {
         walk_flush(c.stats, kWalkProxEdge, wc, has);
     }
 }
@@ -392,8 +391,8 @@ __device__ inline f3 SX(const ppf_static_mesh &sm, uint32_t v) {
 }
 
 // Dynamic vertex vs static face (kind 4), one thread per vertex leaf.
-template <bool FILL> __global__ __launch_bounds__(kQT) void k_m2c(SCtx c) {
-    __shared__ uint32_t stk_all[kStack * kQT];
+template <bool FILL, int STACK> __global__ __launch_bounds__(kQT) void k_m2c(SCtx c) {
+    __shared__ uint32_t stk_all[STACK * kQT];
     const uint32_t qpos = blockIdx.x * kQT + threadIdx.x;
     if (qpos >= c.vb.n) {
         return;
@@ -407,7 +406,7 @@ template <bool FILL> __global__ __launch_bounds__(kQT) void k_m2c(SCtx c) {
         const f3 p = X(m, i);
         QBox q = point_box(p, 0.5f * m.v_ghat[i] + m.v_off[i]);
         q.scene = vertex_scene(m.vscene, m.nscene, i);
-        total = traverse(c.sfb, q, stk, c.overflow, [&](uint32_t fi) {
+        total = traverse<STACK>(c.sfb, q, stk, c.overflow, [&](uint32_t fi) {
             const uint32_t f0 = c.sm.face[3 * (size_t)fi], f1 = c.sm.face[3 * (size_t)fi + 1],
                            f2 = c.sm.face[3 * (size_t)fi + 2];
             const f3 t0 = SX(c.sm, f0) - p, t1 = SX(c.sm, f1) - p, t2 = SX(c.sm, f2) - p;
@@ -430,8 +429,8 @@ template <bool FILL> __global__ __launch_bounds__(kQT) void k_m2c(SCtx c) {
 }
 
 // Static vertex vs dynamic face (kind 5), one thread per static vertex.
-template <bool FILL> __global__ __launch_bounds__(kQT) void k_c2m(SCtx c) {
-    __shared__ uint32_t stk_all[kStack * kQT];
+template <bool FILL, int STACK> __global__ __launch_bounds__(kQT) void k_c2m(SCtx c) {
+    __shared__ uint32_t stk_all[STACK * kQT];
     const uint32_t sv = blockIdx.x * kQT + threadIdx.x;
     if (sv >= c.sm.nv) {
         return;
@@ -443,7 +442,7 @@ template <bool FILL> __global__ __launch_bounds__(kQT) void k_c2m(SCtx c) {
     const f3 y = SX(c.sm, sv);
     QBox q = point_box(y, 0.5f * c.sm.v_ghat[sv] + c.sm.v_off[sv]);
     q.scene = vertex_scene(c.sm.vscene, m.nscene, sv);
-    const uint32_t total = traverse(c.fb, q, stk, c.overflow, [&](uint32_t fi) {
+    const uint32_t total = traverse<STACK>(c.fb, q, stk, c.overflow, [&](uint32_t fi) {
         if ((m.fflag[fi] & 1u) != 0 || !(c.fmass[fi] > 0.0f)) {
             return false;
         }
@@ -468,8 +467,8 @@ template <bool FILL> __global__ __launch_bounds__(kQT) void k_c2m(SCtx c) {
 }
 
 // Dynamic edge vs static edge (kind 6), one thread per edge leaf.
-template <bool FILL> __global__ __launch_bounds__(kQT) void k_cm_ee(SCtx c) {
-    __shared__ uint32_t stk_all[kStack * kQT];
+template <bool FILL, int STACK> __global__ __launch_bounds__(kQT) void k_cm_ee(SCtx c) {
+    __shared__ uint32_t stk_all[STACK * kQT];
     const uint32_t lp = blockIdx.x * kQT + threadIdx.x;
     if (lp >= c.eb.n) {
         return;
@@ -485,7 +484,7 @@ template <bool FILL> __global__ __launch_bounds__(kQT) void k_cm_ee(SCtx c) {
         const f3 p0 = X(m, a0), p1 = X(m, a1);
         QBox q = seg_box(p0, p1, 0.5f * m.e_ghat[ei] + m.e_off[ei]);
         q.scene = vertex_scene(m.vscene, m.nscene, a0);
-        total = traverse(c.seb, q, stk, c.overflow, [&](uint32_t sj) {
+        total = traverse<STACK>(c.seb, q, stk, c.overflow, [&](uint32_t sj) {
             const uint32_t b0 = c.sm.edge[2 * (size_t)sj], b1 = c.sm.edge[2 * (size_t)sj + 1];
             const f3 q0 = SX(c.sm, b0), q1 = SX(c.sm, b1);
             float w[4];
@@ -554,6 +553,7 @@ int Narrow::build_trees(const ppf_contact_mesh &m, hipStream_t s) {
     v.n = m.nv, v.arity = 1, v.elem = nullptr, v.ghat = m.v_ghat, v.offset = m.v_off;
     f.vscene = e.vscene = v.vscene = m.vscene;
     f.nscene = e.nscene = v.nscene = m.nscene;
+    e.bound = 1, v.bound = -1; // edge queries pair upward, vertex queries downward
     int rc = face_.build(f, m.x, nullptr, 0.0f, s);
     if (rc == PPF_OK) {
         rc = edge_.build(e, m.x, nullptr, 0.0f, s);
@@ -574,6 +574,7 @@ int Narrow::refit_trees(const ppf_contact_mesh &m, hipStream_t s) {
     v.n = m.nv, v.arity = 1, v.elem = nullptr, v.ghat = m.v_ghat, v.offset = m.v_off;
     f.vscene = e.vscene = v.vscene = m.vscene;
     f.nscene = e.nscene = v.nscene = m.nscene;
+    e.bound = 1, v.bound = -1; // edge queries pair upward, vertex queries downward
     int rc = face_.refit(f, m.x, nullptr, 0.0f, s);
     if (rc == PPF_OK) {
         rc = edge_.refit(e, m.x, nullptr, 0.0f, s);
@@ -591,6 +592,23 @@ int Narrow::proximity(const ppf_contact_mesh &m, ppf_pair *out, uint64_t cap,
     if (rc != PPF_OK) {
         return rc;
     }
+    rc = proximity_pass<kQueryStack>(m, out, cap, count, s);
+    if (rc == PPF_OK && h_flags_[0]) { // a walk needs the deep stacks
+        rc = proximity_pass<kDeepStack>(m, out, cap, count, s);
+    }
+    if (rc == PPF_OK && h_flags_[0]) {
+        set_error("proximity: a BVH traversal exceeded its %d-entry stack", kDeepStack);
+        return PPF_ERR_CAPACITY;
+    }
+    return rc;
+}
+
+// One enumeration with stacks of STACK entries; h_flags_[0] is set if a walk
+// ran out of them (the pairs are then incomplete).
+template <int STACK>
+int Narrow::proximity_pass(const ppf_contact_mesh &m, ppf_pair *out, uint64_t cap,
+                           uint64_t *count, hipStream_t s) {
+    const uint32_t nq = m.nv + m.ne;
     PPF_HIP(hipMemsetAsync(flags_, 0, 4 * sizeof(uint32_t), s));
     const bool fill = out && cap;
     Ctx c;
@@ -609,13 +627,23 @@ int Narrow::proximity(const ppf_contact_mesh &m, ppf_pair *out, uint64_t cap,
     c.stats = walk_stats_device();
     if (m.nv) {
         WalkClock clk(kWalkProxVertex, s);
-        k_vertex_queries<false><<<xcd_grid(cdiv(m.nv, kQT)), kQT, 0, s>>>(c);
+        if (c.stats) {
+            k_vertex_queries<false, kDeepStack, true>
+                <<<xcd_grid(cdiv(m.nv, kQT)), kQT, 0, s>>>(c);
+        } else {
+            k_vertex_queries<false, STACK><<<xcd_grid(cdiv(m.nv, kQT)), kQT, 0, s>>>(c);
+        }
         PPF_HIP(hipGetLastError());
         clk.stop();
     }
     if (m.ne) {
         WalkClock clk(kWalkProxEdge, s);
-        k_edge_queries<false><<<xcd_grid(cdiv(m.ne, kQT)), kQT, 0, s>>>(c);
+        if (c.stats) {
+            k_edge_queries<false, kDeepStack, true>
+                <<<xcd_grid(cdiv(m.ne, kQT)), kQT, 0, s>>>(c);
+        } else {
+            k_edge_queries<false, STACK><<<xcd_grid(cdiv(m.ne, kQT)), kQT, 0, s>>>(c);
+        }
         PPF_HIP(hipGetLastError());
         clk.stop();
     }
@@ -634,28 +662,24 @@ int Narrow::proximity(const ppf_contact_mesh &m, ppf_pair *out, uint64_t cap,
                            hipMemcpyDeviceToHost, s));
     PPF_HIP(hipStreamSynchronize(s));
     *count = h_flags_[4];
-    if (fill) {
+    if (fill && !h_flags_[0]) {
         const uint32_t nv_redo = h_flags_[2], ne_redo = h_flags_[3];
         if (nv_redo) {
             Ctx cv = c;
             cv.nredo = nv_redo;
-            k_vertex_queries<true><<<xcd_grid(cdiv(nv_redo, kQT)), kQT, 0, s>>>(cv);
+            k_vertex_queries<true, STACK><<<xcd_grid(cdiv(nv_redo, kQT)), kQT, 0, s>>>(cv);
             PPF_HIP(hipGetLastError());
         }
         if (ne_redo) {
             Ctx ce = c;
             ce.redo = redo_ + m.nv;
             ce.nredo = ne_redo;
-            k_edge_queries<true><<<xcd_grid(cdiv(ne_redo, kQT)), kQT, 0, s>>>(ce);
+            k_edge_queries<true, STACK><<<xcd_grid(cdiv(ne_redo, kQT)), kQT, 0, s>>>(ce);
             PPF_HIP(hipGetLastError());
         }
         PPF_HIP(hipMemcpyAsync(h_flags_, flags_, 4 * sizeof(uint32_t),
                                hipMemcpyDeviceToHost, s));
         PPF_HIP(hipStreamSynchronize(s));
-    }
-    if (h_flags_[0]) {
-        set_error("proximity: a BVH traversal exceeded its %d-entry stack", kStack);
-        return PPF_ERR_CAPACITY;
     }
     return PPF_OK;
 }
@@ -700,6 +724,24 @@ int Narrow::static_proximity(const ppf_contact_mesh &m, const ppf_static_mesh &s
     if (rc != PPF_OK) {
         return rc;
     }
+    rc = static_pass<kQueryStack>(m, sm, vmass, emass, fmass, out, cap, count, s);
+    if (rc == PPF_OK && h_flags_[0]) { // a walk needs the deep stacks
+        rc = static_pass<kDeepStack>(m, sm, vmass, emass, fmass, out, cap, count, s);
+    }
+    if (rc == PPF_OK && h_flags_[0]) {
+        set_error("static proximity: a BVH traversal exceeded its %d-entry stack", kDeepStack);
+        return PPF_ERR_CAPACITY;
+    }
+    return rc;
+}
+
+// One enumeration of the collision-mesh pairs, as proximity_pass.
+template <int STACK>
+int Narrow::static_pass(const ppf_contact_mesh &m, const ppf_static_mesh &sm, const float *vmass,
+                        const float *emass, const float *fmass, ppf_pair *out, uint64_t cap,
+                        uint64_t *count, hipStream_t s) {
+    const uint32_t nq = m.nv + sm.nv + m.ne;
+    int rc;
     PPF_HIP(hipMemsetAsync(flags_, 0, 4 * sizeof(uint32_t), s));
     SCtx c;
     c.m = m;
@@ -719,16 +761,16 @@ int Narrow::static_proximity(const ppf_contact_mesh &m, const ppf_static_mesh &s
     c.overflow = flags_;
     auto launch = [&](bool fill) -> int {
         if (m.nv) {
-            if (fill) k_m2c<true><<<cdiv(m.nv, kQT), kQT, 0, s>>>(c);
-            else k_m2c<false><<<cdiv(m.nv, kQT), kQT, 0, s>>>(c);
+            if (fill) k_m2c<true, STACK><<<cdiv(m.nv, kQT), kQT, 0, s>>>(c);
+            else k_m2c<false, STACK><<<cdiv(m.nv, kQT), kQT, 0, s>>>(c);
             PPF_HIP(hipGetLastError());
         }
-        if (fill) k_c2m<true><<<cdiv(sm.nv, kQT), kQT, 0, s>>>(c);
-        else k_c2m<false><<<cdiv(sm.nv, kQT), kQT, 0, s>>>(c);
+        if (fill) k_c2m<true, STACK><<<cdiv(sm.nv, kQT), kQT, 0, s>>>(c);
+        else k_c2m<false, STACK><<<cdiv(sm.nv, kQT), kQT, 0, s>>>(c);
         PPF_HIP(hipGetLastError());
         if (m.ne) {
-            if (fill) k_cm_ee<true><<<cdiv(m.ne, kQT), kQT, 0, s>>>(c);
-            else k_cm_ee<false><<<cdiv(m.ne, kQT), kQT, 0, s>>>(c);
+            if (fill) k_cm_ee<true, STACK><<<cdiv(m.ne, kQT), kQT, 0, s>>>(c);
+            else k_cm_ee<false, STACK><<<cdiv(m.ne, kQT), kQT, 0, s>>>(c);
             PPF_HIP(hipGetLastError());
         }
         return PPF_OK;
@@ -751,10 +793,6 @@ int Narrow::static_proximity(const ppf_contact_mesh &m, const ppf_static_mesh &s
     }
     PPF_HIP(hipMemcpyAsync(h_flags_, flags_, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     PPF_HIP(hipStreamSynchronize(s));
-    if (h_flags_[0]) {
-        set_error("static proximity: a BVH traversal exceeded its %d-entry stack", kStack);
-        return PPF_ERR_CAPACITY;
-    }
     return PPF_OK;
 }
 

@@ -27,6 +27,13 @@ class Narrow {
 
   private:
     int reserve(uint32_t queries);
+    template <int STACK>
+    int proximity_pass(const ppf_contact_mesh &m, ppf_pair *out, uint64_t cap, uint64_t *count,
+                       hipStream_t s);
+    template <int STACK>
+    int static_pass(const ppf_contact_mesh &m, const ppf_static_mesh &sm, const float *vmass,
+                    const float *emass, const float *fmass, ppf_pair *out, uint64_t cap,
+                    uint64_t *count, hipStream_t s);
     // Trees of the collision mesh (nscene: the dynamic mesh's scene count).
     int build_static(const ppf_static_mesh &sm, uint32_t nscene, hipStream_t s);
     Lbvh face_, edge_, vert_, sface_, sedge_;

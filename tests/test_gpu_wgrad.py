@@ -34,8 +34,11 @@ def test_weight_gradient_at_ragged_row_counts(dev, n):
     go = flatten(go).astype(np.float64)
     err = np.linalg.norm(grad - go) / np.linalg.norm(go)
     print(f"n {n}: loss {loss:.6f} / {lo:.6f}, gradient rel err {err:.2e}")
-    # eight bf16-rounded layers of 2^-8 each: 3e-2. A row left out or taken
-    # twice moves the gradient by about 1 / sqrt(rows) >= 3.1e-2 beyond it.
-    assert err < 3e-2
+    # bf16 roundings on the way of a gradient: x, h0, then m, M, h of three
+    # layers forward, dZ and dY of three layers and dZ0 backward: 18, and the
+    # weights' own: 19 of at most 2^-9 each, 3.7e-2 if all go one way. A ragged
+    # tail left out (n mod 32 rows: 2, 31, 1, 1, 6) moves the gradient by
+    # sqrt(tail / n): 6.2e-2 at the least (n = 257).
+    assert err < 19 * 2.0 ** -9
     lpc.close()
     plan.close()

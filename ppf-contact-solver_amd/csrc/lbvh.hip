@@ -3,9 +3,10 @@
 // Tree semantics follow lbvh/lbvh.cu:108-385 (Morton quantization, Karras
 // split with the index tie-break) and the swept leaf boxes of
 // lbvh/lbvh.cu:623-731; the inner boxes are unions of the children. The
-// per-level launches and host round trips of the reference are replaced by a
-// single bottom-up kernel with per-node arrival counters: the second child to
-// arrive writes the union and continues upward.
+// per-level launches and host round trips of the reference are replaced by
+// treelets: a node whose leaves lie in one block of 1,024 is refit in that
+// block's workgroup, in LDS; the few nodes across block borders follow in one
+// launch per 32-fold larger block.
 #include "lbvh.hpp"
 #include <algorithm>
 #include "ppf_mi355x.h"
@@ -16,7 +17,44 @@ namespace ppf {
 namespace {
 
 constexpr int kNT = 256;
-constexpr uint32_t kNoParent = 0xffffffffu;
+
+// Treelet classes: a node of class c has its leaves in one aligned block of
+// 2^class_shift(c) leaves and not in a smaller class's block. A node across a
+// border of class c - 1 blocks lies on the nested chain of that border, whose
+// members have distinct common-prefix lengths: at most 30 code bits, 32 scene
+// bits and class_shift(c) tie bits, so the 31 borders inside a class c block
+// (c >= 1) hold at most 31 x 94 = 2,914 nodes (about 320 in meshes).
+constexpr uint32_t kTreelet = 1024; // leaves of a class 0 block
+constexpr uint32_t kTopCap = 3072;  // nodes of one larger block
+constexpr uint32_t kClassBits = 28; // rank word: class << kClassBits | place
+__host__ __device__ inline uint32_t class_shift(uint32_t c) { return 10u + 5u * c; }
+__host__ __device__ inline uint32_t class_blocks(uint32_t n, uint32_t c) {
+    const uint32_t sh = class_shift(c);
+    return sh >= 32 ? 1u : (uint32_t)(((uint64_t)n + (1ull << sh) - 1) >> sh);
+}
+__host__ __device__ inline uint32_t node_class(uint32_t l, uint32_t r) {
+    uint32_t c = 0;
+    while (class_shift(c) < 32 && (l >> class_shift(c)) != (r >> class_shift(c))) {
+        ++c;
+    }
+    return c;
+}
+// Classes beyond 0 a tree of n leaves needs, and the first block of class c
+// in the lists.
+uint32_t top_classes(uint32_t n) {
+    uint32_t c = 0;
+    while (class_blocks(n, c) > 1) {
+        ++c;
+    }
+    return c;
+}
+__host__ __device__ inline uint32_t class_base(uint32_t n, uint32_t c) {
+    uint32_t b = 0;
+    for (uint32_t k = 1; k < c; ++k) {
+        b += class_blocks(n, k);
+    }
+    return b;
+}
 
 __device__ inline uint32_t prim_vertex(const PrimSet &p, uint32_t i, int k) {
     return p.elem ? p.elem[(size_t)i * p.arity + k] : i;
@@ -254,20 +292,18 @@ __device__ inline int lcp(const uint32_t *__restrict__ k, const uint32_t *__rest
     return base + __clz(a ^ b);
 }
 
-// Karras radix tree over the sorted codes (lbvh.cu:305-385), parents inline.
+// Karras radix tree over the sorted codes (lbvh.cu:305-385), and the treelet
+// class of every internal node.
 __global__ __launch_bounds__(kNT) void k_karras(uint32_t n, const uint32_t *__restrict__ k,
                                                 const uint32_t *__restrict__ sk,
                                                 const uint32_t *__restrict__ idx,
                                                 uint32_t *__restrict__ node,
-                                                uint32_t *__restrict__ parent) {
+                                                uint32_t *__restrict__ rank) {
     const int i = blockIdx.x * kNT + threadIdx.x;
     const int nn = (int)n;
     if (i < nn) {
         node[2 * (size_t)i] = idx[i] + 1;
         node[2 * (size_t)i + 1] = 0;
-    }
-    if (i == 0) {
-        parent[nn == 1 ? 0 : n] = kNoParent;
     }
     if (i >= nn - 1) {
         return;
@@ -299,22 +335,71 @@ __global__ __launch_bounds__(kNT) void k_karras(uint32_t n, const uint32_t *__re
     const uint32_t rc = (split + 1 == r) ? (uint32_t)r : n + (uint32_t)split + 1;
     node[2 * ((size_t)n + i)] = lc + 1;
     node[2 * ((size_t)n + i) + 1] = rc + 1;
-    parent[lc] = n + i;
-    parent[rc] = n + i;
+    rank[i] = node_class((uint32_t)l, (uint32_t)r) << kClassBits;
+}
+
+// The lists of the nodes across class 0 borders, one workgroup per class 1
+// block (32,768 nodes): its class 1 nodes take their places by an LDS counter,
+// the nodes of larger classes (at most the chains of the block's two borders)
+// by one atomic per workgroup and class on their block's count. The order in
+// a list is irrelevant: a node's box depends only on its children's. An
+// atomic per listed node in k_karras made that kernel 140 us longer at 3M
+// leaves (device-scope atomics on a hundred words).
+constexpr uint32_t kListThreads = 1024, kMaxClass = 6, kEdgeCap = 2 * 94;
+
+__global__ __launch_bounds__(1024) void k_top_lists(uint32_t n, uint32_t *__restrict__ rank,
+                                                    uint32_t *__restrict__ count,
+                                                    uint32_t *__restrict__ list) {
+    __shared__ uint32_t cnt[kMaxClass], base[kMaxClass], edge[kEdgeCap], nedge;
+    if (threadIdx.x < kMaxClass) {
+        cnt[threadIdx.x] = 0;
+    }
+    if (threadIdx.x == 0) {
+        nedge = 0;
+    }
+    __syncthreads();
+    const uint32_t lo = blockIdx.x << class_shift(1);
+    const uint32_t hi = min(n - 1, lo + (1u << class_shift(1)));
+    const uint32_t seg1 = class_base(n, 1) + blockIdx.x;
+    for (uint32_t i = lo + threadIdx.x; i < hi; i += kListThreads) {
+        const uint32_t c = rank[i] >> kClassBits;
+        if (c == 1) {
+            const uint32_t place = atomicAdd(cnt + 1, 1u);
+            rank[i] = (1u << kClassBits) | place;
+            if (place < kTopCap) {
+                list[(size_t)seg1 * kTopCap + place] = i;
+            }
+        } else if (c > 1) {
+            rank[i] = (c << kClassBits) | atomicAdd(cnt + c, 1u);
+            const uint32_t e = atomicAdd(&nedge, 1u);
+            if (e < kEdgeCap) {
+                edge[e] = i;
+            }
+        }
+    }
+    __syncthreads();
+    auto seg_of = [&](uint32_t c) {
+        return class_base(n, c) + (class_shift(c) < 32 ? lo >> class_shift(c) : 0u);
+    };
+    if (threadIdx.x == 1) {
+        count[seg1] = cnt[1];
+    } else if (threadIdx.x > 1 && threadIdx.x < kMaxClass && cnt[threadIdx.x]) {
+        base[threadIdx.x] = atomicAdd(count + seg_of(threadIdx.x), cnt[threadIdx.x]);
+    }
+    __syncthreads();
+    for (uint32_t e = threadIdx.x; e < min(nedge, kEdgeCap); e += kListThreads) {
+        const uint32_t i = edge[e], c = rank[i] >> kClassBits;
+        const uint32_t place = base[c] + (rank[i] & ((1u << kClassBits) - 1u));
+        rank[i] = (c << kClassBits) | place;
+        if (place < kTopCap) {
+            list[(size_t)seg_of(c) * kTopCap + place] = i;
+        }
+    }
 }
 
 // Swept leaf box (lbvh.cu:623-731).
-__global__ __launch_bounds__(kNT) void k_leaf_boxes(PrimSet p, const float *__restrict__ x0,
-                                                    const float *__restrict__ x1, float t,
-                                                    const uint32_t *__restrict__ node,
-                                                    Aabb *__restrict__ box,
-                                                    uint32_t *__restrict__ ext) {
-    const uint32_t i = blockIdx.x * kNT + threadIdx.x;
-    if (i >= p.n) {
-        return;
-    }
-    const uint32_t prim = node[2 * (size_t)i] - 1;
-    ext[i] = prim;
+__device__ inline Aabb leaf_box(const PrimSet &p, const float *__restrict__ x0,
+                                const float *__restrict__ x1, float t, uint32_t prim) {
     const float margin = 0.5f * p.ghat[prim] + p.offset[prim];
     float lo0[3], hi0[3], lo1[3], hi1[3];
     for (int k = 0; k < p.arity; ++k) {
@@ -343,163 +428,301 @@ __global__ __launch_bounds__(kNT) void k_leaf_boxes(PrimSet p, const float *__re
     }
     bx.active = 1.0f;
     bx.pad = __uint_as_float(prim_scene(p, prim));
-    box[i] = bx;
+    return bx;
 }
 
-// Depth of every internal node (steps to the root along the parent links),
-// the deepest level and a per-depth count.
-__global__ __launch_bounds__(kNT) void k_depth(uint32_t n, uint32_t root,
-                                               const uint32_t *__restrict__ parent,
-                                               uint32_t *__restrict__ depth,
-                                               uint32_t *__restrict__ maxd) {
-    const uint32_t k = blockIdx.x * kNT + threadIdx.x;
-    if (k >= n - 1) {
+// Tag of a node from its children's: the scene tag in a tree of many scenes,
+// else the primitive bound.
+__device__ inline uint32_t join_tag(uint32_t a, uint32_t b, bool scenes, int bound) {
+    return scenes ? (a == b ? a : kMixedScene) : bound > 0 ? max(a, b) : min(a, b);
+}
+
+__device__ inline void put_child(WalkRec &w, int k, uint32_t code, uint32_t tag,
+                                 const float mn[3], const float mx[3]) {
+    w.code[k] = code;
+    w.tag[k] = tag;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        w.box[6 * k + d] = mn[d];
+        w.box[6 * k + 3 + d] = mx[d];
+    }
+}
+__device__ inline void put_none(WalkRec &w, int k) {
+    const float inf = __builtin_inff();
+    const float mn[3] = {inf, inf, inf}, mx[3] = {-inf, -inf, -inf};
+    put_child(w, k, kNoCode, kInactiveTag, mn, mx);
+}
+
+// One block of 1,024 leaves: their boxes, then the boxes and walk records of
+// the class 0 nodes above them, one leaf and one node per thread. Rounds of
+// nodes whose children were done in an earlier round, one barrier each (as
+// many rounds as the treelet is deep, 11 to 20 in meshes). The boxes stay in
+// LDS until the block is done. A refit of 3M independent triangle edges took
+// 139 (leaf boxes) + 222 (27 launches of inner levels) + 245 us (records)
+// through memory, after 817 us of level tables per build; it takes 276 us here
+// and 3 x 34 us in k_refit_top now, with no tables.
+constexpr uint32_t kRoundsPerVote = 4; // a vote on the end costs several plain barriers
+
+struct TreeletScratch {
+    float lmn[3][kTreelet], lmx[3][kTreelet], nmn[3][kTreelet], nmx[3][kTreelet];
+    uint32_t ltag[kTreelet], ntag[kTreelet], prim[kTreelet], done[kTreelet];
+    uint16_t c0[kTreelet], c1[kTreelet]; // child of a node: leaf place, or kTreelet + node place
+};
+
+__global__ __launch_bounds__(1024) void k_refit_treelet(PrimSet p, const float *__restrict__ x0,
+                                                        const float *__restrict__ x1, float t,
+                                                        const uint32_t *__restrict__ node,
+                                                        const uint32_t *__restrict__ rank,
+                                                        bool scenes, Aabb *__restrict__ box,
+                                                        uint32_t *__restrict__ ext,
+                                                        WalkRec *__restrict__ rec) {
+    __shared__ TreeletScratch s;
+    const uint32_t n = p.n, tid = threadIdx.x;
+    const uint32_t base = blockIdx.x * kTreelet, i = base + tid;
+    if (i < n) {
+        const uint32_t prim = node[2 * (size_t)i] - 1;
+        const Aabb b = leaf_box(p, x0, x1, t, prim);
+        box[i] = b;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            s.lmn[d][tid] = b.mn[d];
+            s.lmx[d][tid] = b.mx[d];
+        }
+        s.prim[tid] = prim;
+        s.ltag[tid] = scenes ? __float_as_uint(b.pad) : prim;
+    }
+    const bool mine = i + 1 < n && (rank[i] >> kClassBits) == 0;
+    uint32_t c[2] = {0u, 0u};
+    if (mine) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const uint32_t v = node[2 * ((size_t)n + i) + k] - 1;
+            c[k] = v < n ? v - base : v - n - base + kTreelet;
+        }
+        s.c0[tid] = (uint16_t)c[0];
+        s.c1[tid] = (uint16_t)c[1];
+    }
+    s.done[tid] = 0;
+    auto mn = [&](uint32_t q, int d) {
+        return q < kTreelet ? s.lmn[d][q] : s.nmn[d][q - kTreelet];
+    };
+    auto mx = [&](uint32_t q, int d) {
+        return q < kTreelet ? s.lmx[d][q] : s.nmx[d][q - kTreelet];
+    };
+    auto tag = [&](uint32_t q) { return q < kTreelet ? s.ltag[q] : s.ntag[q - kTreelet]; };
+    bool todo = mine;
+    __syncthreads();
+    for (uint32_t round = 1; round <= kTreelet; ++round) {
+        // done before this round: a mark of this very round may be seen or not
+        auto ready = [&](uint32_t q) {
+            return q < kTreelet || s.done[q - kTreelet] - 1u < round - 1u;
+        };
+        if (todo && ready(c[0]) && ready(c[1])) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                s.nmn[d][tid] = fminf(mn(c[0], d), mn(c[1], d));
+                s.nmx[d][tid] = fmaxf(mx(c[0], d), mx(c[1], d));
+            }
+            s.ntag[tid] = join_tag(tag(c[0]), tag(c[1]), scenes, p.bound);
+            s.done[tid] = round;
+            todo = false;
+        }
+        if (round % kRoundsPerVote != 0) {
+            __syncthreads();
+        } else if (!__syncthreads_or(todo)) {
+            break;
+        }
+    }
+    if (!mine) {
         return;
-    }
-    uint32_t cur = n + k, d = 0;
-    while (cur != root && d < n) {
-        cur = parent[cur];
-        ++d;
-    }
-    depth[k] = d;
-    atomicMax(maxd, d);
-}
-
-// Per-depth counts. Most nodes of a workgroup share a few depths, so they
-// are counted in LDS first (depths below kLdsDepth) and each workgroup adds
-// one total per depth: a global atomic per node would serialize on the few
-// hot counters.
-constexpr uint32_t kLdsDepth = 256;
-
-__global__ __launch_bounds__(kNT) void k_depth_count(uint32_t m, const uint32_t *__restrict__ depth,
-                                                     uint32_t *__restrict__ count) {
-    __shared__ uint32_t h[kLdsDepth];
-    for (uint32_t d = threadIdx.x; d < kLdsDepth; d += kNT) {
-        h[d] = 0;
-    }
-    __syncthreads();
-    const uint32_t k = blockIdx.x * kNT + threadIdx.x;
-    if (k < m) {
-        const uint32_t d = depth[k];
-        if (d < kLdsDepth) {
-            atomicAdd(h + d, 1u);
-        } else {
-            atomicAdd(count + d, 1u);
-        }
-    }
-    __syncthreads();
-    for (uint32_t d = threadIdx.x; d < kLdsDepth; d += kNT) {
-        if (h[d]) {
-            atomicAdd(count + d, h[d]);
-        }
-    }
-}
-
-// Internal nodes grouped by depth (order within a depth is irrelevant: a
-// node's box depends only on its children's). Each workgroup reserves one
-// range per depth and ranks its nodes inside it in LDS.
-__global__ __launch_bounds__(kNT) void k_depth_scatter(uint32_t m, uint32_t n,
-                                                       const uint32_t *__restrict__ depth,
-                                                       uint32_t *__restrict__ fill,
-                                                       uint32_t *__restrict__ level) {
-    __shared__ uint32_t h[kLdsDepth], base[kLdsDepth];
-    for (uint32_t d = threadIdx.x; d < kLdsDepth; d += kNT) {
-        h[d] = 0;
-    }
-    __syncthreads();
-    const uint32_t k = blockIdx.x * kNT + threadIdx.x;
-    uint32_t d = 0, rank = 0;
-    if (k < m) {
-        d = depth[k];
-        if (d < kLdsDepth) {
-            rank = atomicAdd(h + d, 1u);
-        } else {
-            level[atomicAdd(fill + d, 1u)] = n + k;
-        }
-    }
-    __syncthreads();
-    for (uint32_t e = threadIdx.x; e < kLdsDepth; e += kNT) {
-        base[e] = h[e] ? atomicAdd(fill + e, h[e]) : 0u;
-    }
-    __syncthreads();
-    if (k < m && d < kLdsDepth) {
-        level[base[d] + rank] = n + k;
-    }
-}
-
-// Boxes of the internal nodes of one depth from their children's (the
-// deeper levels are done by the launches before this one).
-__global__ __launch_bounds__(kNT) void k_refit_level(const uint32_t *__restrict__ level,
-                                                     uint32_t count,
-                                                     const uint32_t *__restrict__ node,
-                                                     Aabb *__restrict__ box,
-                                                     uint32_t *__restrict__ ext, int bound) {
-    const uint32_t k = blockIdx.x * kNT + threadIdx.x;
-    if (k >= count) {
-        return;
-    }
-    const uint32_t par = level[k];
-    const uint32_t c0 = node[2 * (size_t)par] - 1, c1 = node[2 * (size_t)par + 1] - 1;
-    const Aabb a = box[c0];
-    const Aabb b = box[c1];
-    if (bound) {
-        ext[par] = bound > 0 ? max(ext[c0], ext[c1]) : min(ext[c0], ext[c1]);
     }
     Aabb u;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        u.mn[d] = fminf(a.mn[d], b.mn[d]);
-        u.mx[d] = fmaxf(a.mx[d], b.mx[d]);
+        u.mn[d] = s.nmn[d][tid];
+        u.mx[d] = s.nmx[d][tid];
     }
-    u.active = (a.active != 0.0f && b.active != 0.0f) ? 1.0f : 0.0f;
-    const uint32_t ta = __float_as_uint(a.pad), tb = __float_as_uint(b.pad);
-    u.pad = __uint_as_float(ta == tb ? ta : kMixedScene);
-    box[par] = u;
-}
-
-// The walk records of the internal nodes from the refit boxes.
-__global__ __launch_bounds__(kNT) void k_walk_records(uint32_t n,
-                                                      const uint32_t *__restrict__ node,
-                                                      const Aabb *__restrict__ box,
-                                                      const uint32_t *__restrict__ ext,
-                                                      bool scenes, WalkRec *__restrict__ rec) {
-    const uint32_t i = blockIdx.x * kNT + threadIdx.x;
-    if (i + 1 >= n) {
-        return;
-    }
-    const uint32_t v = n + i;
-    uint32_t ch[4];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const uint32_t c = node[2 * (size_t)v + k] - 1;
-        const bool leaf = c < n;
-        ch[2 * k] = leaf ? c : node[2 * (size_t)c] - 1;
-        ch[2 * k + 1] = leaf ? kNoCode : node[2 * (size_t)c + 1] - 1;
-    }
+    u.active = 1.0f;
+    u.pad = __uint_as_float(scenes ? s.ntag[tid] : 0u);
+    box[(size_t)n + i] = u;
+    ext[i] = s.ntag[tid];
     WalkRec w;
 #pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) {
-        if (ch[k] == kNoCode) {
-            w.code[k] = kNoCode;
-            w.tag[k] = kInactiveTag;
+    for (int k = 0; k < 2; ++k) {
+        const bool leaf = c[k] < kTreelet;
+        const uint32_t g[2] = {leaf ? c[k] : s.c0[c[k] - kTreelet],
+                               leaf ? 0u : s.c1[c[k] - kTreelet]};
 #pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                w.box[6 * k + d] = __builtin_inff();
-                w.box[6 * k + 3 + d] = -__builtin_inff();
+        for (int h = 0; h < 2; ++h) {
+            if (leaf && h) {
+                put_none(w, 2 * k + h);
+                continue;
             }
-            continue;
-        }
-        const uint32_t c = ch[k];
-        w.code[k] = c < n ? (node[2 * (size_t)c] - 1) | kLeafCode : c;
-        const Aabb b = box[c];
-        w.tag[k] = !scenes ? ext[c] : b.active != 0.0f ? __float_as_uint(b.pad) : kInactiveTag;
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            w.box[6 * k + d] = b.mn[d];
-            w.box[6 * k + 3 + d] = b.mx[d];
+            const uint32_t q = g[h];
+            const float a[3] = {mn(q, 0), mn(q, 1), mn(q, 2)};
+            const float b[3] = {mx(q, 0), mx(q, 1), mx(q, 2)};
+            put_child(w, 2 * k + h,
+                      q < kTreelet ? s.prim[q] | kLeafCode : n + base + q - kTreelet, tag(q), a, b);
         }
     }
     rec[i] = w;
+}
+
+// The listed nodes of one class c block (c >= 1), after the smaller classes:
+// the same rounds over the list, boxes of children of the same class in LDS,
+// the others from memory; then the walk records. One workgroup works through
+// few hundred nodes, so its time is its chains of dependent loads: everything
+// that does not need a box (the grandchildren and their codes) is loaded
+// before the rounds, and nothing is stored inside them (a barrier waits for
+// stores). 39 us a launch without either, 34 us now (3M leaves; 20 us at 8,000).
+struct TopScratch {
+    float mn[3][kTopCap], mx[3][kTopCap];
+    uint32_t tag[kTopCap], done[kTopCap];
+};
+constexpr uint32_t kTopThreads = 1024, kTopPer = kTopCap / kTopThreads;
+
+__global__ __launch_bounds__(1024) void k_refit_top(uint32_t n, uint32_t cls, uint32_t seg0,
+                                                    const uint32_t *__restrict__ count,
+                                                    const uint32_t *__restrict__ list,
+                                                    const uint32_t *__restrict__ node,
+                                                    const uint32_t *__restrict__ rank,
+                                                    bool scenes, int bound, Aabb *box,
+                                                    uint32_t *ext, WalkRec *__restrict__ rec) {
+    __shared__ TopScratch s;
+    const uint32_t seg = seg0 + blockIdx.x;
+    const uint32_t cnt = min(count[seg], kTopCap);
+    const uint32_t *my = list + (size_t)seg * kTopCap;
+    const uint2 *pair = reinterpret_cast<const uint2 *>(node);
+    uint32_t self[kTopPer], gc[kTopPer][4], code[kTopPer][4];
+    uint32_t pend[kTopPer][2]; // places of children of this class, or kTopCap
+    uint32_t todo = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kTopPer; ++k) {
+        const uint32_t e = k * kTopThreads + threadIdx.x;
+        pend[k][0] = pend[k][1] = kTopCap;
+        if (e >= cnt) {
+            continue;
+        }
+        todo |= 1u << k;
+        s.done[e] = 0;
+        self[k] = my[e];
+        const uint2 ch = pair[(size_t)n + self[k]];
+        const uint32_t c[2] = {ch.x - 1, ch.y - 1};
+        const uint2 g[2] = {pair[c[0]], pair[c[1]]};
+        float mn[3], mx[3];
+        uint32_t tag = 0;
+        bool any = false;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const bool leaf = c[h] < n;
+            const uint32_t r = leaf ? 0u : rank[c[h] - n];
+            gc[k][2 * h] = leaf ? c[h] : g[h].x - 1;
+            gc[k][2 * h + 1] = leaf ? kNoCode : g[h].y - 1;
+            if ((r >> kClassBits) == cls) {
+                pend[k][h] = r & ((1u << kClassBits) - 1u);
+                continue;
+            }
+            const Aabb b = box[c[h]];
+            const uint32_t bt = scenes ? __float_as_uint(b.pad)
+                                       : leaf ? g[h].x - 1 : ext[c[h] - n];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                mn[d] = any ? fminf(mn[d], b.mn[d]) : b.mn[d];
+                mx[d] = any ? fmaxf(mx[d], b.mx[d]) : b.mx[d];
+            }
+            tag = any ? join_tag(tag, bt, scenes, bound) : bt;
+            any = true;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t v = gc[k][q];
+            code[k][q] = v == kNoCode ? kNoCode
+                         : v < n      ? (node[2 * (size_t)v] - 1) | kLeafCode
+                                      : v;
+        }
+        if (any) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                s.mn[d][e] = mn[d];
+                s.mx[d][e] = mx[d];
+            }
+            s.tag[e] = tag;
+        }
+    }
+    __syncthreads();
+    for (uint32_t round = 1; round <= kTopCap; ++round) {
+        auto ready = [&](uint32_t q) {
+            return q == kTopCap || s.done[q] - 1u < round - 1u;
+        };
+#pragma unroll
+        for (uint32_t k = 0; k < kTopPer; ++k) {
+            if (!(todo & (1u << k)) || !ready(pend[k][0]) || !ready(pend[k][1])) {
+                continue;
+            }
+            const uint32_t e = k * kTopThreads + threadIdx.x;
+            bool any = pend[k][0] == kTopCap || pend[k][1] == kTopCap;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t q = pend[k][h];
+                if (q == kTopCap) {
+                    continue;
+                }
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    s.mn[d][e] = any ? fminf(s.mn[d][e], s.mn[d][q]) : s.mn[d][q];
+                    s.mx[d][e] = any ? fmaxf(s.mx[d][e], s.mx[d][q]) : s.mx[d][q];
+                }
+                s.tag[e] = any ? join_tag(s.tag[e], s.tag[q], scenes, bound) : s.tag[q];
+                any = true;
+            }
+            s.done[e] = round;
+            todo &= ~(1u << k);
+        }
+        if (round % kRoundsPerVote != 0) {
+            __syncthreads();
+        } else if (!__syncthreads_or(todo != 0)) {
+            break;
+        }
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kTopPer; ++k) {
+        const uint32_t e = k * kTopThreads + threadIdx.x;
+        if (e >= cnt) {
+            continue;
+        }
+        Aabb u;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            u.mn[d] = s.mn[d][e];
+            u.mx[d] = s.mx[d][e];
+        }
+        u.active = 1.0f;
+        u.pad = __uint_as_float(scenes ? s.tag[e] : 0u);
+        box[(size_t)n + self[k]] = u;
+        ext[self[k]] = s.tag[e];
+    }
+    __syncthreads(); // the boxes written above are read below
+#pragma unroll
+    for (uint32_t k = 0; k < kTopPer; ++k) {
+        if (k * kTopThreads + threadIdx.x >= cnt) {
+            continue;
+        }
+        WalkRec w;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t v = gc[k][q];
+            if (v == kNoCode) {
+                put_none(w, q);
+                continue;
+            }
+            const Aabb b = box[v];
+            const uint32_t t = scenes  ? __float_as_uint(b.pad)
+                               : v < n ? code[k][q] & ~kLeafCode
+                                       : ext[v - n];
+            put_child(w, q, code[k][q], t, b.mn, b.mx);
+        }
+        rec[self[k]] = w;
+    }
 }
 
 uint32_t cdiv(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
@@ -509,15 +732,14 @@ uint32_t cdiv(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 Lbvh::~Lbvh() { release(); }
 
 void Lbvh::release() {
-    for (void *p : {(void *)node_, (void *)parent_, (void *)depth_, (void *)level_,
-                    (void *)code_,
+    for (void *p : {(void *)node_, (void *)depth_, (void *)rank_, (void *)list_, (void *)code_,
                     (void *)idx_, (void *)scratch_, (void *)cent_, (void *)part_,
                     (void *)box_, (void *)rec_, (void *)ext_, (void *)sb_}) {
         if (p) {
             (void)dev_free(p);
         }
     }
-    node_ = parent_ = depth_ = level_ = code_ = idx_ = scratch_ = nullptr;
+    node_ = depth_ = rank_ = list_ = code_ = idx_ = scratch_ = nullptr;
     cent_ = part_ = nullptr;
     box_ = nullptr;
     rec_ = nullptr;
@@ -535,9 +757,10 @@ int Lbvh::reserve(uint32_t n) {
     const size_t nodes = 2 * (size_t)n;
     const size_t nb = cdiv(n, kNT);
     PPF_HIP(dev_alloc(&node_, 2 * nodes * sizeof(uint32_t)));
-    PPF_HIP(dev_alloc(&parent_, nodes * sizeof(uint32_t)));
     PPF_HIP(dev_alloc(&depth_, n * sizeof(uint32_t)));
-    PPF_HIP(dev_alloc(&level_, n * sizeof(uint32_t)));
+    PPF_HIP(dev_alloc(&rank_, n * sizeof(uint32_t)));
+    const size_t segs = class_base(n, top_classes(n) + 1);
+    PPF_HIP(dev_alloc(&list_, std::max<size_t>(segs * (kTopCap + 1), 1) * sizeof(uint32_t)));
     PPF_HIP(dev_alloc(&code_, n * sizeof(uint32_t)));
     PPF_HIP(dev_alloc(&idx_, n * sizeof(uint32_t)));
     PPF_HIP(dev_alloc(&scratch_, radix_sort_scratch_words(n) * sizeof(uint32_t)));
@@ -545,7 +768,7 @@ int Lbvh::reserve(uint32_t n) {
     PPF_HIP(dev_alloc(&part_, (6 * nb + 6) * sizeof(float)));
     PPF_HIP(dev_alloc(&box_, nodes * sizeof(Aabb)));
     PPF_HIP(dev_alloc(&rec_, std::max<size_t>(n, 1) * sizeof(WalkRec)));
-    PPF_HIP(dev_alloc(&ext_, nodes * sizeof(uint32_t)));
+    PPF_HIP(dev_alloc(&ext_, std::max<size_t>(n, 1) * sizeof(uint32_t)));
     cap_ = n;
     return PPF_OK;
 }
@@ -593,7 +816,7 @@ int Lbvh::build(const PrimSet &p, const float *x0, const float *x1, float t,
     }
     PPF_HIP(hipGetLastError());
     if (scenes) { // per-primitive codes, kept for the regather after the scene pass
-        PPF_HIP(hipMemcpyAsync(level_, code_, n_ * sizeof(uint32_t), hipMemcpyDeviceToDevice,
+        PPF_HIP(hipMemcpyAsync(rank_, code_, n_ * sizeof(uint32_t), hipMemcpyDeviceToDevice,
                                s));
     }
     PPF_HIP(radix_sort_pairs(code_, idx_, n_, 30, scratch_, s));
@@ -607,59 +830,22 @@ int Lbvh::build(const PrimSet &p, const float *x0, const float *x1, float t,
         k_scene_keys<<<nb, kNT, 0, s>>>(p, idx_, depth_);
         PPF_HIP(hipGetLastError());
         PPF_HIP(radix_sort_pairs(depth_, idx_, n_, bits, scratch_, s));
-        k_regather<<<nb, kNT, 0, s>>>(n_, idx_, level_, code_);
+        k_regather<<<nb, kNT, 0, s>>>(n_, idx_, rank_, code_);
         PPF_HIP(hipGetLastError());
         sk = depth_;
     }
-    k_karras<<<nb, kNT, 0, s>>>(n_, code_, sk, idx_, node_, parent_);
+    // lists of the nodes across treelet borders: counts, then places
+    const uint32_t segs = class_base(n_, top_classes(n_) + 1);
+    if (segs) {
+        PPF_HIP(hipMemsetAsync(list_, 0, segs * sizeof(uint32_t), s));
+    }
+    k_karras<<<nb, kNT, 0, s>>>(n_, code_, sk, idx_, node_, rank_);
     PPF_HIP(hipGetLastError());
-    rc = levels(s);
-    if (rc != PPF_OK) {
-        return rc;
+    if (segs) {
+        k_top_lists<<<class_blocks(n_, 1), kListThreads, 0, s>>>(n_, rank_, list_, list_ + segs);
+        PPF_HIP(hipGetLastError());
     }
     return refit(p, x0, x1, t, s);
-}
-
-// Internal nodes grouped by depth (lbvh.cu:479-616 computes the same levels):
-// the order refit visits them in. The sort keys and indices are free by now
-// and hold the per-depth counts and fill cursors.
-int Lbvh::levels(hipStream_t s) {
-    loff_.assign(1, 0);
-    if (n_ < 2) {
-        return PPF_OK;
-    }
-    const uint32_t m = n_ - 1;
-    uint32_t *maxd = scratch_;
-    PPF_HIP(hipMemsetAsync(maxd, 0, sizeof(uint32_t), s));
-    k_depth<<<cdiv(m, kNT), kNT, 0, s>>>(n_, root_, parent_, depth_, maxd);
-    PPF_HIP(hipGetLastError());
-    uint32_t hmax = 0;
-    PPF_HIP(hipMemcpyAsync(&hmax, maxd, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    PPF_HIP(hipStreamSynchronize(s));
-    if (hmax >= n_) {
-        set_error("Lbvh: parent links do not reach the root");
-        return PPF_ERR_SOLVER;
-    }
-    const uint32_t levels = hmax + 1;
-    uint32_t *count = code_, *fill = idx_;
-    PPF_HIP(hipMemsetAsync(count, 0, levels * sizeof(uint32_t), s));
-    k_depth_count<<<cdiv(m, kNT), kNT, 0, s>>>(m, depth_, count);
-    PPF_HIP(hipGetLastError());
-    std::vector<uint32_t> h(levels);
-    PPF_HIP(hipMemcpyAsync(h.data(), count, levels * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                           s));
-    PPF_HIP(hipStreamSynchronize(s));
-    loff_.assign(levels + 1, 0);
-    for (uint32_t d = 0; d < levels; ++d) {
-        loff_[d + 1] = loff_[d] + h[d];
-    }
-    PPF_HIP(hipMemcpyAsync(fill, loff_.data(), levels * sizeof(uint32_t),
-                           hipMemcpyHostToDevice, s));
-    k_depth_scatter<<<cdiv(m, kNT), kNT, 0, s>>>(m, n_, depth_, fill, level_);
-    PPF_HIP(hipGetLastError());
-    // loff_ must stay intact until the copy above has read it
-    PPF_HIP(hipStreamSynchronize(s));
-    return PPF_OK;
 }
 
 int Lbvh::refit(const PrimSet &p, const float *x0, const float *x1, float t,
@@ -672,21 +858,14 @@ int Lbvh::refit(const PrimSet &p, const float *x0, const float *x1, float t,
     if (n_ == 0) {
         return PPF_OK;
     }
-    k_leaf_boxes<<<cdiv(n_, kNT), kNT, 0, s>>>(p, x0, x1, t, node_, box_, ext_);
+    k_refit_treelet<<<cdiv(n_, kTreelet), kTreelet, 0, s>>>(p, x0, x1, t, node_, rank_, scenes_,
+                                                            box_, ext_, rec_);
     PPF_HIP(hipGetLastError());
-    // Inner boxes level by level from the deepest: a kernel boundary orders
-    // each level after its children, with no fences or arrival counters.
-    for (size_t d = loff_.size() - 1; d-- > 0;) {
-        const uint32_t cnt = loff_[d + 1] - loff_[d];
-        if (cnt) {
-            k_refit_level<<<cdiv(cnt, kNT), kNT, 0, s>>>(level_ + loff_[d], cnt, node_, box_,
-                                                         ext_, bound_);
-            PPF_HIP(hipGetLastError());
-        }
-    }
-    if (n_ > 1) {
-        k_walk_records<<<cdiv(n_ - 1, kNT), kNT, 0, s>>>(n_, node_, box_, ext_, scenes_,
-                                                             rec_);
+    const uint32_t top = top_classes(n_), segs = class_base(n_, top + 1);
+    for (uint32_t c = 1; c <= top; ++c) {
+        k_refit_top<<<class_blocks(n_, c), kTopThreads, 0, s>>>(
+            n_, c, class_base(n_, c), list_, list_ + segs, node_, rank_, scenes_, bound_, box_,
+            ext_, rec_);
         PPF_HIP(hipGetLastError());
     }
     return PPF_OK;

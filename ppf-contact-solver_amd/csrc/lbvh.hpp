@@ -4,11 +4,8 @@
 // bounds of the centroids, 10-bit-per-axis Morton codes, a stable sort of
 // (code, index), and the Karras radix tree with the index tie-break on equal
 // codes. Node i < n is leaf i (prim + 1, 0); node n + i is internal node i
-// (left + 1, right + 1); the root is node n (leaf 0 when n == 1). Boxes are
-// refit bottom-up one depth level per launch (levels computed once per build).
+// (left + 1, right + 1); the root is node n (leaf 0 when n == 1).
 #pragma once
-#include <vector>
-
 #include "common.hpp"
 
 namespace ppf {
@@ -90,19 +87,19 @@ class Lbvh {
 
   private:
     uint32_t cap_ = 0, n_ = 0, root_ = 0;
-    uint32_t *node_ = nullptr, *parent_ = nullptr, *depth_ = nullptr, *level_ = nullptr;
-    std::vector<uint32_t> loff_{0}; // level offsets into level_ (host copy)
+    uint32_t *node_ = nullptr, *depth_ = nullptr;
+    uint32_t *rank_ = nullptr; // treelet class and place of every internal node
+    uint32_t *list_ = nullptr; // nodes across treelet borders, per block: counts, places
     uint32_t *code_ = nullptr, *idx_ = nullptr, *scratch_ = nullptr;
     float *cent_ = nullptr, *part_ = nullptr;
     Aabb *box_ = nullptr;
     WalkRec *rec_ = nullptr;
-    uint32_t *ext_ = nullptr; // primitive bound per node
+    uint32_t *ext_ = nullptr; // tag of every internal node (scene or primitive bound)
     int bound_ = 0;
     bool scenes_ = false;
     uint32_t *sb_ = nullptr; // per-scene centroid bounds (many scenes)
     size_t sb_cap_ = 0;
     void release();
-    int levels(hipStream_t s);
 };
 
 } // namespace ppf

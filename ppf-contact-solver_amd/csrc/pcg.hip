@@ -68,6 +68,12 @@ constexpr uint32_t kOrderRows = 98304;
 // symmetric form too (set_pattern_arrays).
 constexpr double kSymAvg = 14.0;
 constexpr uint64_t kSymBytes = 16ull << 20;
+// Bytes of blocks up to which an iteration forms p inside the SpMV, of the
+// split and symmetric forms and of the ELL form (short rows gather less). us
+// per iteration with a kernel for p / inside: grids of 33^2 14.1 / 12.6, 129^2
+// 15.4 / 13.7, 512^2 (38 MB) 42.1 / 41.3, 724^2 63.2 / 62.7, 1024^2 121 / 126;
+// 8 x 64^2 sheets (11 MB) 17.7 / 16.7, 8 x 91^2 (22 MB) 27.0 / 29.1.
+constexpr uint64_t kFuseBytes = 16ull << 20, kFuseEllBytes = 48ull << 20;
 
 // Device-resident scalars of one solve. Written by exactly one thread of one
 // kernel and read only by later kernels (stream order), except `done`, whose
@@ -112,6 +118,10 @@ struct Args {
     const uint32_t *mq, *tq;
     const float *val, *cdiag, *b;
     float *x, *P, *r, *z, *p, *Ap;
+    // fused iterations (k_spmv_* with FUSE): iteration k of a graph reads the
+    // direction before it from p and writes its own to p2 for even k, the other
+    // way round for odd k
+    float *p2;
     float *part; // [G1 pAp][G1 |terms|][G2 rz][G2 err], one per tile
     float *err_hist; // (one-scene solves)
     Scalars *s;      // [nscene]
@@ -242,14 +252,23 @@ __global__ __launch_bounds__(kNT) void k_diag_invert(const Args *__restrict__ A)
 }
 
 // Longest row of the split operator: stored blocks plus mirrored blocks.
-__global__ void k_row_len_max(uint32_t n, const uint32_t *__restrict__ rp,
+constexpr uint32_t kLenGrid = 256;
+__global__ __launch_bounds__(kNT) void k_row_len_max(uint32_t n, const uint32_t *__restrict__ rp,
                               const uint32_t *__restrict__ tp,
                               uint32_t *__restrict__ out) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) {
-        return;
+    uint32_t len = 0;
+    for (uint32_t i = blockIdx.x * kNT + threadIdx.x; i < n; i += gridDim.x * kNT) {
+        len = max(len, (rp[i + 1] - rp[i]) + (tp[i + 1] - tp[i]));
     }
-    atomicMax(out, (rp[i + 1] - rp[i]) + (tp[i + 1] - tp[i]));
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        len = max(len, (uint32_t)__shfl_xor(len, off, kWave));
+    }
+    // one atomic per wave of at most kLenGrid workgroups: one per row
+    // serialized on the word (1M rows: 190 us, 19 us now)
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        atomicMax(out, len);
+    }
 }
 
 // Per-row entry table of width W: the row's stored blocks (column, slot),
@@ -417,6 +436,125 @@ __global__ void k_order_rows(uint32_t n, uint32_t w, const uint32_t *__restrict_
     }
 }
 
+__device__ inline float reduce_parts(gptr<const float> part, uint32_t cnt,
+                                     float *lds) {
+    float acc = 0.0f;
+    for (uint32_t k = threadIdx.x; k < cnt; k += kNT) {
+        acc = acc + part[k];
+    }
+    return block_sum<kNT>(acc, lds);
+}
+
+// The end of an iteration: the reference's residual-check schedule
+// (solver.cu:1249-1380) on the sums of r.z and |r|_1, by one thread. rz0: r.z
+// of the iteration before; slot: where the new one goes.
+__device__ inline void end_iteration(const Args *__restrict__ A, gptr<Scalars> s, uint32_t slot,
+                                     float rz0, float rz1, float err) {
+    if (!(rz0 > 0.0f) && s->cause == 0) {
+        s->breakdown = 1;
+        s->cause = 2;
+        s->break_iter = (int32_t)s->iter;
+    }
+    s->rz[slot] = rz1;
+    const uint32_t it = s->iter + 1;
+    s->iter = it;
+    if (A->err_hist) {
+        as_global(A->err_hist)[it - 1] = err;
+    }
+    const bool at_cap = it >= s->max_iter;
+    if (it == s->next_check || at_cap) {
+        const float reresid = err / s->err0;
+        s->rep_iter = it;
+        s->rep_resid = reresid;
+        int32_t st = -1;
+        if (reresid < s->tol) {
+            st = 0;
+        } else if (s->breakdown) {
+            st = s->cause == 3 ? 1 : (s->cause == 2 ? 5 : 4);
+        } else if (!isfinite(reresid)) {
+            st = 3;
+        } else if (at_cap) {
+            st = 2;
+        }
+        if (st >= 0) {
+            s->status = st;
+            s->done = 1;
+        } else {
+            if (reresid < 8.0f * s->tol) {
+                s->stride = 1;
+            }
+            s->next_check = it + s->stride;
+        }
+    }
+}
+
+// The direction a fused SpMV applies the operator to: p_k = z + beta p_{k-1}
+// (the fmaf of k_pupdate), formed wherever it is gathered and stored by its
+// row's lanes. beta comes from the partials of the update before (from the
+// scalars in a graph's first iteration, whose bookkeeping k_end_graph did); the
+// scene's first tile does the bookkeeping of the iteration before. One kernel
+// and one pass over p less per iteration, against a second gather per entry:
+// it pays while a launch costs more than the gathers (kFuseBytes).
+struct Direction {
+    gptr<const float> v, z; // z unset: the operand is v itself
+    gptr<float> out;
+    float beta;
+    bool fused;
+    __device__ inline f3 at(uint32_t j) const {
+        const f3 a = load3(v + 3 * (size_t)j);
+        if (!fused) {
+            return a;
+        }
+        const f3 c = load3(z + 3 * (size_t)j);
+        return mk3(fmaf(beta, a.x, 1.0f * c.x), fmaf(beta, a.y, 1.0f * c.y),
+                   fmaf(beta, a.z, 1.0f * c.z));
+    }
+};
+
+// False: the solve of the tile's scene is over. Every thread of the workgroup
+// calls it.
+template <bool FUSE>
+__device__ inline bool start_direction(const Args *__restrict__ A, const Tile &T, uint32_t k,
+                                       const float *vin, float *lds, Direction &d) {
+    d.v = as_global(vin);
+    d.z = as_global((const float *)nullptr);
+    d.out = as_global((float *)nullptr);
+    d.beta = 0.0f;
+    d.fused = FUSE;
+    if (!FUSE) {
+        return true;
+    }
+    gptr<Scalars> s = as_global(A->s + T.scene);
+    d.v = as_global((const float *)((k & 1) ? A->p2 : A->p));
+    d.z = as_global((const float *)A->z);
+    d.out = as_global((k & 1) ? A->p : A->p2);
+    float rz1, rz0;
+    bool first = false;
+    if (k == 0) {
+        rz1 = s->rz[0], rz0 = s->rz[1];
+        first = s->iter == 0; // p_0 = z
+    } else {
+        gptr<const float> part = as_global(A->part);
+        const uint32_t t0 = A->sc2[T.scene], nt = A->sc2[T.scene + 1] - t0;
+        rz1 = reduce_parts(part + 2 * A->G1 + t0, nt, lds);
+        rz0 = s->rz[(k - 1) & 1];
+        if (T.first) {
+            const float err = reduce_parts(part + 2 * A->G1 + A->G2 + t0, nt, lds);
+            __shared__ int32_t over;
+            if (threadIdx.x == 0) {
+                end_iteration(A, s, k & 1, rz0, rz1, err);
+                over = s->done;
+            }
+            __syncthreads();
+            if (over) {
+                return false;
+            }
+        }
+    }
+    d.beta = !first && rz0 > 0.0f ? rz1 / rz0 : 0.0f;
+    return true;
+}
+
 // Split form of k_spmv_ell: the same entry list per row (the row's stored
 // slots, then its mirrored slots) and the same lane assignment (lane q sums
 // entries q, q+4, q+8, ... in that order), so the sums are bit-identical to
@@ -424,15 +562,19 @@ __global__ void k_order_rows(uint32_t n, uint32_t w, const uint32_t *__restrict_
 // table themselves instead of a padded copy (4 B per stored entry, 8 B per
 // mirrored one) and rows of any length are taken in passes of 4*M entries,
 // all loads of a pass issued before any is used.
-template <bool DOT, int M>
+template <bool DOT, int M, bool FUSE>
 __global__ __launch_bounds__(kNT) void k_spmv_split(const Args *__restrict__ A,
                                                     const float *__restrict__ vin,
-                                                    float *__restrict__ yout) {
+                                                    float *__restrict__ yout, uint32_t iter) {
     constexpr uint32_t kRows = kNT / 4;
     __shared__ float lds[kNT / kWave];
     const uint32_t L = xcd_logical_block();
     const Tile T = load_tile(A->tile1, L);
     if (DOT && as_global(A->s + T.scene)->done) {
+        return;
+    }
+    Direction v;
+    if (!start_direction<FUSE>(A, T, iter, vin, lds, v)) {
         return;
     }
     const uint32_t q = threadIdx.x & 3u, sub = threadIdx.x >> 2;
@@ -443,7 +585,6 @@ __global__ __launch_bounds__(kNT) void k_spmv_split(const Args *__restrict__ A,
     gptr<const uint32_t> tslot = as_global(A->tslot);
     gptr<const float> val = as_global(A->val);
     gptr<const float> cd = as_global(A->cdiag);
-    gptr<const float> v = as_global(vin);
     gptr<float> y = as_global(yout);
     const uint32_t lo = T.lo, hi = T.hi;
     float dot = 0.0f, adot = 0.0f;
@@ -463,7 +604,7 @@ __global__ __launch_bounds__(kNT) void k_spmv_split(const Args *__restrict__ A,
             const uint32_t iin = in < hi ? in : lo;
             nb[0] = rp[iin], nb[1] = rp[iin + 1], nb[2] = tp[iin], nb[3] = tp[iin + 1];
         }
-        const f3 vi = load3(v + 3 * (size_t)ii);
+        const f3 vi = v.at(ii);
         f3 sum = mk3(0, 0, 0), as = mk3(0, 0, 0);
         // the first pass is unconditional (straight-line loads for the common
         // row); rows longer than 4 M entries take further passes
@@ -493,7 +634,7 @@ __global__ __launch_bounds__(kNT) void k_spmv_split(const Args *__restrict__ A,
                 for (int c = 0; c < 9; ++c) {
                     blk[m][c] = a[c];
                 }
-                vj[m] = load3(v + 3 * (size_t)cj[m]);
+                vj[m] = v.at(cj[m]);
             }
 #pragma unroll
             for (int m = 0; m < M; ++m) {
@@ -530,6 +671,9 @@ __global__ __launch_bounds__(kNT) void k_spmv_split(const Args *__restrict__ A,
         }
         if (valid && q == 0) {
             store3(y + 3 * (size_t)i, sum);
+            if (FUSE) {
+                store3(v.out + 3 * (size_t)i, vi);
+            }
             if (DOT) {
                 dot = dot + vi.x * sum.x;
                 dot = dot + vi.y * sum.y;
@@ -683,6 +827,7 @@ __global__ __launch_bounds__(1024) void k_tile_order(uint32_t used, uint32_t tot
         uint32_t at = t;
         if (t < used) {
             at = 0;
+#pragma unroll 16
             for (uint32_t k = 0; k < used; ++k) {
                 at += root[k] < root[t] || (root[k] == root[t] && k < t);
             }
@@ -701,16 +846,20 @@ __global__ __launch_bounds__(1024) void k_tile_order(uint32_t used, uint32_t tot
 // form's float expression and every lane sums its entries in the split form's
 // order (lane q takes entries q, q+4, ... of the row's stored-then-mirrored
 // list), so y is bit-identical to k_spmv_split.
-template <bool DOT, int M>
+template <bool DOT, int M, bool FUSE>
 __global__ __launch_bounds__(kNT) void k_spmv_sym(const Args *__restrict__ A,
                                                   const float *__restrict__ vin,
-                                                  float *__restrict__ yout) {
+                                                  float *__restrict__ yout, uint32_t iter) {
     extern __shared__ float mir[]; // 3 floats per in-tile mirror (kSymCap)
     constexpr uint32_t kRows = kNT / 4;
     __shared__ float lds[kNT / kWave];
     const uint32_t L = xcd_logical_block();
     const Tile T = load_tile(A->tile1, L);
     if (DOT && as_global(A->s + T.scene)->done) {
+        return;
+    }
+    Direction v;
+    if (!start_direction<FUSE>(A, T, iter, vin, lds, v)) {
         return;
     }
     const uint32_t q = threadIdx.x & 3u, sub = threadIdx.x >> 2;
@@ -721,7 +870,6 @@ __global__ __launch_bounds__(kNT) void k_spmv_sym(const Args *__restrict__ A,
     gptr<const uint32_t> tq = as_global(A->tq);
     gptr<const float> val = as_global(A->val);
     gptr<const float> cd = as_global(A->cdiag);
-    gptr<const float> v = as_global(vin);
     gptr<float> y = as_global(yout);
     const uint32_t lo = T.lo, hi = T.hi;
     float dot = 0.0f, adot = 0.0f;
@@ -732,7 +880,7 @@ __global__ __launch_bounds__(kNT) void k_spmv_sym(const Args *__restrict__ A,
         const uint32_t r0 = rp[ii], t0 = tp[ii];
         const uint32_t ns = valid ? rp[ii + 1] - r0 : 0u;
         const uint32_t nm = valid ? tp[ii + 1] - t0 : 0u;
-        const f3 vi = load3(v + 3 * (size_t)ii);
+        const f3 vi = v.at(ii);
         f3 sum = mk3(0, 0, 0), as = mk3(0, 0, 0);
         // stored entries: the row's own products, and the transposed ones of
         // in-tile mirrors into LDS
@@ -756,7 +904,7 @@ __global__ __launch_bounds__(kNT) void k_spmv_sym(const Args *__restrict__ A,
                 for (int c = 0; c < 9; ++c) {
                     blk[m][c] = a[c];
                 }
-                vj[m] = load3(v + 3 * (size_t)cj[m]);
+                vj[m] = v.at(cj[m]);
             }
 #pragma unroll
             for (int m = 0; m < M; ++m) {
@@ -798,7 +946,7 @@ __global__ __launch_bounds__(kNT) void k_spmv_sym(const Args *__restrict__ A,
                     for (int c = 0; c < 9; ++c) {
                         blk[m][c] = a[c];
                     }
-                    vj[m] = load3(v + 3 * (size_t)src[m]);
+                    vj[m] = v.at(src[m]);
                 } else {
 #pragma unroll
                     for (int c = 0; c < 9; ++c) {
@@ -837,6 +985,9 @@ __global__ __launch_bounds__(kNT) void k_spmv_sym(const Args *__restrict__ A,
         }
         if (valid && q == 0) {
             store3(y + 3 * (size_t)i, sum);
+            if (FUSE) {
+                store3(v.out + 3 * (size_t)i, vi);
+            }
             if (DOT) {
                 dot = dot + vi.x * sum.x;
                 dot = dot + vi.y * sum.y;
@@ -862,10 +1013,10 @@ __global__ __launch_bounds__(kNT) void k_spmv_sym(const Args *__restrict__ A,
 // takes entries q, q+4, ... of the row's fixed-width table, so no row-offset
 // load sits in the dependent chain and all M block loads of a lane are issued
 // before any is consumed. Padding entries read slot 0 and are discarded.
-template <bool DOT, int M>
+template <bool DOT, int M, bool FUSE>
 __global__ __launch_bounds__(kNT) void k_spmv_ell(const Args *__restrict__ A,
                                                   const float *__restrict__ vin,
-                                                  float *__restrict__ yout) {
+                                                  float *__restrict__ yout, uint32_t iter) {
     constexpr uint32_t W = 4 * M;
     constexpr uint32_t kRows = kNT / 4;
     __shared__ float lds[kNT / kWave];
@@ -874,11 +1025,14 @@ __global__ __launch_bounds__(kNT) void k_spmv_ell(const Args *__restrict__ A,
     if (DOT && as_global(A->s + T.scene)->done) {
         return;
     }
+    Direction v;
+    if (!start_direction<FUSE>(A, T, iter, vin, lds, v)) {
+        return;
+    }
     const uint32_t q = threadIdx.x & 3u, sub = threadIdx.x >> 2;
     gptr<const uint64_t> ent = as_global(reinterpret_cast<const uint64_t *>(A->ent));
     gptr<const float> val = as_global(A->val);
     gptr<const float> cd = as_global(A->cdiag);
-    gptr<const float> v = as_global(vin);
     gptr<float> y = as_global(yout);
     const uint32_t lo = T.lo, hi = T.hi;
     float dot = 0.0f, adot = 0.0f;
@@ -909,7 +1063,7 @@ __global__ __launch_bounds__(kNT) void k_spmv_ell(const Args *__restrict__ A,
                 wnext[m] = ent[(size_t)iin * W + q + 4 * m];
             }
         }
-        const f3 vi = load3(v + 3 * (size_t)ii);
+        const f3 vi = v.at(ii);
         f3 sum = mk3(0, 0, 0), as = mk3(0, 0, 0);
         float blk[M][9];
         f3 vj[M];
@@ -921,7 +1075,7 @@ __global__ __launch_bounds__(kNT) void k_spmv_ell(const Args *__restrict__ A,
             for (int c = 0; c < 9; ++c) {
                 blk[m][c] = a[c];
             }
-            vj[m] = load3(v + 3 * (size_t)e[m].x);
+            vj[m] = v.at(e[m].x);
         }
 #pragma unroll
         for (int m = 0; m < M; ++m) {
@@ -957,6 +1111,9 @@ __global__ __launch_bounds__(kNT) void k_spmv_ell(const Args *__restrict__ A,
         }
         if (valid && q == 0) {
             store3(y + 3 * (size_t)i, sum);
+            if (FUSE) {
+                store3(v.out + 3 * (size_t)i, vi);
+            }
             if (DOT) {
                 dot = dot + vi.x * sum.x;
                 dot = dot + vi.y * sum.y;
@@ -1023,15 +1180,6 @@ __global__ __launch_bounds__(kNT) void k_init_residual(const Args *__restrict__ 
     }
 }
 
-__device__ inline float reduce_parts(gptr<const float> part, uint32_t cnt,
-                                     float *lds) {
-    float acc = 0.0f;
-    for (uint32_t k = threadIdx.x; k < cnt; k += kNT) {
-        acc = acc + part[k];
-    }
-    return block_sum<kNT>(acc, lds);
-}
-
 // Initial scalars and the bookkeeping state (solver.cu:1020-1031, 1170-1175).
 // One workgroup per scene.
 __global__ __launch_bounds__(kNT) void k_init_scalars(const Args *__restrict__ A) {
@@ -1071,7 +1219,7 @@ __global__ __launch_bounds__(kNT) void k_init_scalars(const Args *__restrict__ A
 // alpha from the SpMV partials with the curvature guard, then x += alpha p,
 // r -= alpha Ap, z = P r and the r.z / |r|_1 partials (solver.cu:431-514).
 // k = position of this iteration inside the captured graph.
-template <bool FAC>
+template <bool FAC, bool FUSE>
 __global__ __launch_bounds__(kNT) void k_update(const Args *__restrict__ A,
                                                 uint32_t k) {
     __shared__ float lds[kNT / kWave];
@@ -1099,7 +1247,7 @@ __global__ __launch_bounds__(kNT) void k_update(const Args *__restrict__ A,
     gptr<float> x = as_global(A->x);
     gptr<float> r = as_global(A->r);
     gptr<float> z = as_global(A->z);
-    gptr<const float> p = as_global(A->p);
+    gptr<const float> p = as_global((const float *)(FUSE && !(k & 1) ? A->p2 : A->p));
     gptr<const float> Ap = as_global(A->Ap);
     gptr<const float> P = as_global(A->P);
     float rz = 0.0f, err = 0.0f;
@@ -1310,7 +1458,7 @@ __global__ __launch_bounds__(kNT) void k_fac_gt(const Args *__restrict__ A, int 
 }
 
 // beta = rz1 / rz0 (breakdown if rz0 <= 0), p = z + beta p, and -- on one
-// thread -- the reference's residual-check schedule (solver.cu:1249-1380).
+// thread -- the end of the iteration.
 __global__ __launch_bounds__(kNT) void k_pupdate(const Args *__restrict__ A,
                                                  uint32_t k) {
     __shared__ float lds[kNT / kWave];
@@ -1338,41 +1486,22 @@ __global__ __launch_bounds__(kNT) void k_pupdate(const Args *__restrict__ A,
     if (threadIdx.x != 0) {
         return;
     }
-    if (!rz_ok && s->cause == 0) {
-        s->breakdown = 1;
-        s->cause = 2;
-        s->break_iter = (int32_t)s->iter;
+    end_iteration(A, s, (k + 1) & 1, rz0, rz1, err);
+}
+
+// The bookkeeping of a graph's last fused iteration. One workgroup per scene.
+__global__ __launch_bounds__(kNT) void k_end_graph(const Args *__restrict__ A) {
+    __shared__ float lds[kNT / kWave];
+    gptr<Scalars> s = as_global(A->s + blockIdx.x);
+    if (s->done) {
+        return;
     }
-    s->rz[(k + 1) & 1] = rz1;
-    const uint32_t it = s->iter + 1;
-    s->iter = it;
-    if (A->err_hist) {
-        as_global(A->err_hist)[it - 1] = err;
-    }
-    const bool at_cap = it >= s->max_iter;
-    if (it == s->next_check || at_cap) {
-        const float reresid = err / s->err0;
-        s->rep_iter = it;
-        s->rep_resid = reresid;
-        int32_t st = -1;
-        if (reresid < s->tol) {
-            st = 0;
-        } else if (s->breakdown) {
-            st = s->cause == 3 ? 1 : (s->cause == 2 ? 5 : 4);
-        } else if (!isfinite(reresid)) {
-            st = 3;
-        } else if (at_cap) {
-            st = 2;
-        }
-        if (st >= 0) {
-            s->status = st;
-            s->done = 1;
-        } else {
-            if (reresid < 8.0f * s->tol) {
-                s->stride = 1;
-            }
-            s->next_check = it + s->stride;
-        }
+    gptr<const float> part = as_global(A->part);
+    const uint32_t t0 = A->sc2[blockIdx.x], nt = A->sc2[blockIdx.x + 1] - t0;
+    const float rz1 = reduce_parts(part + 2 * A->G1 + t0, nt, lds);
+    const float err = reduce_parts(part + 2 * A->G1 + A->G2 + t0, nt, lds);
+    if (threadIdx.x == 0) {
+        end_iteration(A, s, 0, s->rz[1], rz1, err);
     }
 }
 
@@ -1417,6 +1546,7 @@ struct PcgPlanImpl {
     uint32_t split_m = 4;      // entries per lane per pass of the split form
     // symmetric form (one-scene plans): in-tile mirrors through LDS
     bool sym = false;
+    bool fuse = false;         // block-Jacobi iterations form p inside the SpMV
     int form = PPF_SPMV_AUTO;  // the caller's choice of form
     uint32_t *symmem = nullptr; // mq (nnz) | tq (nnz), grown with nnz
     size_t sym_cap = 0;
@@ -1485,40 +1615,40 @@ hipError_t plan_free(PcgPlanImpl *pl, void *p) {
 
 // The SpMV kernel a plan launches (its graph is captured for one).
 uint32_t spmv_key(const PcgPlanImpl &pl) {
-    return (pl.h.Gd ? 1000u : 0u) +
+    return (pl.h.Gd ? 1000u : pl.fuse ? 2000u : 0u) +
            (pl.sym ? 200u + pl.split_m : pl.split ? 100u + pl.split_m : pl.h.ell_m);
 }
 
 constexpr size_t kSymLds = kSymCap * 3 * sizeof(float);
 
 // y = M v with the plan's SpMV form (ELL width 4*m, or the CSR walk).
-template <bool DOT>
-hipError_t launch_spmv(const PcgPlanImpl &pl, const float *v, float *y,
-                       hipStream_t st) {
+template <bool DOT, bool FUSE = false>
+hipError_t launch_spmv(const PcgPlanImpl &pl, const float *v, float *y, hipStream_t st,
+                       uint32_t iter = 0) {
     const Args &h = pl.h;
     if (pl.sym) {
         switch (pl.split_m) {
-        case 2: k_spmv_sym<DOT, 2><<<h.G1, kNT, kSymLds, st>>>(pl.d_args, v, y); break;
-        case 3: k_spmv_sym<DOT, 3><<<h.G1, kNT, kSymLds, st>>>(pl.d_args, v, y); break;
-        default: k_spmv_sym<DOT, 4><<<h.G1, kNT, kSymLds, st>>>(pl.d_args, v, y); break;
+        case 2: k_spmv_sym<DOT, 2, FUSE><<<h.G1, kNT, kSymLds, st>>>(pl.d_args, v, y, iter); break;
+        case 3: k_spmv_sym<DOT, 3, FUSE><<<h.G1, kNT, kSymLds, st>>>(pl.d_args, v, y, iter); break;
+        default: k_spmv_sym<DOT, 4, FUSE><<<h.G1, kNT, kSymLds, st>>>(pl.d_args, v, y, iter); break;
         }
         return hipGetLastError();
     }
     if (pl.split) {
         switch (pl.split_m) {
-        case 2: k_spmv_split<DOT, 2><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y); break;
-        case 3: k_spmv_split<DOT, 3><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y); break;
-        default: k_spmv_split<DOT, 4><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y); break;
+        case 2: k_spmv_split<DOT, 2, FUSE><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y, iter); break;
+        case 3: k_spmv_split<DOT, 3, FUSE><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y, iter); break;
+        default: k_spmv_split<DOT, 4, FUSE><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y, iter); break;
         }
         return hipGetLastError();
     }
     switch (h.ell_m) {
-    case 1: k_spmv_ell<DOT, 1><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y); break;
-    case 2: k_spmv_ell<DOT, 2><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y); break;
-    case 3: k_spmv_ell<DOT, 3><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y); break;
-    case 4: k_spmv_ell<DOT, 4><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y); break;
-    case 6: k_spmv_ell<DOT, 6><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y); break;
-    default: k_spmv_ell<DOT, 8><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y); break;
+    case 1: k_spmv_ell<DOT, 1, FUSE><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y, iter); break;
+    case 2: k_spmv_ell<DOT, 2, FUSE><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y, iter); break;
+    case 3: k_spmv_ell<DOT, 3, FUSE><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y, iter); break;
+    case 4: k_spmv_ell<DOT, 4, FUSE><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y, iter); break;
+    case 6: k_spmv_ell<DOT, 6, FUSE><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y, iter); break;
+    default: k_spmv_ell<DOT, 8, FUSE><<<h.G1, kNT, 0, st>>>(pl.d_args, v, y, iter); break;
     }
     return hipGetLastError();
 }
@@ -1531,15 +1661,26 @@ void launch_fac(const PcgPlanImpl &pl, int init, hipStream_t st) {
 
 hipError_t launch_iteration(const PcgPlanImpl &pl, uint32_t k, hipStream_t st) {
     const Args &h = pl.h;
+    if (pl.fuse && !h.Gd) {
+        const hipError_t e = launch_spmv<true, true>(pl, nullptr, h.Ap, st, k);
+        if (e != hipSuccess) {
+            return e;
+        }
+        k_update<false, true><<<h.G2, kNT, 0, st>>>(pl.d_args, k);
+        if (k + 1 == (uint32_t)kGraphIters) {
+            k_end_graph<<<h.nscene, kNT, 0, st>>>(pl.d_args);
+        }
+        return hipGetLastError();
+    }
     hipError_t e = launch_spmv<true>(pl, h.p, h.Ap, st);
     if (e != hipSuccess) {
         return e;
     }
     if (h.Gd) {
-        k_update<true><<<h.G2, kNT, 0, st>>>(pl.d_args, k);
+        k_update<true, false><<<h.G2, kNT, 0, st>>>(pl.d_args, k);
         launch_fac(pl, 0, st);
     } else {
-        k_update<false><<<h.G2, kNT, 0, st>>>(pl.d_args, k);
+        k_update<false, false><<<h.G2, kNT, 0, st>>>(pl.d_args, k);
     }
     k_pupdate<<<h.G2, kNT, 0, st>>>(pl.d_args, k);
     return hipGetLastError();
@@ -1625,7 +1766,7 @@ int set_pattern_arrays(PcgPlanImpl *pl, uint32_t nnz, const uint32_t *rp, const 
     }
     // Choose the SpMV form from the longest row (stored + mirrored blocks).
     PPF_HIP(hipMemsetAsync(flags + 2, 0, sizeof(uint32_t), st));
-    k_row_len_max<<<gb, kNT, 0, st>>>(n, rp, pl->tp, flags + 2);
+    k_row_len_max<<<std::min(gb, kLenGrid), kNT, 0, st>>>(n, rp, pl->tp, flags + 2);
     PPF_HIP(hipGetLastError());
     uint32_t maxlen = 0;
     PPF_HIP(hipMemcpyAsync(&maxlen, flags + 2, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
@@ -1681,6 +1822,7 @@ int set_pattern_arrays(PcgPlanImpl *pl, uint32_t nnz, const uint32_t *rp, const 
             break;
         }
         pl->sym = pl->split && sym_ok && pl->form != PPF_SPMV_SPLIT;
+        pl->fuse = 36ull * nnz < (pl->split ? kFuseBytes : kFuseEllBytes);
     }
     h.ent = nullptr;
     if (h.ell_m && !pl->split) {
@@ -1867,20 +2009,23 @@ int set_tiles(PcgPlanImpl *pl, uint32_t r1, uint32_t r2, hipStream_t st,
         // One round of resident workgroups per kernel (a second, partly
         // filled round costs as much as the first): the SpMV's register use
         // allows 5 workgroups per CU, the vector kernels 8.
-        uint32_t res1 = resident_blocks(k_spmv_split<true, 4>, 1280u);
+        uint32_t res1 = resident_blocks(k_spmv_split<true, 4, false>, 1280u);
         if (!pl->arena) {
             // the symmetric form's LDS may hold fewer workgroups per CU
-            res1 = std::min(res1, resident_blocks(k_spmv_sym<true, 4>, 1280u, kSymLds));
+            res1 = std::min(res1, resident_blocks(k_spmv_sym<true, 4, false>, 1280u, kSymLds));
         }
         const uint32_t g1 = round8(std::min(res1, cdiv(n, 64)));
-        const uint32_t g2 = std::min(resident_blocks(k_update<false>, 2048u), cdiv(n, 64));
+        const uint32_t g2 = std::min(resident_blocks(k_update<false, false>, 2048u), cdiv(n, 64));
         // Rows per tile in chunks of 64, of 32 in a large plan: the product
         // waits for the CU with most rows (527,360 rows, symmetric form: 59.9 us
         // with 416 rows a tile, 61.7 with 448, 68 with 512: 1,030 tiles put a
         // fifth on some CUs).
         const uint32_t step = n >= kOrderRows ? 32u : 64u;
         r1 = cdiv(cdiv(n, g1), step) * step;
-        r2 = cdiv(cdiv(n, g2), 64) * 64;
+        // Vector tiles of at least 128 rows: half the partial sums for every
+        // workgroup to reduce again (65,536 rows: 18.7 -> 17.9 us per iteration;
+        // 256 rows give 17.6, but the factor's second pass then loses 1.4%).
+        r2 = cdiv(cdiv(n, g2), 128) * 128;
         cut(t1, sc1, r1);
         cut(t2, sc2, r2);
         ordered = !pl->arena && n >= kOrderRows;
@@ -2036,8 +2181,8 @@ int plan_init(PcgPlanImpl *pl, uint32_t n, uint32_t nnz, const uint32_t *rp, con
     const size_t n3 = 3 * (size_t)n;
     const size_t scan_words = scan_scratch_words(n + 1);
     size_t bytes = carve_bytes(n + 1, 4) + carve_bytes(n, 4) +
-                   carve_bytes(9 * (size_t)n, 4) + carve_bytes(n3, 4) * 5 +
-                   carve_bytes(1, sizeof(Args)) + carve_bytes(scan_words, 4) +
+                   carve_bytes(9 * (size_t)n, 4) +
+                   carve_bytes(n3, 4) * (pl->arena ? 5 : 6) + carve_bytes(1, sizeof(Args)) + carve_bytes(scan_words, 4) +
                    carve_bytes(4, 4) + carve_bytes(nscene + 1, 4);
     hipError_t e = plan_alloc(pl, &pl->mem, bytes);
     if (e != hipSuccess) {
@@ -2053,6 +2198,7 @@ int plan_init(PcgPlanImpl *pl, uint32_t n, uint32_t nnz, const uint32_t *rp, con
     h.p = carve<float>(cur, n3);
     h.Ap = carve<float>(cur, n3);
     h.gy = carve<float>(cur, n3);
+    h.p2 = pl->arena ? h.gy : carve<float>(cur, n3); // a fixed region solves without a factor
     pl->d_args = carve<Args>(cur, 1);
     pl->scan_tmp = carve<uint32_t>(cur, scan_words);
     pl->flags = carve<uint32_t>(cur, 4);

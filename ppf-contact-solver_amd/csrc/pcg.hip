@@ -18,8 +18,9 @@
 //     the L2 of the XCD that read it as a stored block.
 //   * one iteration = 3 kernels: SpMV + p.Ap + sum|terms|; the fused x/r/z
 //     update with the r.z and |r|_1 partials; p = z + beta p (5 with the
-//     factor preconditioner: G r and G^T (G r) between the last two). Each
-//     kernel writes one partial per workgroup tile; every workgroup of the
+//     factor preconditioner: G r and G^T (G r) between the last two). While
+//     the blocks fit the L2s the SpMV forms p itself, and p's kernel is left
+//     out. Each kernel writes one partial per workgroup tile; every workgroup of the
 //     next kernel reduces its scene's partials itself in a fixed order, so
 //     the scalars are bit-identical everywhere with no atomics and no grid
 //     barrier, and every run is deterministic.

@@ -47,6 +47,8 @@ namespace {
 
 constexpr int kNT = 256;           // threads per workgroup
 constexpr int kGraphIters = 8;     // iterations per captured graph (even)
+constexpr uint32_t kReportIters = 4;       // iterations between progress reports
+constexpr uint32_t kOver = 0x80000000u;    // report: the scene is done
 constexpr unsigned kNone = 0xffffffffu;
 constexpr unsigned kMirror = 0x80000000u; // entry slot flag: apply transposed
 constexpr float kNoiseSlack = 256.0f;       // solver.cu:69
@@ -132,6 +134,10 @@ struct Args {
     // 10-entry (20 B) records; gy holds G r.
     const uint16_t *Gd, *Gl, *Gr; // Gr: the rows of G in order (row j at j + tp[j])
     float *gy;
+    // pinned host memory, or null: per scene the completed iterations (every
+    // kReportIters) and kOver once it is done, and its scalars then
+    uint32_t *report;
+    Scalars *over;
 };
 
 __device__ inline Tile load_tile(const Tile *t, uint32_t L) {
@@ -145,9 +151,10 @@ __global__ void k_count_transpose(uint32_t n, const uint32_t *__restrict__ rp,
                                   const uint32_t *__restrict__ col,
                                   uint32_t *__restrict__ tcount,
                                   uint32_t *__restrict__ dslot,
-                                  uint32_t *__restrict__ bad_pattern) {
+                                  uint32_t *__restrict__ bad_pattern,
+                                  const uint32_t *__restrict__ bad_offsets) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) {
+    if (i >= n || *bad_offsets) {
         return;
     }
     uint32_t ds = kNone;
@@ -174,9 +181,10 @@ __global__ void k_count_transpose(uint32_t n, const uint32_t *__restrict__ rp,
 __global__ void k_transpose_keys(uint32_t n, const uint32_t *__restrict__ rp,
                                  const uint32_t *__restrict__ col,
                                  uint32_t *__restrict__ key, uint32_t *__restrict__ val,
-                                 uint32_t *__restrict__ row) {
+                                 uint32_t *__restrict__ row,
+                                 const uint32_t *__restrict__ bad_offsets) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) {
+    if (i >= n || *bad_offsets) {
         return;
     }
     uint32_t prev = 0;
@@ -209,13 +217,16 @@ __global__ void k_transpose_place(uint32_t nnz, const uint32_t *__restrict__ tp_
 }
 
 // row_offset must start at 0, be non-decreasing and end at nnz.
+// Clears cnt for the count that follows; the kernels that walk the rows do
+// nothing once *bad is set, so that the host reads it with its other answers.
 __global__ void k_check_offsets(uint32_t n, uint32_t nnz,
-                                const uint32_t *__restrict__ rp,
+                                const uint32_t *__restrict__ rp, uint32_t *__restrict__ cnt,
                                 uint32_t *__restrict__ bad) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i > n) {
         return;
     }
+    cnt[i] = 0;
     const uint32_t v = rp[i];
     const bool ok = (i == 0 ? v == 0 : v >= rp[i - 1]) && (i < n || v == nnz) &&
                     v <= nnz;
@@ -326,9 +337,10 @@ __global__ void k_inverse_order(uint32_t n, const uint32_t *__restrict__ order,
 __global__ void k_order_count(uint32_t n, const uint32_t *__restrict__ rp,
                               const uint32_t *__restrict__ col,
                               const uint32_t *__restrict__ inv, uint32_t *__restrict__ cnt,
-                              uint32_t *__restrict__ bad) {
+                              uint32_t *__restrict__ bad,
+                              const uint32_t *__restrict__ bad_offsets) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) {
+    if (i >= n || *bad_offsets) {
         return;
     }
     const uint32_t a = inv[i];
@@ -446,11 +458,36 @@ __device__ inline float reduce_parts(gptr<const float> part, uint32_t cnt,
     return block_sum<kNT>(acc, lds);
 }
 
+// Progress of a scene to the host, which launches the next graph once the
+// current one is half through and stops at kOver: no copy, event or kernel
+// stands between two graphs. The scalars are read after the stream has
+// drained; only the word itself must be seen while kernels run.
+__device__ inline void report_progress(const Args *__restrict__ A, gptr<Scalars> s, uint32_t scene) {
+    if (!A->report) {
+        return;
+    }
+    const bool over = s->done != 0;
+    if (over) {
+        gptr<Scalars> o = as_global(A->over + scene);
+        o->err0 = s->err0;
+        o->status = s->status;
+        o->cause = s->cause;
+        o->break_iter = s->break_iter;
+        o->rep_iter = s->rep_iter;
+        o->rep_resid = s->rep_resid;
+    }
+    if (over || s->iter % kReportIters == 0) {
+        __hip_atomic_store(A->report + scene, s->iter | (over ? kOver : 0u), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 // The end of an iteration: the reference's residual-check schedule
 // (solver.cu:1249-1380) on the sums of r.z and |r|_1, by one thread. rz0: r.z
 // of the iteration before; slot: where the new one goes.
-__device__ inline void end_iteration(const Args *__restrict__ A, gptr<Scalars> s, uint32_t slot,
+__device__ inline void end_iteration(const Args *__restrict__ A, uint32_t scene, uint32_t slot,
                                      float rz0, float rz1, float err) {
+    gptr<Scalars> s = as_global(A->s + scene);
     if (!(rz0 > 0.0f) && s->cause == 0) {
         s->breakdown = 1;
         s->cause = 2;
@@ -487,13 +524,15 @@ __device__ inline void end_iteration(const Args *__restrict__ A, gptr<Scalars> s
             s->next_check = it + s->stride;
         }
     }
+    report_progress(A, s, scene);
 }
 
 // The direction a fused SpMV applies the operator to: p_k = z + beta p_{k-1}
 // (the fmaf of k_pupdate), formed wherever it is gathered and stored by its
-// row's lanes. beta comes from the partials of the update before (from the
-// scalars in a graph's first iteration, whose bookkeeping k_end_graph did); the
-// scene's first tile does the bookkeeping of the iteration before. One kernel
+// row's lanes. beta comes from the partials of the update before and the
+// scene's first tile does the bookkeeping of the iteration before; in a graph's
+// first iteration k = 0 says that k_end_graph has done both, k = kGraphIters
+// that the graph before, if there was one, left them. One kernel
 // and one pass over p less per iteration, against a second gather per entry:
 // it pays while a launch costs more than the gathers (kFuseBytes).
 struct Direction {
@@ -531,7 +570,7 @@ __device__ inline bool start_direction(const Args *__restrict__ A, const Tile &T
     d.out = as_global((k & 1) ? A->p : A->p2);
     float rz1, rz0;
     bool first = false;
-    if (k == 0) {
+    if (k == 0 || (k == (uint32_t)kGraphIters && s->iter == 0)) {
         rz1 = s->rz[0], rz0 = s->rz[1];
         first = s->iter == 0; // p_0 = z
     } else {
@@ -543,7 +582,7 @@ __device__ inline bool start_direction(const Args *__restrict__ A, const Tile &T
             const float err = reduce_parts(part + 2 * A->G1 + A->G2 + t0, nt, lds);
             __shared__ int32_t over;
             if (threadIdx.x == 0) {
-                end_iteration(A, s, k & 1, rz0, rz1, err);
+                end_iteration(A, T.scene, k & 1, rz0, rz1, err);
                 over = s->done;
             }
             __syncthreads();
@@ -1212,6 +1251,21 @@ __global__ __launch_bounds__(kNT) void k_init_scalars(const Args *__restrict__ A
             s->rep_iter = 1;
             s->rep_resid = 0.0f;
         }
+        report_progress(A, s, sc);
+    }
+}
+
+// Arguments and fresh scalars of a solve, from the kernel's own arguments: two
+// copies from host memory took 21 us and a wait.
+__global__ __launch_bounds__(kNT) void k_begin(Args a, Args *dst, float tol, uint32_t max_iter) {
+    if (threadIdx.x == 0) {
+        *dst = a;
+    }
+    for (uint32_t c = threadIdx.x; c < a.nscene; c += kNT) {
+        Scalars s{};
+        s.tol = tol;
+        s.max_iter = max_iter;
+        a.s[c] = s;
     }
 }
 
@@ -1487,10 +1541,11 @@ __global__ __launch_bounds__(kNT) void k_pupdate(const Args *__restrict__ A,
     if (threadIdx.x != 0) {
         return;
     }
-    end_iteration(A, s, (k + 1) & 1, rz0, rz1, err);
+    end_iteration(A, T.scene, (k + 1) & 1, rz0, rz1, err);
 }
 
-// The bookkeeping of a graph's last fused iteration. One workgroup per scene.
+// The bookkeeping of a graph's last fused iteration, for plans whose tiles may
+// change between graphs or whose status is copied there. One workgroup per scene.
 __global__ __launch_bounds__(kNT) void k_end_graph(const Args *__restrict__ A) {
     __shared__ float lds[kNT / kWave];
     gptr<Scalars> s = as_global(A->s + blockIdx.x);
@@ -1502,7 +1557,7 @@ __global__ __launch_bounds__(kNT) void k_end_graph(const Args *__restrict__ A) {
     const float rz1 = reduce_parts(part + 2 * A->G1 + t0, nt, lds);
     const float err = reduce_parts(part + 2 * A->G1 + A->G2 + t0, nt, lds);
     if (threadIdx.x == 0) {
-        end_iteration(A, s, 0, s->rz[1], rz1, err);
+        end_iteration(A, blockIdx.x, 0, s->rz[1], rz1, err);
     }
 }
 
@@ -1531,8 +1586,9 @@ struct PcgPlanImpl {
     uint32_t n = 0, nnz = 0;
     Args h{};             // host copy of the kernel arguments
     Args *d_args = nullptr;
-    Scalars *h_scal = nullptr; // pinned; a one-scene plan holds two (polled in turn)
-    hipEvent_t poll_ev[2] = {nullptr, nullptr}; // status copies of a one-scene plan
+    // pinned, one allocation: scalars and report of every scene, 4 pattern flags
+    Scalars *h_scal = nullptr;
+    uint32_t *h_report = nullptr, *h_flags = nullptr;
     void *mem = nullptr;       // one device allocation for the n-sized scratch
     uint32_t *tp = nullptr, *dslot = nullptr;
     uint32_t *scan_tmp = nullptr, *flags = nullptr;
@@ -1663,12 +1719,14 @@ void launch_fac(const PcgPlanImpl &pl, int init, hipStream_t st) {
 hipError_t launch_iteration(const PcgPlanImpl &pl, uint32_t k, hipStream_t st) {
     const Args &h = pl.h;
     if (pl.fuse && !h.Gd) {
-        const hipError_t e = launch_spmv<true, true>(pl, nullptr, h.Ap, st, k);
+        const bool end = h.nscene > 1 || pl.arena;
+        const hipError_t e = launch_spmv<true, true>(pl, nullptr, h.Ap, st,
+                                                     k || end ? k : (uint32_t)kGraphIters);
         if (e != hipSuccess) {
             return e;
         }
         k_update<false, true><<<h.G2, kNT, 0, st>>>(pl.d_args, k);
-        if (k + 1 == (uint32_t)kGraphIters) {
+        if (end && k + 1 == (uint32_t)kGraphIters) {
             k_end_graph<<<h.nscene, kNT, 0, st>>>(pl.d_args);
         }
         return hipGetLastError();
@@ -1690,6 +1748,27 @@ hipError_t launch_iteration(const PcgPlanImpl &pl, uint32_t k, hipStream_t st) {
 } // namespace
 
 namespace {
+
+// The flags of a pattern's checks, read once behind all the kernels they gate:
+// flags[1] bad offsets, flags[0] bad entries. A read after each check cost a
+// round trip of 30 us.
+int read_pattern_flags(PcgPlanImpl *pl, uint32_t count, uint32_t *out, hipStream_t st) {
+    uint32_t *to = pl->h_flags ? pl->h_flags : out;
+    PPF_HIP(hipMemcpyAsync(to, pl->flags, count * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    PPF_HIP(hipStreamSynchronize(st));
+    std::copy(to, to + count, out);
+    if (out[1]) {
+        set_error("pcg: row_offset is not a valid CSR offset array (0 .. nnz, non-decreasing)");
+        return PPF_ERR_ARG;
+    }
+    if (out[0]) {
+        set_error("pcg: %u pattern entries are not strictly ascending upper-triangle "
+                  "columns < n",
+                  out[0]);
+        return PPF_ERR_ARG;
+    }
+    return PPF_OK;
+}
 
 // Transpose table, row-length choice of the SpMV form and the ELL table for
 // a pattern. Buffers sized by nnz (or n * row width) grow when needed.
@@ -1730,24 +1809,16 @@ int set_pattern_arrays(PcgPlanImpl *pl, uint32_t nnz, const uint32_t *rp, const 
     h.tslot = tslot;
     h.dslot = pl->dslot;
     uint32_t *flags = pl->flags;
-    PPF_HIP(hipMemsetAsync(pl->tp, 0, (n + 1) * sizeof(uint32_t), st));
     PPF_HIP(hipMemsetAsync(flags, 0, 4 * sizeof(uint32_t), st));
     const unsigned gb = cdiv(n, kNT);
-    uint32_t bad = 0;
-    k_check_offsets<<<cdiv(n + 1, kNT), kNT, 0, st>>>(n, nnz, rp, flags + 1);
+    k_check_offsets<<<cdiv(n + 1, kNT), kNT, 0, st>>>(n, nnz, rp, pl->tp, flags + 1);
     PPF_HIP(hipGetLastError());
-    PPF_HIP(hipMemcpyAsync(&bad, flags + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    PPF_HIP(hipStreamSynchronize(st));
-    if (bad) {
-        set_error("pcg: row_offset is not a valid CSR offset array (0 .. nnz, non-decreasing)");
-        return PPF_ERR_ARG;
-    }
-    k_count_transpose<<<gb, kNT, 0, st>>>(n, rp, col, pl->tp, pl->dslot, flags);
+    k_count_transpose<<<gb, kNT, 0, st>>>(n, rp, col, pl->tp, pl->dslot, flags, flags + 1);
     PPF_HIP(hipGetLastError());
     PPF_HIP(exclusive_scan_u32(pl->tp, pl->tp, n + 1, pl->scan_tmp, st));
     if (nnz) {
         uint32_t *key = pl->tsort, *val = key + nnz, *row = val + nnz, *scratch = row + nnz;
-        k_transpose_keys<<<gb, kNT, 0, st>>>(n, rp, col, key, val, row);
+        k_transpose_keys<<<gb, kNT, 0, st>>>(n, rp, col, key, val, row, flags + 1);
         PPF_HIP(hipGetLastError());
         uint32_t bits = 1;
         while (bits < 32 && (n >> bits) != 0) {
@@ -1757,21 +1828,15 @@ int set_pattern_arrays(PcgPlanImpl *pl, uint32_t nnz, const uint32_t *rp, const 
         k_transpose_place<<<cdiv(nnz, kNT), kNT, 0, st>>>(nnz, pl->tp + n, val, row, tcol, tslot);
         PPF_HIP(hipGetLastError());
     }
-    PPF_HIP(hipMemcpyAsync(&bad, flags, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    PPF_HIP(hipStreamSynchronize(st));
-    if (bad) {
-        set_error("pcg: %u pattern entries are not strictly ascending upper-triangle "
-                  "columns < n",
-                  bad);
-        return PPF_ERR_ARG;
-    }
-    // Choose the SpMV form from the longest row (stored + mirrored blocks).
-    PPF_HIP(hipMemsetAsync(flags + 2, 0, sizeof(uint32_t), st));
     k_row_len_max<<<std::min(gb, kLenGrid), kNT, 0, st>>>(n, rp, pl->tp, flags + 2);
     PPF_HIP(hipGetLastError());
-    uint32_t maxlen = 0;
-    PPF_HIP(hipMemcpyAsync(&maxlen, flags + 2, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    PPF_HIP(hipStreamSynchronize(st));
+    uint32_t found[3];
+    int rc = read_pattern_flags(pl, 3, found, st);
+    if (rc != PPF_OK) {
+        return rc;
+    }
+    // Choose the SpMV form from the longest row (stored + mirrored blocks).
+    const uint32_t maxlen = found[2];
     h.ell_m = 0;
     for (uint32_t m : {1u, 2u, 3u, 4u, 6u, 8u}) {
         // Padding entries read block 0, so the ELL form needs nnz >= 1.
@@ -1937,28 +2002,16 @@ int set_pattern_ordered(PcgPlanImpl *pl, uint32_t nnz, const uint32_t *rp, const
         pl->pval = reinterpret_cast<float *>(pl->smap + cap);
     }
     uint32_t *flags = pl->flags;
-    uint32_t bad = 0;
-    PPF_HIP(hipMemsetAsync(flags + 1, 0, sizeof(uint32_t), st));
-    k_check_offsets<<<cdiv(n + 1, kNT), kNT, 0, st>>>(n, nnz, rp, flags + 1);
+    PPF_HIP(hipMemsetAsync(flags, 0, 2 * sizeof(uint32_t), st));
+    k_check_offsets<<<cdiv(n + 1, kNT), kNT, 0, st>>>(n, nnz, rp, pl->cursor, flags + 1);
     PPF_HIP(hipGetLastError());
-    PPF_HIP(hipMemcpyAsync(&bad, flags + 1, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    PPF_HIP(hipStreamSynchronize(st));
-    if (bad) {
-        set_error("pcg: row_offset is not a valid CSR offset array (0 .. nnz, non-decreasing)");
-        return PPF_ERR_ARG;
-    }
     const unsigned gb = cdiv(n, kNT);
-    PPF_HIP(hipMemsetAsync(pl->cursor, 0, (n + 1) * sizeof(uint32_t), st));
-    PPF_HIP(hipMemsetAsync(flags, 0, sizeof(uint32_t), st));
-    k_order_count<<<gb, kNT, 0, st>>>(n, rp, col, pl->inv, pl->cursor, flags);
+    k_order_count<<<gb, kNT, 0, st>>>(n, rp, col, pl->inv, pl->cursor, flags, flags + 1);
     PPF_HIP(hipGetLastError());
-    PPF_HIP(hipMemcpyAsync(&bad, flags, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    PPF_HIP(hipStreamSynchronize(st));
-    if (bad) {
-        set_error("pcg: %u pattern entries are not strictly ascending upper-triangle "
-                  "columns < n",
-                  bad);
-        return PPF_ERR_ARG;
+    uint32_t found[2];
+    int rc = read_pattern_flags(pl, 2, found, st);
+    if (rc != PPF_OK) {
+        return rc;
     }
     PPF_HIP(exclusive_scan_u32(pl->cursor, pl->prp, n + 1, pl->scan_tmp, st));
     PPF_HIP(hipMemsetAsync(pl->cursor, 0, (n + 1) * sizeof(uint32_t), st));
@@ -1967,7 +2020,7 @@ int set_pattern_ordered(PcgPlanImpl *pl, uint32_t nnz, const uint32_t *rp, const
     PPF_HIP(hipGetLastError());
     k_order_sort<<<gb, kNT, 0, st>>>(n, pl->prp, pl->pcol, pl->smap);
     PPF_HIP(hipGetLastError());
-    const int rc = set_pattern_arrays(pl, nnz, pl->prp, pl->pcol, st);
+    rc = set_pattern_arrays(pl, nnz, pl->prp, pl->pcol, st);
     pl->order_built = rc == PPF_OK;
     return rc;
 }
@@ -2183,8 +2236,8 @@ int plan_init(PcgPlanImpl *pl, uint32_t n, uint32_t nnz, const uint32_t *rp, con
     const size_t scan_words = scan_scratch_words(n + 1);
     size_t bytes = carve_bytes(n + 1, 4) + carve_bytes(n, 4) +
                    carve_bytes(9 * (size_t)n, 4) +
-                   carve_bytes(n3, 4) * (pl->arena ? 5 : 6) + carve_bytes(1, sizeof(Args)) + carve_bytes(scan_words, 4) +
-                   carve_bytes(4, 4) + carve_bytes(nscene + 1, 4);
+                   carve_bytes(n3, 4) * (pl->arena ? 5 : 6) + carve_bytes(1, sizeof(Args)) +
+                   carve_bytes(scan_words, 4) + carve_bytes(4 + nscene + 1, 4);
     hipError_t e = plan_alloc(pl, &pl->mem, bytes);
     if (e != hipSuccess) {
         set_error("pcg_plan_create: %zu bytes of scratch: %s", bytes, hipGetErrorString(e));
@@ -2202,24 +2255,17 @@ int plan_init(PcgPlanImpl *pl, uint32_t n, uint32_t nnz, const uint32_t *rp, con
     h.p2 = pl->arena ? h.gy : carve<float>(cur, n3); // a fixed region solves without a factor
     pl->d_args = carve<Args>(cur, 1);
     pl->scan_tmp = carve<uint32_t>(cur, scan_words);
-    pl->flags = carve<uint32_t>(cur, 4);
-    uint32_t *d_srow = carve<uint32_t>(cur, nscene + 1);
+    pl->flags = carve<uint32_t>(cur, 4 + nscene + 1);
+    uint32_t *d_srow = pl->flags + 4;
     if (!pl->arena) {
-        const uint32_t nbuf = nscene == 1 ? 2u : nscene;
-        e = host_alloc(reinterpret_cast<void **>(&pl->h_scal), nbuf * sizeof(Scalars));
+        e = host_alloc(reinterpret_cast<void **>(&pl->h_scal),
+                       nscene * (sizeof(Scalars) + 4) + 4 * 4);
         if (e != hipSuccess) {
             set_error("pcg_plan_create: hipHostMalloc: %s", hipGetErrorString(e));
             return PPF_ERR_HIP;
         }
-        if (nscene == 1) {
-            for (hipEvent_t &ev : pl->poll_ev) {
-                e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-                if (e != hipSuccess) {
-                    set_error("pcg_plan_create: hipEventCreate: %s", hipGetErrorString(e));
-                    return PPF_ERR_HIP;
-                }
-            }
-        }
+        pl->h_report = reinterpret_cast<uint32_t *>(pl->h_scal + nscene);
+        pl->h_flags = pl->h_report + nscene;
     }
     int rc = set_pattern(pl, nnz, rp, col, st);
     if (rc == PPF_OK && nscene > 1) {
@@ -2319,11 +2365,6 @@ void pcg_plan_destroy(PcgPlanImpl *pl) {
     }
     if (pl->cap) {
         (void)hipStreamDestroy(pl->cap);
-    }
-    for (hipEvent_t ev : pl->poll_ev) {
-        if (ev) {
-            (void)hipEventDestroy(ev);
-        }
     }
     if (pl->h_scal) {
         (void)host_free(pl->h_scal);
@@ -2447,6 +2488,98 @@ int pcg_time_spmv(PcgPlanImpl *pl, const float *val, const float *cdiag,
     return PPF_OK;
 }
 
+namespace {
+
+int bookkeeping_lost() {
+    set_error("pcg_solve: bookkeeping did not terminate");
+    return PPF_ERR_SOLVER;
+}
+
+// Replays the iteration graph until every scene reports that it is done. The
+// next graph is launched when the current one is half through, so the device
+// does not wait for the host and at most one and a half graphs, whose kernels
+// exit at entry, follow the last iteration. With many scenes, once the scenes
+// still iterating hold under 3/4 of the tiled rows, the tiles are cut again
+// over those scenes only (the partial sums are written and read within one
+// graph, so the switch between graphs is safe). A status copy and its event
+// after each graph took 21 us of a small solve's 97 for eight iterations.
+int replay_graphs(PcgPlanImpl *pl, uint32_t max_launch, hipStream_t st) {
+    const uint32_t ns = pl->nscene;
+    uint32_t tiled_rows = pl->n, launched = 0, spins = 0;
+    std::vector<uint8_t> active(ns, 1u);
+    bool idle = true; // the stream had run dry when the reports below were read
+    for (;;) {
+        uint32_t live_rows = 0, at = 0;
+        for (uint32_t c = 0; c < ns; ++c) {
+            const uint32_t w = __atomic_load_n(pl->h_report + c, __ATOMIC_ACQUIRE);
+            active[c] = !(w & kOver);
+            if (active[c]) {
+                live_rows += std::max(pl->scene_row[c + 1] - pl->scene_row[c], 1u);
+                at = std::max(at, w);
+            }
+        }
+        if (live_rows == 0) {
+            return PPF_OK;
+        }
+        if (idle && launched >= max_launch) {
+            return bookkeeping_lost();
+        }
+        if (launched < max_launch && (idle || at + kGraphIters / 2 >= launched * kGraphIters)) {
+            if (ns > 1 && launched && 4ull * live_rows < 3ull * tiled_rows) {
+                if (!idle) { // scenes may still end in the graph in flight
+                    PPF_HIP(hipStreamSynchronize(st));
+                    idle = true;
+                    continue;
+                }
+                int rc = set_tiles(pl, pl->tile_r1, pl->tile_r2, st, &active);
+                if (rc == PPF_OK) {
+                    PPF_HIP(hipMemcpyAsync(pl->d_args, &pl->h, sizeof(Args), hipMemcpyHostToDevice,
+                                           st));
+                    rc = capture_graph(pl);
+                }
+                if (rc != PPF_OK) {
+                    return rc;
+                }
+                tiled_rows = live_rows;
+            } else {
+                PPF_HIP(hipGraphLaunch(pl->exec, st));
+                ++launched;
+            }
+            idle = false;
+            continue;
+        }
+        // An error, or a stream that ran dry, shows in the stream's state.
+        if (++spins % 4096 == 0) {
+            const hipError_t e = hipStreamQuery(st);
+            if (e != hipSuccess && e != hipErrorNotReady) {
+                PPF_HIP(e);
+            }
+            idle = e == hipSuccess;
+        }
+        __builtin_ia32_pause();
+    }
+}
+
+// A plan on a fixed region: the graph's iterations, launched one by one, and
+// the status copied after every kGraphIters.
+int run_iterations(PcgPlanImpl *pl, uint32_t max_launch, hipStream_t st) {
+    for (uint32_t g = 0;; ++g) {
+        PPF_HIP(hipMemcpyAsync(pl->h_scal, pl->h.s, sizeof(Scalars), hipMemcpyDeviceToHost, st));
+        PPF_HIP(hipStreamSynchronize(st));
+        if (pl->h_scal->done) {
+            return PPF_OK;
+        }
+        if (g >= max_launch) {
+            return bookkeeping_lost();
+        }
+        for (uint32_t k = 0; k < (uint32_t)kGraphIters; ++k) {
+            PPF_HIP(launch_iteration(*pl, k, st));
+        }
+    }
+}
+
+} // namespace
+
 int pcg_solve(PcgPlanImpl *pl, const float *val, const float *cdiag,
               const float *b, float *x, float tol, uint32_t max_iter,
               float *err_hist, ppf_pcg_result *res, hipStream_t st, const PcgFactor *fac) {
@@ -2501,17 +2634,14 @@ int pcg_solve(PcgPlanImpl *pl, const float *val, const float *cdiag,
             return rc;
         }
     }
-    PPF_HIP(hipMemcpyAsync(pl->d_args, &h, sizeof(Args), hipMemcpyHostToDevice,
-                           st));
-    // the pinned status buffer stages the initial scalars of every scene
-    PPF_HIP(hipStreamSynchronize(st));
-    for (uint32_t c = 0; c < ns; ++c) {
-        Scalars init{};
-        init.tol = tol;
-        init.max_iter = max_iter;
-        pl->h_scal[c] = init;
+    // every solve ends on a drained stream, so no kernel writes these now
+    h.report = pl->h_report;
+    h.over = pl->h_scal;
+    for (uint32_t c = 0; pl->h_report && c < ns; ++c) {
+        __atomic_store_n(pl->h_report + c, 0u, __ATOMIC_RELEASE);
     }
-    PPF_HIP(hipMemcpyAsync(h.s, pl->h_scal, ns * sizeof(Scalars), hipMemcpyHostToDevice, st));
+    k_begin<<<1, kNT, 0, st>>>(h, pl->d_args, tol, max_iter);
+    PPF_HIP(hipGetLastError());
     if (!Gd) {
         k_diag_invert<<<h.G2, kNT, 0, st>>>(pl->d_args);
         PPF_HIP(hipGetLastError());
@@ -2527,99 +2657,17 @@ int pcg_solve(PcgPlanImpl *pl, const float *val, const float *cdiag,
     k_init_scalars<<<ns, kNT, 0, st>>>(pl->d_args);
     PPF_HIP(hipGetLastError());
     const uint32_t max_launch = max_iter / kGraphIters + 2;
-    if (pl->exec && ns == 1) {
-        // One scene: keep one graph of iterations in flight while the host
-        // reads the status copied after the graph before it (two pinned
-        // status words, an event each), so the device never idles on the
-        // host's poll. Graphs launched after the solve is done exit at entry.
-        Scalars *buf[2] = {pl->h_scal, pl->h_scal + 1};
-        for (uint32_t k = 0; k < 2; ++k) {
-            PPF_HIP(hipGraphLaunch(pl->exec, st));
-            PPF_HIP(hipMemcpyAsync(buf[k], h.s, sizeof(Scalars), hipMemcpyDeviceToHost, st));
-            PPF_HIP(hipEventRecord(pl->poll_ev[k], st));
-        }
-        uint32_t k = 0;
-        for (;; ++k) {
-            PPF_HIP(hipEventSynchronize(pl->poll_ev[k & 1]));
-            if (buf[k & 1]->done != 0) {
-                break;
-            }
-            if (k + 2 >= max_launch) {
-                (void)hipStreamSynchronize(st);
-                set_error("pcg_solve: bookkeeping did not terminate");
-                return PPF_ERR_SOLVER;
-            }
-            PPF_HIP(hipGraphLaunch(pl->exec, st));
-            PPF_HIP(hipMemcpyAsync(buf[k & 1], h.s, sizeof(Scalars), hipMemcpyDeviceToHost, st));
-            PPF_HIP(hipEventRecord(pl->poll_ev[k & 1], st));
-        }
-        const Scalars done = *buf[k & 1];
-        if (pl->order) {
-            k_order_rows<true><<<cdiv(3 * pl->n, kNT), kNT, 0, st>>>(pl->n, 3, pl->order, x,
-                                                                     x_caller);
-            PPF_HIP(hipGetLastError());
-        }
-        PPF_HIP(hipStreamSynchronize(st)); // the graph still in flight ends here
-        res[0].iter = done.rep_iter;
-        res[0].resid = done.rep_resid;
-        res[0].status = done.status;
-        res[0].break_cause = done.cause;
-        res[0].break_iter = done.break_iter;
-        res[0].err0 = done.err0;
-        return PPF_OK;
-    }
-    // Replay graphs until the device bookkeeping reports every scene done.
-    // The first status read follows one graph; the iteration cap bounds the
-    // loop. With many scenes, once the scenes still iterating hold under 3/4
-    // of the tiled rows, the tiles are cut again over those scenes only (the
-    // partial sums are written and read within one iteration, so the switch
-    // between graphs is safe).
-    uint32_t tiled_rows = pl->n;
-    std::vector<uint8_t> active(ns, 1u);
-    for (uint32_t g = 0;; ++g) {
-        PPF_HIP(hipMemcpyAsync(pl->h_scal, h.s, ns * sizeof(Scalars),
-                               hipMemcpyDeviceToHost, st));
-        PPF_HIP(hipStreamSynchronize(st));
-        uint32_t live_rows = 0, live = 0;
-        for (uint32_t c = 0; c < ns; ++c) {
-            active[c] = pl->h_scal[c].done == 0;
-            if (active[c]) {
-                ++live;
-                live_rows += pl->scene_row[c + 1] - pl->scene_row[c];
-            }
-        }
-        if (live == 0) {
-            break;
-        }
-        if (g >= max_launch) {
-            set_error("pcg_solve: bookkeeping did not terminate");
-            return PPF_ERR_SOLVER;
-        }
-        if (ns > 1 && 4ull * live_rows < 3ull * tiled_rows) {
-            int rc = set_tiles(pl, pl->tile_r1, pl->tile_r2, st, &active);
-            if (rc == PPF_OK) {
-                PPF_HIP(hipMemcpyAsync(pl->d_args, &h, sizeof(Args), hipMemcpyHostToDevice, st));
-                rc = capture_graph(pl);
-            }
-            if (rc != PPF_OK) {
-                return rc;
-            }
-            tiled_rows = live_rows;
-        }
-        if (pl->exec) {
-            PPF_HIP(hipGraphLaunch(pl->exec, st));
-        } else { // a plan on a fixed region: the graph's iterations, launched one by one
-            for (uint32_t k = 0; k < (uint32_t)kGraphIters; ++k) {
-                PPF_HIP(launch_iteration(*pl, k, st));
-            }
-        }
+    int rc = pl->exec ? replay_graphs(pl, max_launch, st) : run_iterations(pl, max_launch, st);
+    if (rc != PPF_OK) {
+        (void)hipStreamSynchronize(st);
+        return rc;
     }
     if (pl->order) {
         k_order_rows<true><<<cdiv(3 * pl->n, kNT), kNT, 0, st>>>(pl->n, 3, pl->order, x,
                                                                  x_caller);
         PPF_HIP(hipGetLastError());
-        PPF_HIP(hipStreamSynchronize(st));
     }
+    PPF_HIP(hipStreamSynchronize(st)); // the graph still in flight ends here
     for (uint32_t c = 0; c < ns; ++c) {
         const Scalars &sc = pl->h_scal[c];
         res[c].iter = sc.rep_iter;
@@ -2847,7 +2895,7 @@ size_t noalloc_bytes(uint32_t n, uint32_t nnz) {
     const size_t mem = carve_bytes(n + 1, 4) + carve_bytes(n, 4) +
                        carve_bytes(9 * (size_t)n, 4) + carve_bytes(n3, 4) * 5 +
                        carve_bytes(1, sizeof(Args)) + carve_bytes(scan_scratch_words(n + 1), 4) +
-                       carve_bytes(4, 4) + carve_bytes(2, 4);
+                       carve_bytes(4 + 2, 4);
     const size_t pat = carve_bytes(2 * ((size_t)nnz + nnz / 4 + 256), 4);
     const size_t sort_words = 3 * (size_t)nnz + radix_sort_scratch_words(nnz);
     const size_t tsort = carve_bytes(sort_words + sort_words / 4 + 256, 4);

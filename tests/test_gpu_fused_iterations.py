@@ -60,3 +60,28 @@ def test_fused_caps_follow_the_oracle(dev, form):
         assert abs(r.resid - o["resid"]) <= 1e-3 * o["resid"]
         assert np.abs(x.cpu().numpy() - o["x"]).max() <= 1e-3 * np.abs(o["x"]).max()
     plan.close()
+
+
+@pytest.mark.parametrize("ordered", [False, True])
+def test_a_refused_pattern_leaves_the_plan_usable(dev, ordered):
+    """The checks of a pattern are read once, behind the kernels they gate."""
+    s = cloth(21, 1)
+    t = to_dev(s, dev)
+    n = len(s["row_offset"]) - 1
+    plan = BlockJacobiPCG(t["row_offset"], t["col_index"])
+    if ordered:
+        plan.set_order(torch.arange(n - 1, -1, -1, dtype=torch.int32, device=dev))
+        plan.repattern(t["row_offset"], t["col_index"])
+    x0 = torch.zeros_like(t["b"])
+    first = plan.solve(t["value"], t["cdiag"], t["b"], x0)
+    ro, ci = t["row_offset"].clone(), t["col_index"].clone()
+    ro[5] = t["col_index"].numel() + 7  # beyond the pattern: nothing may follow it
+    ci[3] = n + 100
+    for bad in ((ro, t["col_index"]), (t["row_offset"], ci), (ro, ci)):
+        with pytest.raises(RuntimeError):
+            plan.repattern(*bad)
+    plan.repattern(t["row_offset"], t["col_index"])
+    x = torch.zeros_like(t["b"])
+    again = plan.solve(t["value"], t["cdiag"], t["b"], x)
+    assert (again.iter, again.resid) == (first.iter, first.resid) and torch.equal(x, x0)
+    plan.close()

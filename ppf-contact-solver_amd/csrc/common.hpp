@@ -110,9 +110,11 @@ template <int NT> __device__ inline float block_sum(float v, float *lds) {
 // Workgroup id remapped so that each XCD owns one contiguous range of logical
 // ids (the hardware deals workgroups to the 8 XCDs round-robin). Consecutive
 // rows then share one XCD's L2. Requires gridDim.x % 8 == 0.
-__device__ inline unsigned xcd_logical_block() {
-    const unsigned g = gridDim.x, b = blockIdx.x;
+__device__ inline unsigned xcd_logical_block(unsigned b, unsigned g) {
     return (b % kXcd) * (g / kXcd) + b / kXcd;
+}
+__device__ inline unsigned xcd_logical_block() {
+    return xcd_logical_block(blockIdx.x, gridDim.x);
 }
 
 // Grid of at least `blocks` workgroups that xcd_logical_block can remap (the

@@ -36,8 +36,9 @@ struct Ctx {
     uint64_t cap;
     uint32_t *overflow; // [0] stack overflow, [1] output overflow
     ppf_pair *stash;    // kStash per query, filled by the count pass (may be null)
-    uint32_t *redo;     // fill pass: only these leaf positions (null: all)
-    uint32_t nredo;
+    uint32_t *redo;     // fill pass: the leaf positions, vertices', then edges' from [nv] on
+    uint32_t vq, eq;    // vertex and edge queries of a launch, and the workgroups of the
+    uint32_t vblocks;   // vertex queries (a multiple of the XCDs); the edges' follow
     unsigned long long *stats; // walk statistics of the count pass (null: off)
 };
 
@@ -73,25 +74,21 @@ __device__ inline void emit(const Ctx &c, uint64_t &slot, uint32_t qpos, uint32_
 // stashed count) the listed ones. False: none. Consecutive leaves share an
 // XCD (and its L2), as do their tree walks.
 template <bool FILL>
-__device__ inline bool query_pos(const Ctx &c, uint32_t n, uint32_t &leaf_pos) {
-    const uint32_t t = xcd_logical_block() * kQT + threadIdx.x;
-    if (!FILL || !c.redo) {
-        leaf_pos = t;
-        return t < n;
-    }
-    if (t >= c.nredo) {
+__device__ inline bool query_pos(const Ctx &c, uint32_t block, uint32_t n, uint32_t list,
+                                 uint32_t &leaf_pos) {
+    const uint32_t t = block * kQT + threadIdx.x;
+    if (t >= n) {
         return false;
     }
-    leaf_pos = c.redo[t];
+    leaf_pos = FILL ? c.redo[list + t] : t;
     return true;
 }
 
-template <bool FILL, int STACK, bool STATS = false>
-__global__ __launch_bounds__(kQT) void k_vertex_queries(Ctx c) {
-    __shared__ uint32_t stk_all[STACK * kQT];
+template <bool FILL, int STACK, bool STATS>
+__device__ inline void vertex_queries(const Ctx &c, uint32_t block, uint32_t *stk_all) {
     uint32_t leaf_pos;
     const ppf_contact_mesh &m = c.m;
-    const bool has = query_pos<FILL>(c, c.vb.n, leaf_pos);
+    const bool has = query_pos<FILL>(c, block, c.vq, 0, leaf_pos);
     WalkCount wc;
     [&] {
     if (!has) {
@@ -247,12 +244,11 @@ __global__ __launch_bounds__(kQT) void k_vertex_queries(Ctx c) {
 }
 
 // edge-edge (contact.cu:787-870), queries in edge-BVH leaf order.
-template <bool FILL, int STACK, bool STATS = false>
-__global__ __launch_bounds__(kQT) void k_edge_queries(Ctx c) {
-    __shared__ uint32_t stk_all[STACK * kQT];
+template <bool FILL, int STACK, bool STATS>
+__device__ inline void edge_queries(const Ctx &c, uint32_t block, uint32_t *stk_all) {
     uint32_t leaf_pos;
     const ppf_contact_mesh &m = c.m;
-    const bool has = query_pos<FILL>(c, c.eb.n, leaf_pos);
+    const bool has = query_pos<FILL>(c, block, c.eq, c.vb.n, leaf_pos);
     WalkCount wc;
     [&] {
     if (!has) {
@@ -311,6 +307,22 @@ __global__ __launch_bounds__(kQT) void k_edge_queries(Ctx c) {
     }();
     if (STATS) {
         walk_flush(c.stats, kWalkProxEdge, wc, has);
+    }
+}
+
+// Both kinds of queries in one launch: a wave's walks are a chain of dependent
+// loads (a vertex's three 230 us, an edge's 155 on a 64 x 64 sheet over a
+// sphere, with 64 and 190 waves on the chip), so they run side by side
+// (proximity() of that sheet 381 -> 222 us; 8 x 201 x 201 sheets 2,435 ->
+// 2,169 us; 1M independent triangles 4,224 -> 4,149 us).
+template <bool FILL, int STACK, bool STATS = false>
+__global__ __launch_bounds__(kQT) void k_proximity(Ctx c) {
+    __shared__ uint32_t stk_all[STACK * kQT];
+    if (blockIdx.x < c.vblocks) {
+        vertex_queries<FILL, STACK, STATS>(c, xcd_logical_block(blockIdx.x, c.vblocks), stk_all);
+    } else {
+        edge_queries<FILL, STACK, STATS>(
+            c, xcd_logical_block(blockIdx.x - c.vblocks, gridDim.x - c.vblocks), stk_all);
     }
 }
 
@@ -391,9 +403,9 @@ __device__ inline f3 SX(const ppf_static_mesh &sm, uint32_t v) {
 }
 
 // Dynamic vertex vs static face (kind 4), one thread per vertex leaf.
-template <bool FILL, int STACK> __global__ __launch_bounds__(kQT) void k_m2c(SCtx c) {
-    __shared__ uint32_t stk_all[STACK * kQT];
-    const uint32_t qpos = blockIdx.x * kQT + threadIdx.x;
+template <bool FILL, int STACK>
+__device__ inline void m2c_queries(const SCtx &c, uint32_t block, uint32_t *stk_all) {
+    const uint32_t qpos = block * kQT + threadIdx.x;
     if (qpos >= c.vb.n) {
         return;
     }
@@ -429,9 +441,9 @@ template <bool FILL, int STACK> __global__ __launch_bounds__(kQT) void k_m2c(SCt
 }
 
 // Static vertex vs dynamic face (kind 5), one thread per static vertex.
-template <bool FILL, int STACK> __global__ __launch_bounds__(kQT) void k_c2m(SCtx c) {
-    __shared__ uint32_t stk_all[STACK * kQT];
-    const uint32_t sv = blockIdx.x * kQT + threadIdx.x;
+template <bool FILL, int STACK>
+__device__ inline void c2m_queries(const SCtx &c, uint32_t block, uint32_t *stk_all) {
+    const uint32_t sv = block * kQT + threadIdx.x;
     if (sv >= c.sm.nv) {
         return;
     }
@@ -467,9 +479,9 @@ template <bool FILL, int STACK> __global__ __launch_bounds__(kQT) void k_c2m(SCt
 }
 
 // Dynamic edge vs static edge (kind 6), one thread per edge leaf.
-template <bool FILL, int STACK> __global__ __launch_bounds__(kQT) void k_cm_ee(SCtx c) {
-    __shared__ uint32_t stk_all[STACK * kQT];
-    const uint32_t lp = blockIdx.x * kQT + threadIdx.x;
+template <bool FILL, int STACK>
+__device__ inline void cm_ee_queries(const SCtx &c, uint32_t block, uint32_t *stk_all) {
+    const uint32_t lp = block * kQT + threadIdx.x;
     if (lp >= c.eb.n) {
         return;
     }
@@ -502,6 +514,21 @@ template <bool FILL, int STACK> __global__ __launch_bounds__(kQT) void k_cm_ee(S
     }
     if (!FILL) {
         c.cnt[qpos] = total;
+    }
+}
+
+// The three kinds side by side, as in k_proximity: workgroups of the dynamic
+// vertices, of the collision mesh's, of the edges.
+template <bool FILL, int STACK>
+__global__ __launch_bounds__(kQT) void k_static_proximity(SCtx c) {
+    __shared__ uint32_t stk_all[STACK * kQT];
+    const uint32_t b0 = (c.m.nv + kQT - 1) / kQT, b1 = b0 + (c.sm.nv + kQT - 1) / kQT;
+    if (blockIdx.x < b0) {
+        m2c_queries<FILL, STACK>(c, blockIdx.x, stk_all);
+    } else if (blockIdx.x < b1) {
+        c2m_queries<FILL, STACK>(c, blockIdx.x - b0, stk_all);
+    } else {
+        cm_ee_queries<FILL, STACK>(c, blockIdx.x - b1, stk_all);
     }
 }
 
@@ -623,29 +650,26 @@ int Narrow::proximity_pass(const ppf_contact_mesh &m, ppf_pair *out, uint64_t ca
     c.overflow = flags_;
     c.stash = fill ? stash_ : nullptr;
     c.redo = nullptr;
-    c.nredo = 0;
     c.stats = walk_stats_device();
-    if (m.nv) {
-        WalkClock clk(kWalkProxVertex, s);
-        if (c.stats) {
-            k_vertex_queries<false, kDeepStack, true>
-                <<<xcd_grid(cdiv(m.nv, kQT)), kQT, 0, s>>>(c);
-        } else {
-            k_vertex_queries<false, STACK><<<xcd_grid(cdiv(m.nv, kQT)), kQT, 0, s>>>(c);
+    auto queries = [&](auto kernel, uint32_t vq, uint32_t eq) {
+        c.vq = vq, c.eq = eq, c.vblocks = xcd_grid(cdiv(vq, kQT));
+        const uint32_t blocks = c.vblocks + xcd_grid(cdiv(eq, kQT));
+        if (blocks) {
+            kernel<<<blocks, kQT, 0, s>>>(c);
         }
-        PPF_HIP(hipGetLastError());
-        clk.stop();
-    }
-    if (m.ne) {
-        WalkClock clk(kWalkProxEdge, s);
-        if (c.stats) {
-            k_edge_queries<false, kDeepStack, true>
-                <<<xcd_grid(cdiv(m.ne, kQT)), kQT, 0, s>>>(c);
-        } else {
-            k_edge_queries<false, STACK><<<xcd_grid(cdiv(m.ne, kQT)), kQT, 0, s>>>(c);
+        return hipGetLastError();
+    };
+    if (c.stats) { // timed one kind at a time
+        for (int kind = 0; kind < 2; ++kind) {
+            if (kind ? m.ne : m.nv) {
+                WalkClock clk(kind ? kWalkProxEdge : kWalkProxVertex, s);
+                PPF_HIP(queries(k_proximity<false, kDeepStack, true>, kind ? 0 : m.nv,
+                                kind ? m.ne : 0));
+                clk.stop();
+            }
         }
-        PPF_HIP(hipGetLastError());
-        clk.stop();
+    } else {
+        PPF_HIP(queries(k_proximity<false, STACK>, m.nv, m.ne));
     }
     PPF_HIP(hipMemsetAsync(cnt_ + nq, 0, sizeof(uint32_t), s));
     PPF_HIP(exclusive_scan_u32(cnt_, ofs_, nq + 1, scratch_, s));
@@ -663,20 +687,7 @@ int Narrow::proximity_pass(const ppf_contact_mesh &m, ppf_pair *out, uint64_t ca
     PPF_HIP(hipStreamSynchronize(s));
     *count = h_flags_[4];
     if (fill && !h_flags_[0]) {
-        const uint32_t nv_redo = h_flags_[2], ne_redo = h_flags_[3];
-        if (nv_redo) {
-            Ctx cv = c;
-            cv.nredo = nv_redo;
-            k_vertex_queries<true, STACK><<<xcd_grid(cdiv(nv_redo, kQT)), kQT, 0, s>>>(cv);
-            PPF_HIP(hipGetLastError());
-        }
-        if (ne_redo) {
-            Ctx ce = c;
-            ce.redo = redo_ + m.nv;
-            ce.nredo = ne_redo;
-            k_edge_queries<true, STACK><<<xcd_grid(cdiv(ne_redo, kQT)), kQT, 0, s>>>(ce);
-            PPF_HIP(hipGetLastError());
-        }
+        PPF_HIP(queries(k_proximity<true, STACK>, h_flags_[2], h_flags_[3]));
         PPF_HIP(hipMemcpyAsync(h_flags_, flags_, 4 * sizeof(uint32_t),
                                hipMemcpyDeviceToHost, s));
         PPF_HIP(hipStreamSynchronize(s));
@@ -760,19 +771,10 @@ int Narrow::static_pass(const ppf_contact_mesh &m, const ppf_static_mesh &sm, co
     c.cap = cap;
     c.overflow = flags_;
     auto launch = [&](bool fill) -> int {
-        if (m.nv) {
-            if (fill) k_m2c<true, STACK><<<cdiv(m.nv, kQT), kQT, 0, s>>>(c);
-            else k_m2c<false, STACK><<<cdiv(m.nv, kQT), kQT, 0, s>>>(c);
-            PPF_HIP(hipGetLastError());
-        }
-        if (fill) k_c2m<true, STACK><<<cdiv(sm.nv, kQT), kQT, 0, s>>>(c);
-        else k_c2m<false, STACK><<<cdiv(sm.nv, kQT), kQT, 0, s>>>(c);
+        const uint32_t blocks = cdiv(m.nv, kQT) + cdiv(sm.nv, kQT) + cdiv(m.ne, kQT);
+        if (fill) k_static_proximity<true, STACK><<<blocks, kQT, 0, s>>>(c);
+        else k_static_proximity<false, STACK><<<blocks, kQT, 0, s>>>(c);
         PPF_HIP(hipGetLastError());
-        if (m.ne) {
-            if (fill) k_cm_ee<true, STACK><<<cdiv(m.ne, kQT), kQT, 0, s>>>(c);
-            else k_cm_ee<false, STACK><<<cdiv(m.ne, kQT), kQT, 0, s>>>(c);
-            PPF_HIP(hipGetLastError());
-        }
         return PPF_OK;
     };
     rc = launch(false);

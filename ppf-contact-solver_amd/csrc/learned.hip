@@ -1201,14 +1201,17 @@ int Lpc::gradient(PcgPlanImpl *plan, const float *val, const float *cdiag, const
         set_error("lpc: no probes");
         return PPF_ERR_ARG;
     }
-    if (K > nprobe_cap_ || !pv_) {
-        for (float *p : {pv_, pav_, py_}) {
-            if (p) (void)dev_free(p);
+    const size_t probe = (size_t)K * 3 * n; // more probes, or more rows than before
+    if (probe > probe_cap_) {
+        probe_cap_ = 0;
+        for (float **p : {&pv_, &pav_, &py_}) {
+            if (*p) (void)dev_free(*p);
+            *p = nullptr;
         }
-        PPF_HIP(dev_alloc(&pv_, (size_t)K * 3 * n * sizeof(float)));
-        PPF_HIP(dev_alloc(&pav_, (size_t)K * 3 * n * sizeof(float)));
-        PPF_HIP(dev_alloc(&py_, (size_t)K * 3 * n * sizeof(float)));
-        nprobe_cap_ = K;
+        PPF_HIP(dev_alloc(&pv_, probe * sizeof(float)));
+        PPF_HIP(dev_alloc(&pav_, probe * sizeof(float)));
+        PPF_HIP(dev_alloc(&py_, probe * sizeof(float)));
+        probe_cap_ = probe;
     }
     PPF_HIP(hipMemsetAsync(grad_, 0, LpcLayout::count * sizeof(float), s));
     PPF_HIP(hipMemsetAsync(scal_, 0, 4 * sizeof(float), s));

@@ -93,7 +93,7 @@ class Lpc {
     float *part_ = nullptr;
     size_t part_words_ = 0;
     float *pv_ = nullptr, *pav_ = nullptr, *py_ = nullptr;
-    uint32_t nprobe_cap_ = 0;
+    size_t probe_cap_ = 0; // floats of each
 };
 
 } // namespace ppf

@@ -42,3 +42,26 @@ def test_weight_gradient_at_ragged_row_counts(dev, n):
     assert err < 19 * 2.0 ** -9
     lpc.close()
     plan.close()
+
+
+def test_gradient_of_a_larger_system_after_a_smaller_one(dev):
+    """The probe buffers grow with the rows as well as with the probes."""
+    w = flatten(OL.init_weights(5, zero_head=False))
+
+    def gradient(lpc, n):
+        s = scenes.long_row_spd_system(n=n, hubs=0, fan=0, seed=n)
+        t = {k: torch.from_numpy(np.ascontiguousarray(s[k])).to(dev).reshape(-1)
+             for k in ("row_offset", "col_index", "value", "cdiag", "b")}
+        z = torch.from_numpy(OL.probe_vectors(n, 2, seed=n).astype(np.float32)).to(dev)
+        plan = BlockJacobiPCG(t["row_offset"].int(), t["col_index"].int())
+        lpc.factor(plan, t["value"], t["cdiag"], t["b"])
+        out = lpc.gradient(plan, t["value"], t["cdiag"], z.contiguous())
+        plan.close()
+        return out
+
+    lpc, fresh = LearnedPreconditioner(w), LearnedPreconditioner(w)
+    gradient(lpc, 33)
+    (l0, g0), (l1, g1) = gradient(lpc, 1030), gradient(fresh, 1030)
+    assert l0 == l1 and np.array_equal(g0, g1)
+    lpc.close()
+    fresh.close()

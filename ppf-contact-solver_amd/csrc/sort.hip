@@ -1,10 +1,10 @@
 // sort.hip -- stable LSD radix sort of (uint32 key, uint32 value) pairs.
 //
 // 8-bit digits, one histogram + one scatter kernel per digit. Stability comes
-// from ranking inside a tile in input order: each 256-item round is ranked
-// with wave64 ballots (8 ballots give every lane the mask of lanes holding the
-// same digit), per-wave digit counts go through LDS, and a running per-digit
-// count carries the order across rounds. Replaces the reference's 4-bit,
+// from ranking inside a tile in input order: each 64-pair round of a wave is
+// ranked with ballots (8 ballots give every lane the mask of lanes holding the
+// same digit), and per-wave digit places in LDS carry the order across rounds
+// and waves. Replaces the reference's 4-bit,
 // 8-pass sort (kernels/radix_sort.cu:22-178): 30-bit Morton keys need 4 passes.
 #include "scan.hpp"
 #include "sort.hpp"
@@ -14,76 +14,155 @@ namespace ppf {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kRounds = 4;
-constexpr int kTile = kThreads * kRounds;
 constexpr int kWaves = kThreads / kWave;
+constexpr int kTile = 4 * kThreads; // the small tile
+// Tiles of 16 rounds once they fill the chip (1,048,576 pairs: 256 of them): a
+// digit's run in a tile is then 16 pairs, two cache lines of keys and values,
+// and the scans read a quarter of the counts. Below, tiles of 4 rounds.
+constexpr int kBigRounds = 16;
+constexpr size_t kBigSort = 256 * (size_t)kBigRounds * kThreads;
 
-__global__ __launch_bounds__(kThreads) void k_digit_hist(
-    const uint32_t *__restrict__ keys, size_t n, uint32_t shift,
-    uint32_t ntiles, uint32_t *__restrict__ hist) {
-    __shared__ uint32_t h[256];
-    h[threadIdx.x] = 0;
-    __syncthreads();
-    const size_t base = (size_t)blockIdx.x * kTile;
-#pragma unroll
-    for (int r = 0; r < kRounds; ++r) {
-        const size_t idx = base + (size_t)r * kThreads + threadIdx.x;
-        if (idx < n) {
-            atomicAdd(&h[(keys[idx] >> shift) & 0xffu], 1u);
-        }
+// A wave's count of digit d into h: one addition when all its pairs share a
+// digit (the upper digits of sorted pairs), where 64 would wait for each other.
+__device__ inline void count_digit(uint32_t *h, uint32_t d, bool valid) {
+    const uint64_t all = __ballot(valid);
+    if (all == 0) {
+        return;
     }
-    __syncthreads();
-    hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+    const uint32_t d0 = __shfl(d, __builtin_ctzll(all));
+    if (__ballot(valid && d == d0) == all) {
+        if ((threadIdx.x & (kWave - 1)) == 0) {
+            atomicAdd(h + d0, (uint32_t)__popcll(all));
+        }
+    } else if (valid) {
+        atomicAdd(h + d, 1u);
+    }
 }
 
-__global__ __launch_bounds__(kThreads) void k_digit_scatter(
-    const uint32_t *__restrict__ keys, const uint32_t *__restrict__ vals,
-    size_t n, uint32_t shift, uint32_t ntiles,
-    const uint32_t *__restrict__ hist_scan, uint32_t *__restrict__ okeys,
-    uint32_t *__restrict__ ovals) {
-    __shared__ uint32_t wcount[kWaves][256];
-    __shared__ uint32_t running[256];
-    running[threadIdx.x] = hist_scan[(size_t)threadIdx.x * ntiles + blockIdx.x];
-    const size_t base = (size_t)blockIdx.x * kTile;
-    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (kWave - lane));
-    for (int r = 0; r < kRounds; ++r) {
+template <int ROUNDS>
+__global__ __launch_bounds__(kThreads) void k_digit_hist(const uint32_t *__restrict__ keys,
+                                                         size_t n, uint32_t shift, uint32_t ntiles,
+                                                         uint32_t *__restrict__ hist) {
+    __shared__ uint32_t h[kWaves][256];
 #pragma unroll
-        for (int k = 0; k < kWaves; ++k) {
-            wcount[k][threadIdx.x] = 0;
+    for (int q = 0; q < kWaves; ++q) {
+        h[q][threadIdx.x] = 0;
+    }
+    __syncthreads();
+    const size_t base = (size_t)blockIdx.x * ROUNDS * kThreads + threadIdx.x;
+    uint32_t k[ROUNDS];
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
+        const size_t i = base + (size_t)r * kThreads;
+        k[r] = i < n ? keys[i] : 0u;
+    }
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
+        count_digit(h[threadIdx.x / kWave], (k[r] >> shift) & 0xffu,
+                    base + (size_t)r * kThreads < n);
+    }
+    __syncthreads();
+    uint32_t sum = 0;
+#pragma unroll
+    for (int q = 0; q < kWaves; ++q) {
+        sum += h[q][threadIdx.x];
+    }
+    hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = sum;
+}
+
+// A tile's pairs, ranked as in k_sort_one (a wave owns a contiguous segment),
+// are put in digit order in LDS and leave from there, so that a digit's pairs
+// are written as one run: 3M pairs 56 -> 20 us a pass (2.4 TB/s), 0.1M 11 -> 9.
+template <int ROUNDS>
+__global__ __launch_bounds__(kThreads) void k_digit_scatter(
+    const uint32_t *__restrict__ keys, const uint32_t *__restrict__ vals, size_t n, uint32_t shift,
+    uint32_t ntiles, const uint32_t *__restrict__ hist_scan, uint32_t *__restrict__ okeys,
+    uint32_t *__restrict__ ovals) {
+    __shared__ uint32_t lk[ROUNDS * kThreads], lv[ROUNDS * kThreads];
+    __shared__ uint32_t cnt[kWaves][256]; // per wave and digit: counts, then places
+    __shared__ uint32_t to[256];          // output place of LDS place 0, per digit
+    __shared__ uint32_t wsum[kWaves];
+    const uint32_t lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (kWave - lane));
+    const size_t tile = (size_t)blockIdx.x * ROUNDS * kThreads;
+    const size_t base = tile + w * ROUNDS * kWave + lane;
+    uint32_t k[ROUNDS], v[ROUNDS];
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
+        const size_t i = base + r * kWave;
+        k[r] = i < n ? keys[i] : 0u;
+        v[r] = i < n ? vals[i] : 0u;
+    }
+    const uint32_t first = hist_scan[(size_t)threadIdx.x * ntiles + blockIdx.x];
+#pragma unroll
+    for (int q = 0; q < kWaves; ++q) {
+        cnt[q][threadIdx.x] = 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
+        count_digit(cnt[w], (k[r] >> shift) & 0xffu, base + r * kWave < n);
+    }
+    __syncthreads();
+    uint32_t total = 0;
+#pragma unroll
+    for (int q = 0; q < kWaves; ++q) {
+        total += cnt[q][threadIdx.x];
+    }
+    uint32_t incl = total;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const uint32_t t = __shfl_up(incl, off, kWave);
+        if (lane >= (uint32_t)off) {
+            incl += t;
         }
-        __syncthreads();
-        const size_t idx = base + (size_t)r * kThreads + threadIdx.x;
-        const bool valid = idx < n;
-        const uint32_t key = valid ? keys[idx] : 0u;
-        const uint32_t d = (key >> shift) & 0xffu;
+    }
+    if (lane == kWave - 1) {
+        wsum[w] = incl;
+    }
+    __syncthreads();
+    uint32_t run = incl - total;
+    for (uint32_t q = 0; q < w; ++q) {
+        run += wsum[q];
+    }
+    to[threadIdx.x] = first - run;
+#pragma unroll
+    for (int q = 0; q < kWaves; ++q) {
+        const uint32_t c = cnt[q][threadIdx.x];
+        cnt[q][threadIdx.x] = run;
+        run += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
+        const bool valid = base + r * kWave < n;
+        const uint32_t d = (k[r] >> shift) & 0xffu;
         uint64_t peers = __ballot(valid);
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
             const uint64_t m = __ballot(valid && ((d >> b) & 1u));
             peers &= ((d >> b) & 1u) ? m : ~m;
         }
-        const uint32_t rank_w = __popcll(peers & below);
-        if (valid && rank_w == 0) {
-            wcount[w][d] = (uint32_t)__popcll(peers);
-        }
-        __syncthreads();
         if (valid) {
-            uint32_t pos = running[d] + rank_w;
-            for (int k = 0; k < w; ++k) {
-                pos += wcount[k][d];
-            }
-            okeys[pos] = key;
-            ovals[pos] = vals[idx];
+            const uint32_t at = cnt[w][d] + __popcll(peers & below);
+            lk[at] = k[r];
+            lv[at] = v[r];
         }
-        __syncthreads();
-        uint32_t add = 0;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (valid && (peers & below) == 0) {
+            cnt[w][d] += (uint32_t)__popcll(peers);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    __syncthreads();
 #pragma unroll
-        for (int k = 0; k < kWaves; ++k) {
-            add += wcount[k][threadIdx.x];
+    for (int r = 0; r < ROUNDS; ++r) {
+        const uint32_t j = r * kThreads + threadIdx.x;
+        if (tile + j < n) {
+            const uint32_t key = lk[j], pos = to[(key >> shift) & 0xffu] + j;
+            okeys[pos] = key;
+            ovals[pos] = lv[j];
         }
-        running[threadIdx.x] += add;
-        __syncthreads();
     }
 }
 
@@ -225,7 +304,9 @@ hipError_t radix_sort_pairs(uint32_t *keys, uint32_t *vals, size_t n,
         }
         return hipGetLastError();
     }
-    const uint32_t nt = (uint32_t)tiles(n);
+    const bool big = n >= kBigSort;
+    const uint32_t nt = (uint32_t)(big ? (n + kBigRounds * kThreads - 1) / (kBigRounds * kThreads)
+                                       : tiles(n));
     const size_t h = 256 * (size_t)nt;
     uint32_t *k2 = scratch, *v2 = scratch + n;
     uint32_t *hist = scratch + 2 * n, *hscan = hist + h, *sscr = hscan + h;
@@ -233,7 +314,11 @@ hipError_t radix_sort_pairs(uint32_t *keys, uint32_t *vals, size_t n,
     const uint32_t passes = (key_bits + 7) / 8;
     for (uint32_t p = 0; p < passes; ++p) {
         const uint32_t shift = 8 * p;
-        k_digit_hist<<<nt, kThreads, 0, s>>>(ka, n, shift, nt, hist);
+        if (big) {
+            k_digit_hist<kBigRounds><<<nt, kThreads, 0, s>>>(ka, n, shift, nt, hist);
+        } else {
+            k_digit_hist<4><<<nt, kThreads, 0, s>>>(ka, n, shift, nt, hist);
+        }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) {
             return e;
@@ -242,8 +327,12 @@ hipError_t radix_sort_pairs(uint32_t *keys, uint32_t *vals, size_t n,
         if (e != hipSuccess) {
             return e;
         }
-        k_digit_scatter<<<nt, kThreads, 0, s>>>(ka, va, n, shift, nt, hscan, kb,
-                                                vb);
+        if (big) {
+            k_digit_scatter<kBigRounds>
+                <<<nt, kThreads, 0, s>>>(ka, va, n, shift, nt, hscan, kb, vb);
+        } else {
+            k_digit_scatter<4><<<nt, kThreads, 0, s>>>(ka, va, n, shift, nt, hscan, kb, vb);
+        }
         e = hipGetLastError();
         if (e != hipSuccess) {
             return e;

@@ -287,7 +287,7 @@ def walk_stats_step(one_step):
     """One more time step (after the timed window, untimed) with the BVH walk
     statistics on: per kind of walk, launches, queries, nodes taken off the
     walk stacks per query, CCD sweeps, the mean launch time (HIP events), and
-    the walk's algorithmic bytes per launch -- the 64-byte walk record of
+    the walk's algorithmic bytes per launch -- 64 bytes for
     every internal node entered (both children's boxes, tags and codes) --
     over that time."""
     from ppf_amd import _lib

@@ -2076,10 +2076,12 @@ int set_tiles(PcgPlanImpl *pl, uint32_t r1, uint32_t r2, hipStream_t st,
         // fifth on some CUs).
         const uint32_t step = n >= kOrderRows ? 32u : 64u;
         r1 = cdiv(cdiv(n, g1), step) * step;
-        // Vector tiles of at least 128 rows: half the partial sums for every
+        // Vector tiles of at least 128 rows once 64-row tiles would leave a
+        // thread more than one partial sum to read: half the partials for every
         // workgroup to reduce again (65,536 rows: 18.7 -> 17.9 us per iteration;
         // 256 rows give 17.6, but the factor's second pass then loses 1.4%).
-        r2 = cdiv(cdiv(n, g2), 128) * 128;
+        const uint32_t step2 = n > 64u * kNT ? 128u : 64u;
+        r2 = cdiv(cdiv(n, g2), step2) * step2;
         cut(t1, sc1, r1);
         cut(t2, sc2, r2);
         ordered = !pl->arena && n >= kOrderRows;

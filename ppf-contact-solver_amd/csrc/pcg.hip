@@ -64,9 +64,6 @@ constexpr uint32_t kPlaceNone = (1u << kPlaceBits) - 1u;
 constexpr uint32_t kSymCap = kPlaceNone;
 constexpr uint32_t kSymMaxRows = 1u << (32 - kPlaceBits);
 constexpr uint32_t kInTile = 0x80000000u;
-// Rows from which the tiles of a one-scene plan are ordered by their
-// couplings (order_tiles): below, the vectors and blocks stay in the L2s.
-constexpr uint32_t kOrderRows = 98304;
 // Average row length and bytes of blocks from which short rows take the
 // symmetric form too (set_pattern_arrays).
 constexpr double kSymAvg = 14.0;
@@ -796,83 +793,6 @@ __global__ __launch_bounds__(kNT) void k_sym_prep(const Args *__restrict__ A,
     }
     if (threadIdx.x == 0) {
         atomicMax(max_inner, running);
-    }
-}
-
-// Partner of every tile (rows in [t rows, (t + 1) rows)): the tile before it
-// that stores most of its mirrored blocks, if those are at least one per row
-// (sheets in contact; the couplings across a tile's border within a sheet are
-// fewer), else itself.
-constexpr uint32_t kOrderTiles = 2048;
-
-__global__ __launch_bounds__(kNT) void k_tile_links(uint32_t rows, const Tile *__restrict__ tile,
-                                                    const uint32_t *__restrict__ tp,
-                                                    const uint32_t *__restrict__ tcol,
-                                                    uint32_t *__restrict__ link) {
-    __shared__ uint32_t hist[kOrderTiles];
-    __shared__ uint32_t best[kNT];
-    const uint32_t t = blockIdx.x;
-    const Tile T = tile[t];
-    for (uint32_t k = threadIdx.x; k < t; k += kNT) {
-        hist[k] = 0;
-    }
-    __syncthreads();
-    for (uint32_t e = tp[T.lo] + threadIdx.x; e < tp[T.hi]; e += kNT) {
-        const uint32_t u = tcol[e] / rows;
-        if (u < t) {
-            atomicAdd(hist + u, 1u);
-        }
-    }
-    __syncthreads();
-    uint32_t at = t;
-    for (uint32_t k = threadIdx.x; k < t; k += kNT) {
-        if (hist[k] >= T.hi - T.lo && (at == t || hist[k] > hist[at])) {
-            at = k;
-        }
-    }
-    best[threadIdx.x] = at;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (uint32_t k = 0; k < kNT; ++k) { // the largest, the first among equals
-            const uint32_t c = best[k];
-            if (c != t && (at == t || hist[c] > hist[at] || (hist[c] == hist[at] && c < at))) {
-                at = c;
-            }
-        }
-        link[t] = at;
-    }
-}
-
-// The tiles sorted by the first tile of their chain of partners, then by row:
-// the tiles over one another of stacked sheets follow each other. `used`
-// tiles, then padding up to `total`.
-__global__ __launch_bounds__(1024) void k_tile_order(uint32_t used, uint32_t total,
-                                                     const Tile *__restrict__ base,
-                                                     const uint32_t *__restrict__ link,
-                                                     Tile *__restrict__ out) {
-    __shared__ uint32_t l[kOrderTiles], root[kOrderTiles];
-    for (uint32_t t = threadIdx.x; t < used; t += 1024) {
-        l[t] = link[t];
-    }
-    __syncthreads();
-    for (uint32_t t = threadIdx.x; t < used; t += 1024) {
-        uint32_t r = t;
-        while (l[r] < r) { // partners lie before their tile
-            r = l[r];
-        }
-        root[t] = r;
-    }
-    __syncthreads();
-    for (uint32_t t = threadIdx.x; t < total; t += 1024) {
-        uint32_t at = t;
-        if (t < used) {
-            at = 0;
-#pragma unroll 16
-            for (uint32_t k = 0; k < used; ++k) {
-                at += root[k] < root[t] || (root[k] == root[t] && k < t);
-            }
-        }
-        out[at] = base[t];
     }
 }
 
@@ -1614,10 +1534,6 @@ struct PcgPlanImpl {
     uint32_t nscene = 1;
     std::vector<uint32_t> scene_row; // [nscene + 1] first row of each scene
     uint32_t tile_r1 = 0, tile_r2 = 0; // rows per tile; 0: one resident round
-    // large one-scene plans: the tiles in row order and each one's partner
-    // (order_tiles), and the rows per tile
-    Tile *tile_base = nullptr;
-    uint32_t *tile_link = nullptr, tile_rows = 0;
     bool compacted = false;    // tiles cover only the scenes still iterating
     // row order: new row k is original row order[k] (caller's device array);
     // null: the original order
@@ -1909,35 +1825,9 @@ int set_pattern_arrays(PcgPlanImpl *pl, uint32_t nnz, const uint32_t *rp, const 
     return PPF_OK;
 }
 
-// Order of the tiles of a large one-scene plan for the current pattern: tiles
-// that couple strongly share an XCD and run side by side (k_tile_links), so
-// the blocks one stores and the other mirrors, and the rows of v both gather,
-// are fetched into that L2 once. The sums of a row do not change, only the
-// grouping of the partial sums. 8 x 256^2 sheets: 73.3 -> 69.3 us per product
-// within the iteration, 62.8 -> 61.1 us on the stacked drape's own systems.
-int order_tiles(PcgPlanImpl *pl, hipStream_t st) {
-    Args &h = pl->h;
-    if (!pl->tile_base || !h.tile1 || h.G1 > kOrderTiles) {
-        return PPF_OK;
-    }
-    const uint32_t used = cdiv(pl->n, pl->tile_rows);
-    k_tile_links<<<used, kNT, 0, st>>>(pl->tile_rows, pl->tile_base, h.tp, h.tcol, pl->tile_link);
-    PPF_HIP(hipGetLastError());
-    k_tile_order<<<1, 1024, 0, st>>>(used, h.G1, pl->tile_base, pl->tile_link,
-                                     const_cast<Tile *>(h.tile1));
-    PPF_HIP(hipGetLastError());
-    return PPF_OK;
-}
-
 // Tables of the symmetric form for the current pattern and tiles.
 int build_sym(PcgPlanImpl *pl, hipStream_t st) {
     Args &h = pl->h;
-    if (pl->split) {
-        int rc = order_tiles(pl, st);
-        if (rc != PPF_OK) {
-            return rc;
-        }
-    }
     h.mq = h.tq = nullptr;
     if (!pl->sym || !h.tile1) {
         return PPF_OK;
@@ -2038,7 +1928,6 @@ int set_tiles(PcgPlanImpl *pl, uint32_t r1, uint32_t r2, hipStream_t st,
     const uint32_t n = pl->n, ns = pl->nscene;
     Args &h = pl->h;
     std::vector<Tile> t1, t2;
-    bool ordered = false; // tiles follow order_tiles
     std::vector<uint32_t> sc1(ns + 1), sc2(ns + 1);
     auto cut = [&](std::vector<Tile> &t, std::vector<uint32_t> &sc, uint32_t rows) {
         for (uint32_t c = 0; c < ns; ++c) {
@@ -2070,12 +1959,7 @@ int set_tiles(PcgPlanImpl *pl, uint32_t r1, uint32_t r2, hipStream_t st,
         }
         const uint32_t g1 = round8(std::min(res1, cdiv(n, 64)));
         const uint32_t g2 = std::min(resident_blocks(k_update<false, false>, 2048u), cdiv(n, 64));
-        // Rows per tile in chunks of 64, of 32 in a large plan: the product
-        // waits for the CU with most rows (527,360 rows, symmetric form: 59.9 us
-        // with 416 rows a tile, 61.7 with 448, 68 with 512: 1,030 tiles put a
-        // fifth on some CUs).
-        const uint32_t step = n >= kOrderRows ? 32u : 64u;
-        r1 = cdiv(cdiv(n, g1), step) * step;
+        r1 = cdiv(cdiv(n, g1), 64) * 64;
         // Vector tiles of at least 128 rows once 64-row tiles would leave a
         // thread more than one partial sum to read: half the partials for every
         // workgroup to reduce again (65,536 rows: 18.7 -> 17.9 us per iteration;
@@ -2084,7 +1968,6 @@ int set_tiles(PcgPlanImpl *pl, uint32_t r1, uint32_t r2, hipStream_t st,
         r2 = cdiv(cdiv(n, g2), step2) * step2;
         cut(t1, sc1, r1);
         cut(t2, sc2, r2);
-        ordered = !pl->arena && n >= kOrderRows;
         pl->tile_r1 = pl->tile_r2 = 0;
     } else {
         cut(t1, sc1, r1);
@@ -2103,8 +1986,6 @@ int set_tiles(PcgPlanImpl *pl, uint32_t r1, uint32_t r2, hipStream_t st,
     const size_t bytes = carve_bytes(ns, sizeof(Scalars)) + 2 * carve_bytes(ns + 1, 4) +
                          carve_bytes(t1.size(), sizeof(Tile)) +
                          carve_bytes(t2.size(), sizeof(Tile)) +
-                         carve_bytes(ordered ? t1.size() : 0, sizeof(Tile)) +
-                         carve_bytes(ordered ? t1.size() : 0, 4) +
                          carve_bytes(2 * t1.size() + 2 * t2.size(), 4);
     if (bytes > pl->tmem_cap) {
         if (active) {
@@ -2127,16 +2008,6 @@ int set_tiles(PcgPlanImpl *pl, uint32_t r1, uint32_t r2, hipStream_t st,
     Tile *d2 = carve<Tile>(cur, t2.size());
     h.tile1 = d1, h.tile2 = d2, h.sc1 = dsc1, h.sc2 = dsc2;
     h.part = carve<float>(cur, 2 * t1.size() + 2 * t2.size());
-    pl->tile_base = nullptr;
-    pl->tile_link = nullptr;
-    pl->tile_rows = 0;
-    if (ordered) {
-        pl->tile_base = carve<Tile>(cur, t1.size());
-        pl->tile_link = carve<uint32_t>(cur, t1.size());
-        pl->tile_rows = r1;
-        PPF_HIP(hipMemcpyAsync(pl->tile_base, t1.data(), t1.size() * sizeof(Tile),
-                               hipMemcpyHostToDevice, st));
-    }
     PPF_HIP(hipMemcpyAsync(d1, t1.data(), t1.size() * sizeof(Tile), hipMemcpyHostToDevice, st));
     PPF_HIP(hipMemcpyAsync(d2, t2.data(), t2.size() * sizeof(Tile), hipMemcpyHostToDevice, st));
     PPF_HIP(hipMemcpyAsync(dsc1, sc1.data(), sc1.size() * 4, hipMemcpyHostToDevice, st));

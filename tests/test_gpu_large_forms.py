@@ -1,6 +1,6 @@
-"""One-scene plans large enough for ordered tiles (98,304 rows): sheets coupled
-to one another, where tiles have partners, and a single grid, where they have
-none. Split and symmetric forms agree bit for bit and with fp64."""
+"""Large one-scene plans that choose between the ELL and the symmetric form by
+their average row: sheets coupled to one another and a single grid. Split and
+symmetric forms agree bit for bit and with fp64."""
 import numpy as np
 import pytest
 import torch
@@ -34,7 +34,7 @@ def coupled_sheets(res, layers, seed=0):
 
 
 @pytest.mark.parametrize("res,layers", [(223, 2), (131, 6), (314, 1)])
-def test_ordered_tiles(dev, res, layers):
+def test_forms_of_large_plans(dev, res, layers):
     s = coupled_sheets(res, layers)
     assert s["n"] >= 98304
     t = {k: torch.from_numpy(np.ascontiguousarray(s[k])).to(dev).reshape(-1)

@@ -96,11 +96,51 @@ __device__ inline uint32_t root_code(const BvhView &bvh) {
 // and leaves.
 enum Pairing { kPairAll = 0, kPairAbove = 1, kPairBelow = -1 };
 
-// Reads internal node v's walk record and tests its children against q: codes
-// and a bit per overlapping child (aabb::overlap on the stored boxes and
-// scene tags). own: the query's primitive for kPairAbove / kPairBelow. With
-// `inner` (statistics) adds the number of node v's own internal children that
-// overlap q: their boxes are the unions of the stored pairs.
+// Tests the children of a walk record against q: a bit per overlapping child
+// (aabb::overlap on the stored boxes and scene tags; bound: BvhView's). The
+// comparisons keep out unused places, whose boxes are NaN. own: the query's
+// primitive for kPairAbove / kPairBelow. With `inner` (statistics) adds the
+// number of the node's own internal children that overlap q: their boxes are
+// the unions of the stored pairs.
+template <int PAIR>
+PPF_HD uint32_t record_hits(const uint32_t code[4], const uint32_t tag[4], const float b[24],
+                            const QBox &q, uint32_t own, bool scenes, int bound,
+                            uint32_t *inner = nullptr) {
+    uint32_t hit = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float *bx = b + 6 * k;
+        bool ok = (bx[0] <= q.mx[0]) & (bx[3] >= q.mn[0]) & (bx[1] <= q.mx[1]) &
+                  (bx[4] >= q.mn[1]) & (bx[2] <= q.mx[2]) & (bx[5] >= q.mn[2]);
+        if (scenes) {
+            ok &= tag[k] == q.scene || tag[k] == kMixedScene;
+        }
+        if (PAIR != kPairAll) {
+            const uint32_t key = (code[k] & kLeafCode) ? code[k] & ~kLeafCode : tag[k];
+            const bool bounded = (code[k] & kLeafCode) != 0 || bound == PAIR;
+            ok &= !bounded || (PAIR == kPairAbove ? key > own : key < own);
+        }
+        hit |= ok ? 1u << k : 0u;
+    }
+    if (inner) {
+#pragma unroll
+        for (int k = 0; k < 4; k += 2) {
+            const float *u = b + 6 * k, *w = u + 6;
+            bool ok = code[k + 1] != kNoCode;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                ok &= fminf(u[d], w[d]) <= q.mx[d] && fmaxf(u[3 + d], w[3 + d]) >= q.mn[d];
+            }
+            if (scenes) {
+                ok &= tag[k] != tag[k + 1] || tag[k] == q.scene || tag[k] == kMixedScene;
+            }
+            *inner += ok ? 1u : 0u;
+        }
+    }
+    return hit;
+}
+
+// Reads internal node v's walk record and tests its children (record_hits).
 template <int PAIR>
 __device__ inline uint32_t enter(const BvhView &bvh, uint32_t v, const QBox &q, uint32_t own,
                                  uint32_t code[4], uint32_t *inner = nullptr) {
@@ -115,38 +155,7 @@ __device__ inline uint32_t enter(const BvhView &bvh, uint32_t v, const QBox &q, 
     }
     code[0] = a.x, code[1] = a.y, code[2] = a.z, code[3] = a.w;
     const uint32_t tag[4] = {t.x, t.y, t.z, t.w};
-    uint32_t hit = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const float *bx = b + 6 * k;
-        bool ok = (bx[0] <= q.mx[0]) & (bx[3] >= q.mn[0]) & (bx[1] <= q.mx[1]) &
-                  (bx[4] >= q.mn[1]) & (bx[2] <= q.mx[2]) & (bx[5] >= q.mn[2]);
-        if (bvh.scenes) {
-            ok &= tag[k] == q.scene || tag[k] == kMixedScene;
-        }
-        if (PAIR != kPairAll) {
-            const uint32_t key = (code[k] & kLeafCode) ? code[k] & ~kLeafCode : tag[k];
-            const bool bounded = (code[k] & kLeafCode) != 0 || bvh.bound == PAIR;
-            ok &= !bounded || (PAIR == kPairAbove ? key > own : key < own);
-        }
-        hit |= ok ? 1u << k : 0u;
-    }
-    if (inner) {
-#pragma unroll
-        for (int k = 0; k < 4; k += 2) {
-            const float *u = b + 6 * k, *w = u + 6;
-            bool ok = code[k + 1] != kNoCode;
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                ok &= fminf(u[d], w[d]) <= q.mx[d] && fmaxf(u[3 + d], w[3 + d]) >= q.mn[d];
-            }
-            if (bvh.scenes) {
-                ok &= tag[k] != tag[k + 1] || tag[k] == q.scene || tag[k] == kMixedScene;
-            }
-            *inner += ok ? 1u : 0u;
-        }
-    }
-    return hit;
+    return record_hits<PAIR>(code, tag, b, q, own, bvh.scenes, bvh.bound, inner);
 }
 
 // Work of one lane's tree walks, for the walk statistics: tree nodes whose

@@ -462,22 +462,6 @@ __device__ inline uint32_t join_tag(uint32_t a, uint32_t b, bool scenes, int bou
     return scenes ? (a == b ? a : kMixedScene) : bound > 0 ? max(a, b) : min(a, b);
 }
 
-__device__ inline void put_child(WalkRec &w, int k, uint32_t code, uint32_t tag,
-                                 const float mn[3], const float mx[3]) {
-    w.code[k] = code;
-    w.tag[k] = tag;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        w.box[6 * k + d] = mn[d];
-        w.box[6 * k + 3 + d] = mx[d];
-    }
-}
-__device__ inline void put_none(WalkRec &w, int k) {
-    const float inf = __builtin_inff();
-    const float mn[3] = {inf, inf, inf}, mx[3] = {-inf, -inf, -inf};
-    put_child(w, k, kNoCode, kInactiveTag, mn, mx);
-}
-
 // One block of 1,024 leaves: their boxes, then the boxes and walk records of
 // the class 0 nodes above them, one leaf and one node per thread. Rounds of
 // nodes whose children were done in an earlier round, one barrier each (as

@@ -627,19 +627,14 @@ __global__ __launch_bounds__(kNT) void k_spmv_split(const Args *__restrict__ A,
     float dot = 0.0f, adot = 0.0f;
     // row bounds of the next chunk are loaded while this chunk is in flight
     uint32_t nb[4];
-    {
-        const uint32_t i0 = lo + sub < hi ? lo + sub : lo;
-        nb[0] = rp[i0], nb[1] = rp[i0 + 1], nb[2] = tp[i0], nb[3] = tp[i0 + 1];
-    }
+    load_row_bounds(rp, tp, lo, hi, lo + sub, nb);
     for (uint32_t base = lo; base < hi; base += kRows) {
         const uint32_t i = base + sub;
         const bool valid = i < hi;
         const uint32_t ii = valid ? i : lo;
         const uint32_t r0 = nb[0], ns = nb[1] - nb[0], t0 = nb[2], nm = nb[3] - nb[2];
         if (base + kRows < hi) {
-            const uint32_t in = base + kRows + sub;
-            const uint32_t iin = in < hi ? in : lo;
-            nb[0] = rp[iin], nb[1] = rp[iin + 1], nb[2] = tp[iin], nb[3] = tp[iin + 1];
+            load_row_bounds(rp, tp, lo, hi, base + kRows + sub, nb);
         }
         const f3 vi = v.at(ii);
         f3 sum = mk3(0, 0, 0), as = mk3(0, 0, 0);

@@ -7,6 +7,20 @@ namespace ppf {
 
 struct PcgPlanImpl;
 
+// Bounds of the pattern row i and of its transpose-table entries that a lane
+// reads for the tile [lo, hi): the tile's first row past its end. Nothing is
+// read for an empty tile: those that pad a tile list lie at row n, and the
+// caller's offset array ends with rp[n].
+template <class P>
+PPF_HD void load_row_bounds(P rp, P tp, uint32_t lo, uint32_t hi, uint32_t i, uint32_t nb[4]) {
+    nb[0] = nb[1] = nb[2] = nb[3] = 0u;
+    if (lo >= hi) {
+        return;
+    }
+    const uint32_t ii = i < hi ? i : lo;
+    nb[0] = rp[ii], nb[1] = rp[ii + 1], nb[2] = tp[ii], nb[3] = tp[ii + 1];
+}
+
 int pcg_plan_create(uint32_t n, uint32_t nnz, const uint32_t *rp,
                     const uint32_t *col, hipStream_t st, PcgPlanImpl **out);
 // A plan over the block-diagonal union of nscene systems: scene c owns rows

@@ -426,7 +426,9 @@ int ppf_contact_blocks(ppf_contact *h, const uint32_t **d_row_offset,
 
 /* Static collision mesh (data.constraint.mesh, data.hpp:225-240): positions,
  * edges, faces and per-element contact gap / offset, all device pointers.
- * nv == 0 (or a null pointer to it) means no collision mesh. */
+ * nv == 0 (or a null pointer to it) means no collision mesh. The arrays may be
+ * rewritten in place between calls (a stepper's between its steps): every call
+ * works on their present contents. */
 typedef struct ppf_static_mesh {
     uint32_t nv, ne, nf;
     const float *x;

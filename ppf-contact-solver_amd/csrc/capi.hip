@@ -630,8 +630,14 @@ int ppf_intersection_check(ppf_narrow *h, const ppf_contact_mesh *m,
         set_error("ppf_intersection_check: static mesh arrays missing");
         return PPF_ERR_ARG;
     }
-    return h->isect.run(h->impl.tree(0).view(), h->impl.tree(1).view(),
-                        h->impl.tree(2).view(), *m, sm, d_vmass, d_emass, d_fmass,
+    if (sm && sm->nv) {
+        const int rc = h->impl.follow_static(*sm, m->nscene, (hipStream_t)stream, 0, false);
+        if (rc != PPF_OK) {
+            return rc;
+        }
+    }
+    return h->isect.run(h->impl.tree(0).view(), h->impl.tree(1).view(), h->impl.tree(2).view(),
+                        h->impl.static_trees().face, *m, sm, d_vmass, d_emass, d_fmass,
                         surface_vert_count, records, cap, count, (hipStream_t)stream);
 }
 

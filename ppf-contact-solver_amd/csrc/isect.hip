@@ -272,8 +272,8 @@ IntersectionCheck::~IntersectionCheck() {
 }
 
 int IntersectionCheck::run(const BvhView &face, const BvhView &edge, const BvhView &vert,
-                           const ppf_contact_mesh &m, const ppf_static_mesh *sm,
-                           const float *vmass, const float *emass, const float *fmass,
+                           const BvhView &cface, const ppf_contact_mesh &m,
+                           const ppf_static_mesh *sm, const float *vmass, const float *emass, const float *fmass,
                            uint32_t surface_vert_count, ppf_isect_record *records,
                            uint32_t cap, uint32_t *count, hipStream_t s,
                            uint32_t *scene_count) {
@@ -302,25 +302,13 @@ int IntersectionCheck::run(const BvhView &face, const BvhView &edge, const BvhVi
     }
     ppf_static_mesh none{};
     const ppf_static_mesh &S = sm ? *sm : none;
-    if (S.nv && (cm_x_ != S.x || cm_nf_ != S.nf || cm_face_.view().n != S.nf)) {
-        PrimSet sf;
-        sf.n = S.nf, sf.arity = 3, sf.elem = S.face, sf.ghat = S.f_ghat, sf.offset = S.f_off;
-        sf.vscene = S.vscene;
-        sf.nscene = m.nscene;
-        int rc = cm_face_.build(sf, S.x, nullptr, 0.0f, s);
-        if (rc != PPF_OK) {
-            return rc;
-        }
-        cm_x_ = S.x;
-        cm_nf_ = S.nf;
-    }
     IsCtx c;
     c.m = m;
     c.sm = S;
     c.fb = face;
     c.eb = edge;
     c.vb = vert;
-    c.cfb = S.nv ? cm_face_.view() : BvhView{};
+    c.cfb = S.nv ? cface : BvhView{};
     c.vmass = vmass;
     c.emass = emass;
     c.fmass = fmass;

@@ -880,6 +880,20 @@ int Lbvh::refit(const PrimSet &p, const float *x0, const float *x1, float t,
     return PPF_OK;
 }
 
+int Lbvh::follow(const PrimSet &p, const float *x, hipStream_t s, bool fresh) {
+    if (!fresh && followed_x_ == x && followed_elem_ == p.elem && n_ == p.n && bound_ == p.bound &&
+        scenes_ == (p.vscene && p.nscene > 1)) {
+        return refit(p, x, nullptr, 0.0f, s);
+    }
+    followed_x_ = nullptr;
+    const int rc = build(p, x, nullptr, 0.0f, s);
+    if (rc == PPF_OK) {
+        followed_x_ = x;
+        followed_elem_ = p.elem;
+    }
+    return rc;
+}
+
 BvhView Lbvh::view() const {
     BvhView v;
     v.n = n_;

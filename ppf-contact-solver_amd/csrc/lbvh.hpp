@@ -27,8 +27,9 @@ constexpr uint32_t kMixedScene = 0xffffffffu;
 // stands for itself in the first; an unused place holds kNoCode and NaN), so a
 // walk takes two levels of the tree per record. A code is the child's node id,
 // or for a leaf its primitive | kLeafCode. The tag is the scene tag of the
-// child's box in a tree of many scenes; in a one-scene tree it is the child's primitive
-// bound (PrimSet::bound), which lets a query skip subtrees without partners.
+// child's box in a tree of many scenes; in a one-scene tree it is the child's
+// primitive bound (PrimSet::bound), which lets a query skip subtrees without
+// partners.
 // The records are the largest part of a tree: 128 B per leaf beside 80 B of
 // nodes and boxes (two trees of 6M leaves: 1.5 GB of records).
 struct alignas(128) WalkRec {
@@ -69,6 +70,11 @@ struct BvhView {
     int bound = 0;             // tags are primitive bounds: +1 largest, -1 smallest
 };
 
+// The trees of a collision mesh.
+struct StaticTrees {
+    BvhView face, edge;
+};
+
 // Primitive set a tree is built over: `arity` vertex indices per primitive
 // (3 faces, 2 edges, 1 vertices; index = element for vertices), margin
 // 0.5*ghat + offset per primitive.
@@ -101,6 +107,11 @@ class Lbvh {
     // Refit the leaf boxes and the inner boxes, same topology.
     int refit(const PrimSet &p, const float *x0, const float *x1, float t,
               hipStream_t s);
+    // The tree of arrays that their owner may rewrite between calls: refit to
+    // what they hold now, or built where they are others than at the last
+    // call. A refit takes any contents (every primitive keeps a leaf); the
+    // addresses only decide whether the tree is a fresh one, as `fresh` asks for.
+    int follow(const PrimSet &p, const float *x, hipStream_t s, bool fresh = false);
     BvhView view() const;
     uint32_t *nodes() { return node_; }
     Aabb *boxes() { return box_; }
@@ -117,6 +128,8 @@ class Lbvh {
     uint32_t *ext_ = nullptr; // tag of every internal node (scene or primitive bound)
     int bound_ = 0;
     bool scenes_ = false;
+    const float *followed_x_ = nullptr; // arrays of the last follow() that built
+    const uint32_t *followed_elem_ = nullptr;
     uint32_t *sb_ = nullptr; // per-scene centroid bounds (many scenes)
     size_t sb_cap_ = 0;
     void release();

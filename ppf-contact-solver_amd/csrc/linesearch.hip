@@ -467,7 +467,8 @@ LineSearch::~LineSearch() {
 
 int LineSearch::run(const ppf_contact_mesh &m, const ppf_static_mesh *sm,
                     const ppf_ls_params &lp, bool rebuild, float *toi, int *overlap,
-                    hipStream_t s, float *scene_toi, int *scene_overlap, uint32_t *pin_bad) {
+                    hipStream_t s, float *scene_toi, int *scene_overlap, uint32_t *pin_bad,
+                    const StaticTrees *st) {
     const uint32_t ns = (m.vscene && m.nscene > 1) ? m.nscene : 0u;
     const uint32_t words = 5 + 3 * ns;
     if (words > out_cap_) {
@@ -507,20 +508,20 @@ int LineSearch::run(const ppf_contact_mesh &m, const ppf_static_mesh *sm,
     if (rc != PPF_OK) {
         return rc;
     }
-    if (S.nv && (rebuild || sface_.view().n != S.nf || sedge_.view().n != S.ne ||
-                 static_x_ != S.x)) {
+    if (S.nv && !st) {
         PrimSet sf, se;
         sf.n = S.nf, sf.arity = 3, sf.elem = S.face, sf.ghat = S.f_ghat, sf.offset = S.f_off;
         se.n = S.ne, se.arity = 2, se.elem = S.edge, se.ghat = S.e_ghat, se.offset = S.e_off;
         sf.vscene = se.vscene = S.vscene;
         sf.nscene = se.nscene = m.nscene;
-        rc = sface_.build(sf, S.x, nullptr, 0.0f, s);
-        if (rc == PPF_OK) rc = sedge_.build(se, S.x, nullptr, 0.0f, s);
+        rc = sface_.follow(sf, S.x, s, rebuild);
+        if (rc == PPF_OK) rc = sedge_.follow(se, S.x, s, rebuild);
         if (rc != PPF_OK) {
             return rc;
         }
-        static_x_ = S.x;
     }
+    const StaticTrees trees =
+        !S.nv ? StaticTrees{} : st ? *st : StaticTrees{sface_.view(), sedge_.view()};
     // minima start at max_t (per scene too), flags at zero
     const uint32_t tmax = __builtin_bit_cast(uint32_t, lp.max_t);
     std::vector<uint32_t> init(words, 0u);
@@ -536,8 +537,8 @@ int LineSearch::run(const ppf_contact_mesh &m, const ppf_static_mesh *sm,
     c.fb = face_.view();
     c.eb = edge_.view();
     c.vb = vert_.view();
-    c.sfb = S.nv ? sface_.view() : BvhView{};
-    c.seb = S.nv ? sedge_.view() : BvhView{};
+    c.sfb = trees.face;
+    c.seb = trees.edge;
     c.out = out_;
     c.sout = ns ? out_ + 5 : nullptr;
     c.ns = ns;

@@ -695,12 +695,9 @@ int Narrow::proximity_pass(const ppf_contact_mesh &m, ppf_pair *out, uint64_t ca
     return PPF_OK;
 }
 
-int Narrow::build_static(const ppf_static_mesh &sm, uint32_t nscene, hipStream_t s) {
-    if (sm.nv == 0) {
-        return PPF_OK;
-    }
-    if (static_x_ == sm.x && sface_.view().n == sm.nf && sedge_.view().n == sm.ne &&
-        static_nv_ == sm.nv) {
+int Narrow::follow_static(const ppf_static_mesh &sm, uint32_t nscene, hipStream_t s,
+                          uint64_t epoch, bool edges) {
+    if (epoch != 0 && epoch == static_epoch_) {
         return PPF_OK;
     }
     PrimSet f, e;
@@ -708,25 +705,24 @@ int Narrow::build_static(const ppf_static_mesh &sm, uint32_t nscene, hipStream_t
     e.n = sm.ne, e.arity = 2, e.elem = sm.edge, e.ghat = sm.e_ghat, e.offset = sm.e_off;
     f.vscene = e.vscene = sm.vscene;
     f.nscene = e.nscene = nscene;
-    int rc = sface_.build(f, sm.x, nullptr, 0.0f, s);
-    if (rc == PPF_OK) {
-        rc = sedge_.build(e, sm.x, nullptr, 0.0f, s);
-    }
-    if (rc == PPF_OK) {
-        static_x_ = sm.x;
-        static_nv_ = sm.nv;
+    static_epoch_ = 0;
+    int rc = sface_.follow(f, sm.x, s);
+    if (rc == PPF_OK && edges) {
+        rc = sedge_.follow(e, sm.x, s);
+        static_epoch_ = rc == PPF_OK ? epoch : 0;
     }
     return rc;
 }
 
 int Narrow::static_proximity(const ppf_contact_mesh &m, const ppf_static_mesh &sm,
                              const float *vmass, const float *emass, const float *fmass,
-                             ppf_pair *out, uint64_t cap, uint64_t *count, hipStream_t s) {
+                             ppf_pair *out, uint64_t cap, uint64_t *count, hipStream_t s,
+                             uint64_t epoch) {
     *count = 0;
     if (sm.nv == 0) {
         return PPF_OK;
     }
-    int rc = build_static(sm, m.nscene, s);
+    int rc = follow_static(sm, m.nscene, s, epoch);
     if (rc != PPF_OK) {
         return rc;
     }

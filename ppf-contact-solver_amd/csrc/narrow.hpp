@@ -19,11 +19,19 @@ class Narrow {
     int proximity(const ppf_contact_mesh &m, ppf_pair *out, uint64_t cap,
                   uint64_t *count, hipStream_t s);
     Lbvh &tree(int kind) { return kind == 0 ? face_ : (kind == 1 ? edge_ : vert_); }
+    // The collision mesh's trees (nscene: the dynamic mesh's scene count), refit
+    // to its arrays on every call, since their owner may have rewritten them. A
+    // caller that knows them unchanged since its call with the same (non-zero)
+    // epoch passes it again. edges = false: the face tree only.
+    int follow_static(const ppf_static_mesh &sm, uint32_t nscene, hipStream_t s,
+                      uint64_t epoch = 0, bool edges = true);
+    StaticTrees static_trees() const { return {sface_.view(), sedge_.view()}; }
     // Collision-mesh pairs (kinds 4, 5, 6) at the positions of the last
-    // build_trees; the static trees are rebuilt when the static mesh changes.
+    // build_trees (epoch: follow_static's).
     int static_proximity(const ppf_contact_mesh &m, const ppf_static_mesh &sm,
                          const float *vmass, const float *emass, const float *fmass,
-                         ppf_pair *out, uint64_t cap, uint64_t *count, hipStream_t s);
+                         ppf_pair *out, uint64_t cap, uint64_t *count, hipStream_t s,
+                         uint64_t epoch = 0);
 
   private:
     int reserve(uint32_t queries);
@@ -34,11 +42,8 @@ class Narrow {
     int static_pass(const ppf_contact_mesh &m, const ppf_static_mesh &sm, const float *vmass,
                     const float *emass, const float *fmass, ppf_pair *out, uint64_t cap,
                     uint64_t *count, hipStream_t s);
-    // Trees of the collision mesh (nscene: the dynamic mesh's scene count).
-    int build_static(const ppf_static_mesh &sm, uint32_t nscene, hipStream_t s);
     Lbvh face_, edge_, vert_, sface_, sedge_;
-    const float *static_x_ = nullptr;
-    uint32_t static_nv_ = 0;
+    uint64_t static_epoch_ = 0;
     uint32_t qcap_ = 0;
     uint32_t *cnt_ = nullptr, *ofs_ = nullptr, *scratch_ = nullptr;
     ppf_pair *stash_ = nullptr;  // the count pass's first pairs of every query

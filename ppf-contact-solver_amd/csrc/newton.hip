@@ -738,7 +738,7 @@ int Stepper::newton_iteration(const ppf_scene &sc, const ppf_step_params &p, flo
         if (sc.collision.nv) {
             rc = narrow_.static_proximity(m, sc.collision, sc.shell.vmass, sc.emass,
                                           sc.shell.fmass, pairs_ + nself,
-                                          pair_cap_ - nself, &nstat, s);
+                                          pair_cap_ - nself, &nstat, s, epoch_);
             if (rc != PPF_OK) {
                 return rc;
             }
@@ -751,7 +751,7 @@ int Stepper::newton_iteration(const ppf_scene &sc, const ppf_step_params &p, flo
                 if (rc == PPF_OK) {
                     rc = narrow_.static_proximity(m, sc.collision, sc.shell.vmass, sc.emass,
                                                   sc.shell.fmass, pairs_ + nself,
-                                                  pair_cap_ - nself, &nstat, s);
+                                                  pair_cap_ - nself, &nstat, s, epoch_);
                 }
                 if (rc != PPF_OK) {
                     return rc;
@@ -967,8 +967,17 @@ int Stepper::newton_iteration(const ppf_scene &sc, const ppf_step_params &p, flo
         float t = 1.0f;
         uint32_t pin_bad = 0xffffffffu;
         std::vector<int> sovl(ns, 0);
+        StaticTrees st;
+        if (sc.collision.nv) {
+            rc = narrow_.follow_static(sc.collision, lm.nscene, s, epoch_);
+            if (rc != PPF_OK) {
+                return rc;
+            }
+            st = narrow_.static_trees();
+        }
         rc = ls_.run(lm, sc.collision.nv ? &sc.collision : nullptr, lp, first_iteration, &t,
-                     &overlap, s, vs ? toi_out : nullptr, vs ? sovl.data() : nullptr, &pin_bad);
+                     &overlap, s, vs ? toi_out : nullptr, vs ? sovl.data() : nullptr, &pin_bad,
+                     &st);
         if (rc != PPF_OK) {
             return rc;
         }
@@ -1130,6 +1139,7 @@ int Stepper::advance_scenes(const ppf_scene &sc, const ppf_step_params &p, const
                                s));
     }
     records_count_ = 0;
+    ++epoch_;
     uint64_t alloc0 = 0, free0 = 0;
     alloc_totals(&alloc0, &free0);
     const uint32_t n = nv_;
@@ -1246,11 +1256,18 @@ int Stepper::advance_scenes(const ppf_scene &sc, const ppf_step_params &p, const
         if (rc != PPF_OK) {
             return rc;
         }
+        if (sc.collision.nv) {
+            rc = narrow_.follow_static(sc.collision, m.nscene, s, epoch_);
+            if (rc != PPF_OK) {
+                return rc;
+            }
+        }
         uint32_t count = 0;
         std::vector<uint32_t> per(ns, 0u);
         rc = isect_.run(narrow_.tree(0).view(), narrow_.tree(1).view(), narrow_.tree(2).view(),
-                        m, sc.collision.nv ? &sc.collision : nullptr, sc.shell.vmass,
-                        sc.emass, sc.shell.fmass, n, records_, kMaxRecords, &count, s,
+                        narrow_.static_trees().face, m,
+                        sc.collision.nv ? &sc.collision : nullptr, sc.shell.vmass, sc.emass,
+                        sc.shell.fmass, n, records_, kMaxRecords, &count, s,
                         vs ? per.data() : nullptr);
         if (rc != PPF_OK) {
             return rc;

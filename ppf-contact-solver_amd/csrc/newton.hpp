@@ -90,6 +90,8 @@ class Stepper {
     uint32_t npinned_ = 0;
     PcgPlanImpl *plan_ = nullptr;
     Lpc *lpc_ = nullptr;
+    // counts the steps: the collision mesh's arrays keep their contents within one
+    uint64_t epoch_ = 0;
     uint32_t sys_nnz_ = 0;
     ppf_isect_record records_[kMaxRecords] = {};
     uint32_t records_count_ = 0;

@@ -318,14 +318,19 @@ __device__ inline int lcp(const uint32_t *__restrict__ k, const uint32_t *__rest
 }
 
 // Karras radix tree over the sorted codes (lbvh.cu:305-385), and the treelet
-// class of every internal node.
+// class of every internal node. Clears the counts of the lists that follow
+// (segs of them, fewer than leaves): a build may be captured into a graph.
 __global__ __launch_bounds__(kNT) void k_karras(uint32_t n, const uint32_t *__restrict__ k,
                                                 const uint32_t *__restrict__ sk,
                                                 const uint32_t *__restrict__ idx,
                                                 uint32_t *__restrict__ node,
-                                                uint32_t *__restrict__ rank) {
+                                                uint32_t *__restrict__ rank, uint32_t segs,
+                                                uint32_t *__restrict__ count) {
     const int i = blockIdx.x * kNT + threadIdx.x;
     const int nn = (int)n;
+    if ((uint32_t)i < segs) {
+        count[i] = 0;
+    }
     if (i < nn) {
         node[2 * (size_t)i] = idx[i] + 1;
         node[2 * (size_t)i + 1] = 0;
@@ -845,10 +850,7 @@ int Lbvh::build(const PrimSet &p, const float *x0, const float *x1, float t,
     }
     // lists of the nodes across treelet borders: counts, then places
     const uint32_t segs = class_base(n_, top_classes(n_) + 1);
-    if (segs) {
-        PPF_HIP(hipMemsetAsync(list_, 0, segs * sizeof(uint32_t), s));
-    }
-    k_karras<<<nb, kNT, 0, s>>>(n_, code_, sk, idx_, node_, rank_);
+    k_karras<<<nb, kNT, 0, s>>>(n_, code_, sk, idx_, node_, rank_, segs, list_);
     PPF_HIP(hipGetLastError());
     if (segs) {
         k_top_lists<<<class_blocks(n_, 1), kListThreads, 0, s>>>(n_, rank_, list_, list_ + segs);

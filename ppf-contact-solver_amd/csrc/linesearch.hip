@@ -555,7 +555,7 @@ int LineSearch::run(const ppf_contact_mesh &m, const ppf_static_mesh *sm,
                 clk.stop();
             }
             if (sblocks) {
-                k_ls_vertices<D, false><<<sblocks, kWQ, 0, s>>>(c, 0u, 0u);
+                k_ls_vertices<kStack, false><<<sblocks, kWQ, 0, s>>>(c, 0u, 0u);
                 PPF_HIP(hipGetLastError());
             }
         } else if (vblocks + sblocks) {
@@ -581,8 +581,10 @@ int LineSearch::run(const ppf_contact_mesh &m, const ppf_static_mesh *sm,
         PPF_HIP(hipStreamSynchronize(s));
         return PPF_OK;
     };
-    rc = sweeps(std::integral_constant<int, kShortStack>{});
-    if (rc == PPF_OK && h_out_[3]) {
+    // the statistics count every walk once: no second pass
+    rc = c.stats ? sweeps(std::integral_constant<int, kStack>{})
+                 : sweeps(std::integral_constant<int, kShortStack>{});
+    if (rc == PPF_OK && h_out_[3] && !c.stats) {
         // a walk overflowed the short stacks: every sweep again from the start
         PPF_HIP(hipMemcpyAsync(out_, init.data(), words * sizeof(uint32_t),
                                hipMemcpyHostToDevice, s));

@@ -619,8 +619,10 @@ int Narrow::proximity(const ppf_contact_mesh &m, ppf_pair *out, uint64_t cap,
     if (rc != PPF_OK) {
         return rc;
     }
-    rc = proximity_pass<kQueryStack>(m, out, cap, count, s);
-    if (rc == PPF_OK && h_flags_[0]) { // a walk needs the deep stacks
+    // the statistics count every walk once: no second pass
+    const bool once = walk_stats_device() != nullptr;
+    rc = once ? PPF_OK : proximity_pass<kQueryStack>(m, out, cap, count, s);
+    if (rc == PPF_OK && (once || h_flags_[0])) { // a walk needs the deep stacks
         rc = proximity_pass<kDeepStack>(m, out, cap, count, s);
     }
     if (rc == PPF_OK && h_flags_[0]) {

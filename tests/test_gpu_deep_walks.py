@@ -3,9 +3,10 @@
 with the deep stacks and gives the oracle's result."""
 import numpy as np
 import pytest
+import torch
 
 import oracle
-from ppf_amd import scenes
+from ppf_amd import _lib, scenes
 from ppf_amd.ccd import static_to_device
 from ppf_amd.narrow import NarrowPhase, mesh_to_device, pairs_to_numpy
 from test_gpu_ccd import _comb_mesh, _to
@@ -92,4 +93,23 @@ def test_intersections_with_and_without_offsets(dev, offset):
     print(f"offset {offset}: {n} / {nw} by type {kinds}")
     assert n == nw and np.array_equal(kinds, np.bincount(want["type"], minlength=4))
     assert (kinds[1] + kinds[3] > 0) == (offset > 0.0)
+    nph.close()
+
+
+def test_statistics_count_a_deep_walk_once(dev):
+    """The statistics walk with the deep stacks from the start: one launch per
+    kind and call, every element one query."""
+    m = comb_with_span()
+    t = mesh_to_device(m, dev)
+    nph = NarrowPhase()
+    nph.build(t)
+    out = torch.empty((len(oracle.proximity(m)), 4), dtype=torch.int32, device=dev)
+    _lib.walk_stats_enable(True)
+    got = pairs_to_numpy(nph.proximity(t, out))
+    st = _lib.walk_stats()
+    _lib.walk_stats_enable(False)
+    order = ("kind", "a", "b", "count")
+    assert np.array_equal(np.sort(got, order=order), np.sort(oracle.proximity(m), order=order))
+    seen = [(st[k]["launches"], st[k]["queries"]) for k in _lib.WALK_KINDS[2:]]
+    assert seen == [(1, m["nv"]), (1, m["ne"])]
     nph.close()

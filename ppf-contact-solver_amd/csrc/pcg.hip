@@ -35,10 +35,12 @@
 #include "scan.hpp"
 #include "sort.hpp"
 #include <algorithm>
+#include <chrono>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <thread>
 #include <vector>
 
 namespace ppf {
@@ -2371,9 +2373,17 @@ int bookkeeping_lost() {
 // over those scenes only (the partial sums are written and read within one
 // graph, so the switch between graphs is safe). A status copy and its event
 // after each graph took 21 us of a small solve's 97 for eight iterations.
+// Between two looks at the reports the host gives its core away: to whoever is
+// ready to run, and once kNapAfter has passed without progress for kNap. Four
+// iterations (over kNapAfter) are then still to run before the device is short
+// of work.
+constexpr std::chrono::microseconds kNapAfter{100}, kNap{20}, kQueryEvery{1000};
+
 int replay_graphs(PcgPlanImpl *pl, uint32_t max_launch, hipStream_t st) {
     const uint32_t ns = pl->nscene;
-    uint32_t tiled_rows = pl->n, launched = 0, spins = 0;
+    using Clock = std::chrono::steady_clock;
+    Clock::time_point moved = Clock::now(), asked = moved; // last progress, last query
+    uint32_t tiled_rows = pl->n, launched = 0, seen = 0;
     std::vector<uint8_t> active(ns, 1u);
     bool idle = true; // the stream had run dry when the reports below were read
     for (;;) {
@@ -2416,15 +2426,25 @@ int replay_graphs(PcgPlanImpl *pl, uint32_t max_launch, hipStream_t st) {
             idle = false;
             continue;
         }
+        const Clock::time_point now = Clock::now();
+        if (at != seen) {
+            seen = at;
+            moved = now;
+        }
         // An error, or a stream that ran dry, shows in the stream's state.
-        if (++spins % 4096 == 0) {
+        if (now - asked > kQueryEvery) {
+            asked = now;
             const hipError_t e = hipStreamQuery(st);
             if (e != hipSuccess && e != hipErrorNotReady) {
                 PPF_HIP(e);
             }
             idle = e == hipSuccess;
         }
-        __builtin_ia32_pause();
+        if (now - moved > kNapAfter) {
+            std::this_thread::sleep_for(kNap);
+        } else {
+            std::this_thread::yield();
+        }
     }
 }
 

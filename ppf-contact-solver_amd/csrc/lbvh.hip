@@ -68,7 +68,8 @@ __device__ inline uint32_t expand_bits(uint32_t v) {
     return v;
 }
 
-// Centroids (lbvh.cu:120-167 term order) and per-block min/max partials.
+// Centroids (lbvh.cu:120-167 term order) and per-block min/max partials (part
+// null: none, a tree of many scenes has bounds of its own per scene).
 __global__ __launch_bounds__(kNT) void k_centroid(PrimSet p, const float *__restrict__ x,
                                                   float *__restrict__ cent,
                                                   float *__restrict__ part) {
@@ -93,6 +94,9 @@ __global__ __launch_bounds__(kNT) void k_centroid(PrimSet p, const float *__rest
         c[0] = mx[0] = m.x;
         c[1] = mx[1] = m.y;
         c[2] = mx[2] = m.z;
+    }
+    if (!part) {
+        return;
     }
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -805,12 +809,9 @@ int Lbvh::build(const PrimSet &p, const float *x0, const float *x1, float t,
         return PPF_OK;
     }
     const uint32_t nb = cdiv(n_, kNT);
-    float *bounds = part_ + 6 * (size_t)nb;
-    k_centroid<<<nb, kNT, 0, s>>>(p, x0, cent_, part_);
+    const bool scenes = scenes_;
+    k_centroid<<<nb, kNT, 0, s>>>(p, x0, cent_, scenes ? nullptr : part_);
     PPF_HIP(hipGetLastError());
-    k_bounds<<<1, kNT, 0, s>>>(nb, part_, bounds);
-    PPF_HIP(hipGetLastError());
-    const bool scenes = p.vscene && p.nscene > 1;
     if (scenes) {
         // each scene quantized in its own box: a scene's tree does not depend
         // on the other scenes of the mesh
@@ -826,6 +827,8 @@ int Lbvh::build(const PrimSet &p, const float *x0, const float *x1, float t,
         k_scene_bounds<<<cdiv(p.n, kNT * kSceneRun), kNT, 0, s>>>(p, cent_, sb_);
         k_morton_scenes<<<nb, kNT, 0, s>>>(p, cent_, sb_, code_, idx_);
     } else {
+        float *bounds = part_ + 6 * (size_t)nb;
+        k_bounds<<<1, kNT, 0, s>>>(nb, part_, bounds);
         k_morton<<<nb, kNT, 0, s>>>(n_, cent_, bounds, code_, idx_);
     }
     PPF_HIP(hipGetLastError());

@@ -736,7 +736,7 @@ __global__ __launch_bounds__(kNT) void k_spmv_split(const Args *__restrict__ A,
 // (kSymCap), and both the entry (tq, flagged kInTile) and the stored slot it
 // mirrors (mq, beside the slot's column) hold it. Every other entry holds the
 // slot it mirrors, and every stored slot not mirrored in its tile holds
-// kPlaceNone (k_sym_init presets mq). *max_inner receives the largest count.
+// kPlaceNone (k_sym_init presets mq).
 __global__ __launch_bounds__(kNT) void k_sym_init(uint32_t nnz, const uint32_t *__restrict__ col,
                                                   uint32_t *__restrict__ mq) {
     const uint32_t s = blockIdx.x * kNT + threadIdx.x;
@@ -747,8 +747,7 @@ __global__ __launch_bounds__(kNT) void k_sym_init(uint32_t nnz, const uint32_t *
 
 __global__ __launch_bounds__(kNT) void k_sym_prep(const Args *__restrict__ A,
                                                   uint32_t *__restrict__ mq,
-                                                  uint32_t *__restrict__ tq,
-                                                  uint32_t *__restrict__ max_inner) {
+                                                  uint32_t *__restrict__ tq) {
     __shared__ uint32_t wsum[kNT / kWave];
     const Tile T = load_tile(A->tile1, blockIdx.x);
     if (T.lo >= T.hi) {
@@ -787,9 +786,6 @@ __global__ __launch_bounds__(kNT) void k_sym_prep(const Args *__restrict__ A,
             }
         }
         running += total;
-    }
-    if (threadIdx.x == 0) {
-        atomicMax(max_inner, running);
     }
 }
 
@@ -1845,11 +1841,10 @@ int build_sym(PcgPlanImpl *pl, hipStream_t st) {
         k_sym_init<<<cdiv(pl->nnz, kNT), kNT, 0, st>>>(pl->nnz, h.col, mq);
         PPF_HIP(hipGetLastError());
     }
-    PPF_HIP(hipMemsetAsync(pl->flags + 3, 0, sizeof(uint32_t), st));
     h.mq = mq;
     h.tq = tq;
     PPF_HIP(hipMemcpyAsync(pl->d_args, &h, sizeof(Args), hipMemcpyHostToDevice, st));
-    k_sym_prep<<<h.G1, kNT, 0, st>>>(pl->d_args, mq, tq, pl->flags + 3);
+    k_sym_prep<<<h.G1, kNT, 0, st>>>(pl->d_args, mq, tq);
     PPF_HIP(hipGetLastError());
     return PPF_OK;
 }

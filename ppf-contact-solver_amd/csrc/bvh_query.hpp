@@ -5,7 +5,8 @@
 // stack lives in LDS, strided by the workgroup size so a wave's stack slots
 // fall in distinct banks. Children are tested before they are pushed, so the
 // stack only ever holds overlapping nodes. A query that would push past the
-// stack flags `overflow` and stops (the caller reports a capacity error).
+// stack flags `overflow` and stops (the caller runs the pass again with deep
+// stacks, and reports a capacity error if those overflow too).
 #pragma once
 #include "lbvh.hpp"
 
@@ -13,14 +14,16 @@ namespace ppf {
 
 constexpr int kQueryThreads = 128; // threads per query workgroup
 // Stack entries per thread. A walk enters one record (two levels of the tree)
-// at a time, goes on with its rightmost overlapping child and pushes the
-// others, so a walk of a tree d levels deep holds at most 3 ceil(d / 2)
-// entries, and far fewer in use. The walks first run with kQueryStack entries
-// (16 KB of LDS per workgroup, ten per CU); a walk that needs more raises the
-// overflow flag and never writes past the stack, and the caller runs the pass
-// again with kDeepStack entries. Those cover every tree of 64 levels; a
-// Karras tree over 30-bit Morton codes is at most 30 levels deep over distinct
-// codes, plus log2 of the largest run of equal codes (ties split by index).
+// at a time and keeps at most three of its children for later, and on its way
+// to the k-th record of a path it holds 3 (k - 1) of them. The walks first run
+// with kQueryStack entries (16 KB of LDS per workgroup, ten per CU); a walk that
+// needs more raises the overflow flag and never writes past the stack, and the
+// caller runs the pass again with kDeepStack entries. traverse() goes on with the
+// rightmost child: 3 k <= kDeepStack, 32 records or trees of 64 levels.
+// traverse_wave() pushes all four: 3 (k - 1) + 4 <= kDeepStack, 31 records or 62
+// levels. A Karras tree is at most as deep as its keys have bits: log2 of the
+// scene count, 30 of the Morton code, and log2 of the largest run of equal codes
+// (ties split by index).
 constexpr int kQueryStack = 32;
 constexpr int kDeepStack = 96;
 

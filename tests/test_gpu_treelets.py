@@ -1,12 +1,16 @@
-"""Trees whose leaf counts lie around the treelet and block borders (1,024 and
-32,768 leaves), with equal codes across borders: nodes and boxes equal the
-oracle's, after a build and after a refit; pairs too, for one scene and many."""
+"""Trees whose leaf counts lie around the treelet and block borders (1,024,
+32,768 and 1,048,576 leaves), with equal codes across borders: nodes and boxes
+of a build equal the oracle's, and pairs too, for one scene and many; after a
+refit at other positions the certified step and the pairs with a collision mesh
+are the oracle's."""
 import numpy as np
 import pytest
 
 import oracle
 from ppf_amd import scenes
+from ppf_amd.ccd import LineSearch, static_to_device
 from ppf_amd.narrow import NarrowPhase, mesh_to_device, pairs_to_numpy
+from test_gpu_ccd import _to
 
 pytestmark = pytest.mark.gpu
 
@@ -63,11 +67,67 @@ def test_trees_of_many_scenes(dev):
     t = mesh_to_device(m, dev)
     nph.build(t)
     got = pairs_to_numpy(nph.proximity(t))
-    want = [len(oracle.proximity(p)) for p in parts]
-    edge = got["kind"] & 255 == 3
-    v = got["a"].astype(np.int64)
-    v[edge] = m["edge"][v[edge], 0]
-    have = np.bincount(m["vscene"][v], minlength=len(sizes))
-    print(f"pairs per scene {have.tolist()} / {want}")
-    assert have.tolist() == want and sum(want) > 0
+    order = ("kind", "a", "b", "count")
+    at = np.cumsum([[0, 0, 0]] + [[p[k] for k in ("nv", "ne", "nf")] for p in parts], axis=0)
+    want = []
+    for p, (v0, e0, f0) in zip(parts, at):
+        w = oracle.proximity(p)
+        kind = w["kind"] & 255  # 0 vertex-face, 1 vertex-edge, 2 vertex-vertex, 3 edge-edge
+        w["a"] += np.where(kind == 3, e0, v0).astype(np.uint32)
+        w["b"] += np.choose(kind, [f0, e0, v0, e0]).astype(np.uint32)
+        want.append(w)
+    print(f"pairs per scene {[len(w) for w in want]}")
+    assert min(len(want[-1]), len(want[1])) > 0
+    assert np.array_equal(np.sort(got, order=order), np.sort(np.concatenate(want), order=order))
+    nph.close()
+
+
+# vertex and edge trees of 3 nf leaves
+@pytest.mark.parametrize("nf", [1, 341, 342, 1025, 10922, 10923])
+def test_refits_around_the_treelet_borders(dev, nf):
+    """The trees of one set of positions, refit at another set: every triangle
+    moves to another's place."""
+    rng = np.random.default_rng(nf)
+    m = triangles(nf, seed=nf)
+    one = [np.ones(m[k], np.float32) for k in ("nv", "ne", "nf")]
+    t, t1 = mesh_to_device(m, dev), _to(dev, *one)
+    step = rng.normal(0, 0.2 * nf ** (-1.0 / 3.0), m["x"].shape).astype(np.float32)
+    probe = triangles(300, seed=nf + 7)  # walks the refit collision mesh
+    p1 = [np.ones(probe[k], np.float32) for k in ("nv", "ne", "nf")]
+    tp, tp1 = mesh_to_device(probe, dev), _to(dev, *p1)
+    sm = scenes.static_mesh(m["x"], m["face"], ghat=0.02)
+    st = static_to_device(sm, dev)
+    ls, nph = LineSearch(), NarrowPhase()
+    nph.build(tp)
+    order = ("kind", "a", "b", "count")
+    seen = 0
+    for turn in range(3):
+        x = m["x"].reshape(nf, 3, 3)
+        if turn:
+            x = x[rng.permutation(nf)] + rng.normal(0, 1e-3, (nf, 1, 3)).astype(np.float32)
+        now = dict(m, x=np.ascontiguousarray(x.reshape(-1, 3), np.float32))
+        x1 = now["x"] + step
+        t["x"].copy_(_to(dev, now["x"].reshape(-1))[0])
+        toi, ov = ls(t, *_to(dev, x1.reshape(-1)), *t1, rebuild=turn == 0)
+        want, wov = oracle.line_search(now, x1, *one)
+        assert np.float32(toi).tobytes() == np.float32(want).tobytes() and ov == wov
+        st["x"].copy_(t["x"])
+        got = pairs_to_numpy(nph.static_pairs(tp, st, *tp1))
+        want = oracle.static_proximity(probe, dict(sm, x=now["x"]), *p1)
+        assert np.array_equal(np.sort(got, order=order), np.sort(want, order=order))
+        seen += len(got)
+    assert seen > 0 or nf == 1
+    ls.close()
+    nph.close()
+
+
+def test_boxes_of_the_third_class(dev):
+    """1,048,578 vertex leaves: nodes across the border of a 1,048,576-leaf block."""
+    m = triangles(349526, seed=349526)
+    nph = NarrowPhase()
+    nph.build(mesh_to_device(m, dev))
+    nodes, boxes, root = nph.tree(2)
+    on, ob, oroot = oracle.bvh_build(m, 2)
+    assert root == oroot and np.array_equal(nodes, on)
+    assert np.array_equal(boxes[:, [0, 1, 2, 4, 5, 6]].view(np.uint32), ob.view(np.uint32))
     nph.close()

@@ -1,6 +1,7 @@
-"""Large one-scene plans that choose between the ELL and the symmetric form by
-their average row: sheets coupled to one another and a single grid. Split and
-symmetric forms agree bit for bit and with fp64."""
+"""Large one-scene plans in each SpMV form: sheets coupled to one another and a
+single grid, whose split and symmetric forms agree bit for bit and with fp64;
+and the form that a plan takes by itself on both sides of the lines (14 entries
+a row on average, 16 MiB of blocks) at which short rows become symmetric."""
 import numpy as np
 import pytest
 import torch
@@ -60,4 +61,47 @@ def test_forms_of_large_plans(dev, res, layers):
     res_l1 = np.abs(s["b"] - M @ out["sym"][1].astype(np.float64)).sum() / np.abs(s["b"]).sum()
     print(f"{res} x {layers}: {out['sym'][2]} iterations, true residual {res_l1:.2e}")
     assert res_l1 < 1.5e-4
+    plan.close()
+
+
+def banded(n, band, seed=0):
+    """Row i coupled to the `band` rows after it: 2 band + 1 entries a row, a
+    diagonally dominant system."""
+    rng = np.random.default_rng(seed)
+    i = np.repeat(np.arange(n), band)
+    j = i + np.tile(np.arange(1, band + 1), n)
+    keep = j < n
+    pairs = np.stack([i[keep], j[keep]], 1)
+    blk = rng.normal(0, 1, (len(pairs), 3, 3))
+    diag = np.tile(np.eye(3) * (12.0 * band), (n, 1, 1))
+    ro, ci, val = scenes.upper_bsr(n, pairs, blk, diag)
+    cd = np.tile(np.eye(3, dtype=np.float32).reshape(-1), (n, 1))
+    return dict(n=n, row_offset=ro, col_index=ci, value=val, cdiag=cd,
+                b=rng.standard_normal(3 * n).astype(np.float32))
+
+
+# 8 (7) stored blocks of 36 B a row: 16 MiB are 58,255 (66,577) rows
+@pytest.mark.parametrize("n,band,want", [(59000, 7, "sym"), (58000, 7, "ell"), (70000, 6, "ell"),
+                                         (1000, 7, "ell")])
+def test_form_by_rule(dev, n, band, want):
+    s = banded(n, band)
+    avg = (2 * len(s["col_index"]) - n) / n
+    size = 36 * len(s["col_index"])
+    print(f"{avg:.3f} entries a row, {size / 2**20:.2f} MiB of blocks")
+    assert (want == "sym") == (avg >= 14.0 and size >= 16 << 20)
+    t = {k: torch.from_numpy(np.ascontiguousarray(s[k])).to(dev).reshape(-1)
+         for k in ("row_offset", "col_index", "value", "cdiag", "b")}
+    plan = BlockJacobiPCG(t["row_offset"], t["col_index"])
+    out = []
+    for form in (None, "split", "sym", "auto"):
+        if form is not None:
+            assert plan.set_form(form) == (want if form == "auto" else form)
+        y = plan.spmv(t["value"], t["cdiag"], t["b"])
+        x = torch.zeros_like(t["b"])
+        r = plan.solve(t["value"], t["cdiag"], t["b"], x, tol=1e-4)
+        assert r.status == 0
+        out.append((y.cpu().numpy(), x.cpu().numpy(), r.iter))
+    # the three forms sum a row in one order
+    for y, x, it in out[1:]:
+        assert np.array_equal(y, out[0][0]) and np.array_equal(x, out[0][1]) and it == out[0][2]
     plan.close()

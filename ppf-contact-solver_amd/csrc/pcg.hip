@@ -72,9 +72,10 @@ constexpr double kSymAvg = 14.0;
 constexpr uint64_t kSymBytes = 16ull << 20;
 // Bytes of blocks up to which an iteration forms p inside the SpMV, of the
 // split and symmetric forms and of the ELL form (short rows gather less). us
-// per iteration with a kernel for p / inside: grids of 33^2 14.1 / 12.6, 129^2
-// 15.4 / 13.7, 512^2 (38 MB) 42.1 / 41.3, 724^2 63.2 / 62.7, 1024^2 121 / 126;
-// 8 x 64^2 sheets (11 MB) 17.7 / 16.7, 8 x 91^2 (22 MB) 27.0 / 29.1.
+// per iteration of a solve with a kernel for p / inside: grids of 33^2 12.9 /
+// 11.0, 129^2 14.4 / 12.5, 512^2 (36 MiB) 38.0 / 35.6, 724^2 (72 MiB) 64.9 /
+// 63.6, 1024^2 120 / 126; 8 x 64^2 sheets (10 MiB) 16.4 / 14.5, 8 x 91^2 (21 MiB)
+// 25.9 / 26.8.
 constexpr uint64_t kFuseBytes = 16ull << 20, kFuseEllBytes = 48ull << 20;
 
 // Device-resident scalars of one solve. Written by exactly one thread of one
@@ -1763,11 +1764,11 @@ int set_pattern_arrays(PcgPlanImpl *pl, uint32_t nnz, const uint32_t *rp, const 
     // symmetric variant (in-tile mirrors through LDS) wherever it would take
     // the split form, and for long rows (kSymAvg entries on average) once the
     // blocks outgrow half of the L2s (kSymBytes): their second read then costs
-    // more than the LDS hand-over. Symmetric against ELL, us per product:
-    // 8 x 64^2 sheets (10.6 MB of blocks) 6.4 / 5.9, 8 x 91^2 (21.7 MB) 11.4 /
-    // 13.3, 8 x 129^2 19.5 / 22.9, 8 x 256^2 64 / 78, 2 x 256^2 16.5 / 19.7; one
-    // 320^2 sheet (13 entries a row) 13.3 / 13.1. The caller may fix the form
-    // instead.
+    // more than the LDS hand-over. Symmetric against ELL, us per product (50 in
+    // a row): 8 x 64^2 sheets (10 MiB of blocks) 6.7 / 6.0, 8 x 91^2 (21 MiB) 11.4
+    // / 13.0, 8 x 129^2 20.6 / 23.4, 8 x 256^2 71 / 85, 3 x 200^2 17.8 / 20.4, 2 x
+    // 256^2 17.0 / 19.7; one 320^2 sheet (13 entries a row) 13.5 / 13.0. The
+    // caller may fix the form instead.
     {
         const double avg = n ? (2.0 * nnz - n) / n : 0.0;
         const uint32_t m = (uint32_t)((avg + 1.0 + 3.999) / 4.0);
@@ -1954,8 +1955,9 @@ int set_tiles(PcgPlanImpl *pl, uint32_t r1, uint32_t r2, hipStream_t st,
         r1 = cdiv(cdiv(n, g1), 64) * 64;
         // Vector tiles of at least 128 rows once 64-row tiles would leave a
         // thread more than one partial sum to read: half the partials for every
-        // workgroup to reduce again (65,536 rows: 18.7 -> 17.9 us per iteration;
-        // 256 rows give 17.6, but the factor's second pass then loses 1.4%).
+        // workgroup to reduce again (65,536 rows: 17.4 -> 16.6 us per iteration;
+        // 256 rows give 16.0, but the factor's second pass then loses 2%: 54.7 ->
+        // 56.1 us an iteration of 8 x 129^2 sheets).
         const uint32_t step2 = n > 64u * kNT ? 128u : 64u;
         r2 = cdiv(cdiv(n, g2), step2) * step2;
         cut(t1, sc1, r1);

@@ -376,7 +376,7 @@ inline uint32_t wgrad_rows(uint32_t M) {
 // 2 (K + 64) + 8 B puts the four row groups of a fragment in different banks.
 // With gridDim.y = 2 (two 64-wide segments: the node layers) block y sums
 // segment y only, which keeps its sums in registers and doubles the blocks.
-// 459k edge rows x 80: 2,700 us with one 16x16 tile per wave and pass and
+// 526k edge rows x 80: 2,700 us with one 16x16 tile per wave and pass and
 // unstaged 2 B column loads, 76 us now; 32,768 node rows x 128: 2,000 us, 14 us
 // now.
 template <int KT>
@@ -743,7 +743,7 @@ __global__ void k_dhead_out(PcgPattern pt, const float *t, const float *u, float
 // gathered by row, d = fp32 with 9 floats per row, the first NC used), then
 // [NC] column sums of d. With skip / skip2, a row where they agree (a stored
 // diagonal block) counts as zero. fp32 throughout (v_mfma_f32_16x16x4_f32,
-// the bf16 inputs widened exactly); staged as in k_wgrad. 290k blocks x 144:
+// the bf16 inputs widened exactly); staged as in k_wgrad. 296k blocks x 144:
 // 2,027 us with one thread per weight and chunk of rows, 60 us now.
 template <int KT, int NC>
 __global__ __launch_bounds__(256, 2) void k_head_wgrad(uint32_t M, uint32_t rows, Seg s0, Seg s1,
